@@ -17,6 +17,15 @@ FO_COPY_AUTO, FO_COPY_STREAM, FO_COPY_CACHED = range(3)   # store policy of fo_c
 
 _vp, _ip, _i, _ll, _sz, _f = C.c_void_p, C.POINTER(C.c_int), C.c_int, C.c_longlong, C.c_size_t, C.c_float
 
+
+class GemmCall(C.Structure):
+    """struct fo_gemm_call of the header."""
+    _fields_ = [("mode", _i), ("dtype", _i), ("algo", _i), ("M", _i), ("N", _i), ("K", _i), ("rLDN", _i),
+                ("cseg_dev", _vp), ("G", _i), ("group_table", _vp), ("A", _vp), ("B", _vp), ("D", _vp), ("MM", _vp),
+                ("RA", _vp), ("RE", _vp), ("monitor", _i), ("deliver", _vp), ("deliver_from", _i), ("nslices", _i),
+                ("slice_first", _i), ("slice_count", _i), ("slice_stride", _ll), ("group_start", _vp)]
+
+
 # name -> (restype, argtypes); one entry per declaration in the header.
 SIGNATURES = {
     "fo_version": (_i, []),
@@ -28,6 +37,8 @@ SIGNATURES = {
     "fo_gemm_signal": (_i, [_i, _i, _i, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp]),
     "fo_gemm_scatter": (_i, [_i, _i, _i, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp]),
     "fo_gemm_signal_static": (_i, [_i, _i, _i, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp]),
+    "fo_gemm_launch": (_i, [C.POINTER(GemmCall), _vp]),
+    "fo_gemm_last_round": (_i, [_i, _i, _i, _ip]),
     "fo_build_group_table": (_i, [_vp, _i, _i, _vp, _vp]),
     "fo_raster_hint": (_i, [_i, _i, _i, _ip]),
     "fo_tune": (_i, [C.c_char_p, _i]),

@@ -68,23 +68,38 @@ int fo_device_info(int* cu_count, int* clock_khz, int* xcd_count) {
 }
 
 int fo_gemm(int dtype, int algo, int M, int N, int K, const void* A, const void* B, void* D, void* stream) {
-    return launch_gemm(0, dtype, algo, M, N, K, 1, nullptr, 0, nullptr, A, B, D, nullptr, nullptr, nullptr, 0,
-                       (hipStream_t)stream);
+    fo_gemm_call c{};
+    c.mode = FO_GEMM_PLAIN; c.dtype = dtype; c.algo = algo; c.M = M; c.N = N; c.K = K; c.rLDN = 1;
+    c.A = A; c.B = B; c.D = D;
+    return launch_gemm(c, (hipStream_t)stream);
 }
 
 int fo_gemm_signal(int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg_dev, int G,
                    const int* group_table, const void* A, const void* B, void* D, int* MM, const int* RA,
                    int monitor, void* stream) {
-    return launch_gemm(1, dtype, algo, M, N, K, rLDN, cseg_dev, G, group_table, A, B, D, MM, RA, nullptr, monitor,
-                       (hipStream_t)stream);
+    fo_gemm_call c{};
+    c.mode = FO_GEMM_SIGNAL; c.dtype = dtype; c.algo = algo; c.M = M; c.N = N; c.K = K; c.rLDN = rLDN;
+    c.cseg_dev = cseg_dev; c.G = G; c.group_table = group_table;
+    c.A = A; c.B = B; c.D = D; c.MM = MM; c.RA = RA; c.monitor = monitor;
+    return launch_gemm(c, (hipStream_t)stream);
 }
 
 int fo_gemm_scatter(int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg_dev, int G,
                     const int* group_table, const void* A, const void* B, void* D, int* MM, const int* RA,
                     const int* RE, int monitor, void* stream) {
-    return launch_gemm(2, dtype, algo, M, N, K, rLDN, cseg_dev, G, group_table, A, B, D, MM, RA, RE, monitor,
-                       (hipStream_t)stream);
+    fo_gemm_call c{};
+    c.mode = FO_GEMM_SCATTER; c.dtype = dtype; c.algo = algo; c.M = M; c.N = N; c.K = K; c.rLDN = rLDN;
+    c.cseg_dev = cseg_dev; c.G = G; c.group_table = group_table;
+    c.A = A; c.B = B; c.D = D; c.MM = MM; c.RA = RA; c.RE = RE; c.monitor = monitor;
+    return launch_gemm(c, (hipStream_t)stream);
 }
+
+int fo_gemm_launch(const struct fo_gemm_call* call, void* stream) {
+    if (!call) return fail(FO_ERR_ARG, "fo_gemm_launch: null call");
+    return launch_gemm(*call, (hipStream_t)stream);
+}
+
+int fo_gemm_last_round(int algo, int M, int N, int* first_slot) { return last_round(algo, M, N, first_slot); }
 
 int fo_gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg_dev, int G,
                           const void* A, const void* B, void* D, int* MM, const int* RA, int monitor, void* stream) {

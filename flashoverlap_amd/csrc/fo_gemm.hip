@@ -53,6 +53,16 @@
 // tuning knob: its buffer_wbl2 costs 3-10 % of a short-K GEMM.)  The plain
 // GEMM is the same kernel with the signalling compiled out.
 //
+// Delivery: a tile whose group completes with the GEMM has no later work to hide
+// its copy behind, so the epilogue stores it a second time, to where the consumer
+// would have copied it, and leaves its counter alone.  The second store of a strip
+// comes from the same registers; what it saves is the read of C and one wait and
+// one copy launch per group behind the GEMM (4096x4096x4096 fp16 in 16 groups:
+// the overlapped call and its norm 239 -> 117 us; 1024x1024x1024 in 16: 135 -> 14;
+// 128x4096x7168 bf16 in one: 65.6 -> 61.1; plain GEMM 16x4096x7168 with its bulk
+// copy: 63.1 -> 58.8).  It costs the store drain of the round it is in some 4 us
+// per 33 MB, less than the copy kernel that it replaces (11 us and two launch gaps).
+//
 // Semantics follow the reference epilogues src/overlap/gemm_with_signal.h:145-201
 // and src/overlap/gemm_with_scatter.h:146-196; the kernel itself shares nothing
 // with the reference's MUTlass mainloop.
@@ -69,6 +79,23 @@
 #include "fo_raster.h"
 
 namespace fo {
+
+// Scatter, delivered tiles.  A group's rows are cut into nslices equal parts (fo_wait_consume).
+struct GroupRows {
+    int first, part;   // first row of a group in the permuted view, rows of a slice
+};
+__device__ __forceinline__ GroupRows group_rows(const GemmParams& p, int slot) {
+    const int g = p.gtable[slot];
+    return {p.gstart[g] << p.log_bm, (p.cseg[g] << p.log_bm) / p.nslices};
+}
+// The row of the receive buffers that row q of the permuted view goes to, -1 if this call keeps no
+// buffer for its slice.
+__device__ __forceinline__ int receive_row(const GemmParams& p, int q, GroupRows r) {
+    const unsigned in_group = (unsigned)(q - r.first);
+    const int slice = (int)(in_group / (unsigned)r.part) - p.slice_first;
+    if (slice < 0 || slice >= p.slice_count) return -1;
+    return slice * p.slice_rows + r.first / p.nslices + (int)(in_group % (unsigned)r.part);
+}
 
 // STORE: 0 cached, 1 write-through tile stores; REL: 0 release atomic, 1 relaxed atomic.
 // EDGE (plain GEMM only): M and N are arbitrary; the rows and columns of a macro tile that lie
@@ -131,18 +158,25 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
         if (sig_lane) sig_slot = p.RA[(mt.m * tiles_m + sig_m) * p.TN + mt.n * tiles_n + sig_n];
     }
     [[maybe_unused]] int re_lo = 0, re_hi = 0;   // scatter: the remapped destination rows of this quadrant
+    [[maybe_unused]] int dl_lo = -1, dl_hi = -1; // scatter: their rows in the receive buffers, -1: not delivered
+    [[maybe_unused]] GroupRows tile_group{0, 1};
+    bool deliver = MODE == kPlain && p.D2 != nullptr;
     auto resolve_destination = [&]() {
         if constexpr (MODE != kPlain) {
             const int s = __builtin_amdgcn_readfirstlane(quad_slot);
             row0 = (s / p.rLDN) * p.BM + ((wm * WT) & (p.BM - 1));
             col0 = (s % p.rLDN) * p.BN + ((wn * WT) & (p.BN - 1));
             ld = p.rLDN * p.BN;
-            if (sig_lane) sig_group = p.gtable ? p.gtable[sig_slot] : scan_group(p.cseg, sig_slot);
+            // a delivered tile is not signalled: nobody waits for it
+            if (sig_lane && !(p.D2 && sig_slot >= p.deliver_from))
+                sig_group = p.gtable ? p.gtable[sig_slot] : scan_group(p.cseg, sig_slot);
+            deliver = p.D2 && s >= p.deliver_from;
         }
         // Scatter: one or two remapped rows per lane, handed round between the lanes in the epilogue.
         if constexpr (MODE == kScatter) {
             re_lo = p.RE[row0 + (lane < WT ? lane : 0)];
             if constexpr (WT > 64) re_hi = p.RE[row0 + 64 + lane];
+            if (deliver) tile_group = group_rows(p, __builtin_amdgcn_readfirstlane(quad_slot));
         }
     };
 
@@ -410,12 +444,23 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
     settle_mfma();
     __builtin_amdgcn_sched_barrier(0);   // no accumulator read is scheduled ahead of the delay
     __syncthreads();  // every wave is done with the panel buffers
+    if constexpr (MODE == kScatter)
+        if (deliver) {
+            // the row map permutes rows inside a group; a row that it sends elsewhere looks its group up
+            auto row_of = [&](int q) {
+                const bool same = (unsigned)(q - tile_group.first) < (unsigned)(tile_group.part * p.nslices);
+                return receive_row(p, q, same ? tile_group : group_rows(p, q >> p.log_bm));
+            };
+            dl_lo = row_of(re_lo);
+            if constexpr (WT > 64) dl_hi = row_of(re_hi);
+        }
     constexpr int PITCH = WT * 2 + 16;                  // strip row pitch in bytes
     constexpr int ROWCH = WT / 8;                       // 16-byte chunks per strip row
     // Two strip buffers per wave, used in turn: the next strip is written while this one is being stored.
     unsigned char* ep0 = smem + wave * (32 * PITCH);
     unsigned char* ep1 = ep0 + 4 * 32 * PITCH;
     T* D = (T*)p.D;
+    T* D2 = (T*)p.D2;
     [[maybe_unused]] __amdgpu_buffer_rsrc_t drsrc;
     if constexpr (STORE == 1) drsrc = __builtin_amdgcn_make_buffer_rsrc(p.D, 0, 0xffffffff, 0x00020000);
 #pragma unroll
@@ -439,6 +484,10 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
             if constexpr (MODE == kScatter) {
                 const int q_row = 32 * i + r;   // row within the quadrant: held by lane q_row % 64
                 row = __shfl((WT > 64 && i >= 2) ? re_hi : re_lo, q_row & 63, 64);
+                if (deliver) {
+                    const int recv = __shfl((WT > 64 && i >= 2) ? dl_hi : dl_lo, q_row & 63, 64);
+                    if (live && recv >= 0) *(u32x4*)(D2 + (size_t)recv * ld + col0 + cc * 8) = v;
+                }
             }
             const size_t off = (size_t)row * ld + col0 + cc * 8;
             if (!live) continue;   // a quadrant outside the matrix goes through the motions and stores nothing
@@ -449,7 +498,10 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
                     const T* e = (const T*)&v;
 #pragma unroll
                     for (int k = 0; k < 8; ++k)
-                        if (gcol + k < p.N) D[off + k] = e[k];
+                        if (gcol + k < p.N) {
+                            D[off + k] = e[k];
+                            if (deliver) D2[off + k] = e[k];
+                        }
                     continue;
                 }
             }
@@ -457,6 +509,9 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
                 __builtin_amdgcn_raw_buffer_store_b128(v, drsrc, (int)(off * 2), 0, 16);  // sc1: write-through
             else
                 *(u32x4*)(D + off) = v;
+            // ordinary stores: the receive buffer is read next
+            if constexpr (MODE != kScatter)
+                if (deliver) *(u32x4*)(D2 + off) = v;
         }
     }
 
@@ -557,9 +612,10 @@ int choose_macro_tile(int BM, int BN, int M, int N, bool any_shape) {
     return 256;
 }
 
-int launch_gemm(int mode, int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg, int G,
-                const int* gtable, const void* A, const void* B, void* D, int* MM, const int* RA,
-                const int* RE, int monitor, hipStream_t stream) {
+int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
+    const int mode = c.mode, dtype = c.dtype, algo = c.algo, M = c.M, N = c.N, K = c.K, rLDN = c.rLDN, G = c.G;
+    const void *A = c.A, *B = c.B;
+    void* D = c.D;
     // An event pair armed by fo_time_next_launch belongs to this call whether or not it gets as far
     // as a launch: taken here, ahead of the validation, so that a rejected call cannot leave it
     // behind for some later, unrelated launch.
@@ -606,19 +662,51 @@ int launch_gemm(int mode, int dtype, int algo, int M, int N, int K, int rLDN, co
     p.BM = BM; p.BN = BN; p.TN = N / BN;
     p.log_bm = BM == 256 ? 8 : 7; p.log_bn = BN == 256 ? 8 : 7;
     p.rLDN = rLDN;
-    p.RA = RA; p.RE = RE; p.cseg = cseg; p.G = G; p.gtable = gtable; p.MM = MM; p.monitor = monitor;
+    p.RA = c.RA; p.RE = c.RE; p.cseg = c.cseg_dev; p.G = G; p.gtable = c.group_table; p.MM = c.MM; p.monitor = c.monitor;
+    p.D2 = c.deliver; p.deliver_from = c.deliver_from; p.gstart = c.group_start;
+    p.nslices = c.nslices; p.slice_first = c.slice_first; p.slice_count = c.slice_count;
 
     if (mode != kPlain) {
-        if (!MM || !RA || !cseg) return fail(FO_ERR_ARG, "fo_gemm_signal: null MM/RA/cSeg");
+        if (!c.MM || !c.RA || !c.cseg_dev) return fail(FO_ERR_ARG, "fo_gemm_signal: null MM/RA/cSeg");
         if (G <= 0) return fail(FO_ERR_ARG, "fo_gemm_signal: G=%d", G);
         const int T = (M / BM) * (N / BN);
         if (rLDN <= 0 || T % rLDN) return fail(FO_ERR_SHAPE, "fo_gemm_signal: rLDN=%d must divide the %d tiles", rLDN, T);
-        if (mode == kScatter && !RE) return fail(FO_ERR_ARG, "fo_gemm_scatter: null RE");
+        if (mode == kScatter && !c.RE) return fail(FO_ERR_ARG, "fo_gemm_scatter: null RE");
+        if (c.deliver && (c.deliver_from < 0 || c.deliver_from > T))
+            return fail(FO_ERR_ARG, "fo_gemm_launch: deliver_from=%d outside 0..%d", c.deliver_from, T);
+        if (c.deliver && c.monitor) return fail(FO_ERR_ARG, "fo_gemm_launch: monitor tickets are taken by signalled tiles; nothing may be delivered");
+        if (c.deliver && mode == kScatter) {
+            if (!c.group_table || !c.group_start) return fail(FO_ERR_ARG, "fo_gemm_launch: a delivered scatter needs group_table and group_start");
+            if (rLDN != 1) return fail(FO_ERR_SHAPE, "fo_gemm_launch: a delivered scatter needs rLDN 1, got %d", rLDN);
+            if (c.nslices <= 0 || BM % c.nslices) return fail(FO_ERR_SHAPE, "fo_gemm_launch: %d slices of a tile of %d rows", c.nslices, BM);
+            if (c.slice_first < 0 || c.slice_count <= 0 || c.slice_first + c.slice_count > c.nslices)
+                return fail(FO_ERR_ARG, "fo_gemm_launch: slices [%d, %d) outside 0..%d", c.slice_first, c.slice_first + c.slice_count, c.nslices);
+            if (c.slice_count > 1 && (c.slice_stride < 0 || c.slice_stride % BN))
+                return fail(FO_ERR_SHAPE, "fo_gemm_launch: slice_stride=%lld is not a whole number of rows of %d", c.slice_stride, BN);
+            p.slice_rows = (int)(c.slice_stride / BN);
+        }
     }
+    if ((uintptr_t)c.deliver & 15) return fail(FO_ERR_ARG, "fo_gemm: operands must be 16-byte aligned");
     if (dtype == FO_F16)
         return macro == 256 ? launch_mt<_Float16, 256>(mode, edge, p, timer, stream)
                             : launch_mt<_Float16, 128>(mode, edge, p, timer, stream);
     return macro == 256 ? launch_mt<__bf16, 256>(mode, edge, p, timer, stream) : launch_mt<__bf16, 128>(mode, edge, p, timer, stream);
+}
+
+int last_round(int algo, int M, int N, int* first_slot) {
+    int BM, BN, BK;
+    if (!first_slot) return fail(FO_ERR_ARG, "fo_gemm_last_round: null output");
+    if (algo_tile(algo, &BM, &BN, &BK) != FO_OK) return fail(FO_ERR_ARG, "fo_gemm_last_round: Algo %d out of range", algo);
+    if (M <= 0 || N <= 0 || M % BM || N % BN) return fail(FO_ERR_SHAPE, "fo_gemm_last_round: M=%d N=%d vs tile %dx%d", M, N, BM, BN);
+    const DeviceFacts* facts;
+    if (int e = device_facts(&facts)) return e;
+    const int macro = choose_macro_tile(BM, BN, M, N, false);
+    const long long total = (long long)((M + macro - 1) / macro) * ((N + macro - 1) / macro);
+    const long long at_once = (long long)facts->cus * (macro == 256 ? 1 : 2);   // workgroups a CU holds: LDS
+    const long long before = (total - 1) / at_once * at_once;
+    const long long T = (long long)(M / BM) * (N / BN);
+    *first_slot = (int)((T * before + total - 1) / total);   // half macro tiles at the edges make it approximate: it is a hint
+    return FO_OK;
 }
 
 int raster_hint(int algo, int M, int N, int* hint) {

@@ -82,6 +82,12 @@ struct GemmParams {
     const int* gtable;
     int* MM;
     int monitor;
+    // delivery (null: none): tiles at slots >= deliver_from are stored there too, and not signalled
+    void* D2;
+    int deliver_from;
+    const int* gstart;                          // scatter: first slot of every group
+    int nslices, slice_first, slice_count;      // scatter: BM is a multiple of nslices
+    int slice_rows;                             // scatter: rows of BN elements between the receive buffers
 };
 
 typedef __attribute__((address_space(3))) void lds_void;

@@ -31,9 +31,8 @@ extern thread_local LaunchTimer t_launch_timer;
 
 // fo_gemm.hip
 int choose_macro_tile(int BM, int BN, int M, int N, bool any_shape);
-int launch_gemm(int mode, int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg, int G,
-                const int* gtable, const void* A, const void* B, void* D, int* MM, const int* RA,
-                const int* RE, int monitor, hipStream_t stream);
+int launch_gemm(const fo_gemm_call& c, hipStream_t stream);
+int last_round(int algo, int M, int N, int* first_slot);
 int raster_hint(int algo, int M, int N, int* hint);
 int tune(const char* key, int value);
 
@@ -51,6 +50,12 @@ int launch_consume(const void* src, void* dst, size_t bytes, hipStream_t stream,
                    int nslices = 1, size_t dst_stride_bytes = 0, int policy = FO_COPY_AUTO, int* expired = nullptr);
 int set_wait_timeout_ms(int ms);
 int wait_timeouts(int* count, int reset);
+
+struct DeviceFacts {
+    int wall_khz = 0;   // rate of wall_clock64()
+    int cus = 0;
+};
+int device_facts(const DeviceFacts** out);   // of the current device
 
 // fo_rmsnorm.hip
 int launch_rmsnorm(int dtype, const void* x, const void* gamma, void* out, int nbatch, int bs, int dim, int BM,

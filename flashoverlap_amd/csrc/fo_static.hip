@@ -61,7 +61,10 @@ int gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, const
     if (int e = scratch_for_current_device(&table)) return e;
     if (int e = launch_group_table(cseg, G, (int)T, table, stream)) return e;
     t_launch_timer = timer;   // for the GEMM's own dispatch
-    return launch_gemm(1, dtype, algo, M, N, K, rLDN, cseg, G, table, A, B, D, MM, RA, nullptr, monitor, stream);
+    fo_gemm_call c{};
+    c.mode = FO_GEMM_SIGNAL; c.dtype = dtype; c.algo = algo; c.M = M; c.N = N; c.K = K; c.rLDN = rLDN;
+    c.cseg_dev = cseg; c.G = G; c.group_table = table; c.A = A; c.B = B; c.D = D; c.MM = MM; c.RA = RA; c.monitor = monitor;
+    return launch_gemm(c, stream);
 }
 
 }  // namespace fo

@@ -286,11 +286,7 @@ __global__ void __launch_bounds__(1024) group_table_kernel(const int* __restrict
 }
 
 // Per-device facts the launchers need on every call, looked up once per device.
-struct DeviceFacts {
-    int wall_khz = 0;   // rate of wall_clock64()
-    int cus = 0;
-};
-static int device_facts(const DeviceFacts** out) {
+int device_facts(const DeviceFacts** out) {
     static DeviceFacts facts[64];
     static std::atomic<unsigned long long> known{0};
     int dev = 0;

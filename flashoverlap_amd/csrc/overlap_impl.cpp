@@ -144,6 +144,9 @@ const int* OverlapImpl::group_table_for(const at::Tensor& cseg_cpu, const at::Te
     if (!same_device || key != table_key_) {
         group_table_ = at::empty({T}, cseg_gpu.options());
         FO_CALL(fo_build_group_table(cseg_gpu.data_ptr<int>(), G, T, group_table_.data_ptr<int>(), gemm_stream_));
+        at::Tensor start = at::empty({G}, cseg_cpu.options());
+        for (int g = 0, acc = 0; g < G; acc += host[g++]) start.data_ptr<int>()[g] = acc;
+        group_start_ = start.to(cseg_gpu.device());
         table_key_ = std::move(key);
     }
     return group_table_.data_ptr<int>();
@@ -151,6 +154,14 @@ const int* OverlapImpl::group_table_for(const at::Tensor& cseg_cpu, const at::Te
 
 void OverlapImpl::bulk_consume(const void* src, void* dst, size_t bytes) {
     FO_CALL(fo_consume(src, dst, bytes, gemm_stream_));
+}
+
+// Whether a receive buffer shares memory with an operand: then it cannot be written while the GEMM reads.
+static bool reads_from(const fo_gemm_call& c, const void* dst, int64_t dst_elems) {
+    const auto hits = [&](const void* p, int64_t elems) {
+        return (const char*)dst < (const char*)p + 2 * elems && (const char*)p < (const char*)dst + 2 * dst_elems;
+    };
+    return hits(c.A, (int64_t)c.M * c.K) || hits(c.B, (int64_t)c.N * c.K);
 }
 
 void OverlapImpl::Gemm(at::Tensor A, at::Tensor B, at::Tensor C, int64_t Algo) {
@@ -185,28 +196,48 @@ void OverlapImpl::refuse_checked_capture(const char* who) {
                 "wait_timeouts() after a replay instead");
 }
 
-void OverlapImpl::fork_comm_stream(int G) {
-    const bool persistent = consumer_mode_ == 2 || (consumer_mode_ == 0 && G > 32);
-    if (!persistent && G <= 1) return;   // the second stream is not used
+void OverlapImpl::fork_comm_stream(int waited, int G) {
+    if (waited == 0 || (waited == G && G <= 1 && !persistent_consumer(waited))) return;   // the second stream is not used
     int capturing = 0;
     FO_CALL(fo_stream_is_capturing(gemm_stream_, &capturing));
     if (capturing) FO_CALL(fo_stream_join(gemm_stream_, comm_stream_));
 }
 
+// How many of the groups are released through their counters; the others are delivered by the
+// GEMM's epilogue.  A group's wait and copy overlap with the GEMM only if the group completes
+// before the GEMM does.  The last group never does, and neither do the groups whose tiles all
+// belong to the last round of workgroups: their copies used to start when the GEMM had ended, one
+// wait and one copy launch after the other (sixteen groups of one round, 4096x4096x4096: 140 us
+// behind a GEMM of 97).  The epilogue has these tiles in registers and stores them twice instead.
+// Checked mode and monitor mode keep every group on its counter (the first reports a count that
+// does not come out, the second takes its tickets from the signals), and so do the explicit modes.
+int OverlapImpl::groups_to_wait_for(const fo_gemm_call& call, const int* cseg, int nslices, int* first_slot) {
+    int BM, BN, BK, late = 0;
+    FO_CALL(fo_algo_tile(call.algo, &BM, &BN, &BK));
+    if (consumer_mode_ != 0 || check_timeouts_ || call.monitor || BM % nslices) return call.G;
+    FO_CALL(fo_gemm_last_round(call.algo, call.M, call.N, &late));
+    int g = 0, slot = 0;
+    while (g + 1 < call.G && slot < late) slot += cseg[g++];
+    *first_slot = slot;
+    return g;
+}
+
 // Per-group release: either the reference's host loop (one wait kernel and one
 // consumer launch per group, src/overlap_impl.cu:257-265 / 312-323) or one
 // persistent kernel that does the same walk on the device.  On return the GEMM
-// stream is ordered behind every group's copy.
+// stream is ordered behind every group's copy.  The first `waited` groups are
+// released here; the others have been delivered by the GEMM itself.
 void OverlapImpl::consume_groups(const at::Tensor& C, void* dst, int64_t tile_elems, const at::Tensor& cseg_cpu,
-                                 const at::Tensor& cseg_gpu, at::Tensor& MM, int nslices, int64_t slice_stride) {
+                                 const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int nslices,
+                                 int64_t slice_stride) {
     const int G = (int)cseg_cpu.numel();
     const int* cseg = cseg_cpu.data_ptr<int>();
     const int slice_first = slice_stride ? 0 : (int)my_rank_;      // stride 0: only this rank's slice
     const int slice_count = slice_stride ? nslices : 1;
-    const bool persistent = consumer_mode_ == 2 || (consumer_mode_ == 0 && G > 32);
     int* expired = expired_.data_ptr<int>();   // this object's own count of expired waits (prepare_call)
-    if (persistent) {
-        FO_CALL(fo_wait_consume(cseg_gpu.data_ptr<int>(), G, MM.data_ptr<int>(), C.data_ptr(), dst, tile_elems,
+    if (waited == 0) return;
+    if (persistent_consumer(waited)) {
+        FO_CALL(fo_wait_consume(cseg_gpu.data_ptr<int>(), waited, MM.data_ptr<int>(), C.data_ptr(), dst, tile_elems,
                                 nslices, slice_first, slice_count, slice_stride, nullptr, consumer_blocks(),
                                 expired, comm_stream_));
         // The caller's stream continues only after the last group is consumed
@@ -219,11 +250,12 @@ void OverlapImpl::consume_groups(const at::Tensor& C, void* dst, int64_t tile_el
     // The groups before the last are copied while the GEMM runs: if that is a lot of data,
     // with stores that leave the GEMM's operands in the memory-side cache.
     int64_t beside = 0;
-    for (int g = 0; g + 1 < G; ++g) beside += tile_elems * cseg[g] / nslices * slice_count * (int64_t)esz;
+    for (int g = 0; g < waited && g + 1 < G; ++g) beside += tile_elems * cseg[g] / nslices * slice_count * (int64_t)esz;
     const int beside_policy = beside >= (int64_t)kStreamCopiesFrom ? FO_COPY_STREAM : FO_COPY_CACHED;
     int64_t acc = 0;
-    for (int g = 0; g < G; ++g) {
-        // The last group completes with the GEMM, so nothing is left for it to overlap with:
+    for (int g = 0; g < waited; ++g) {
+        // If the last group of the call is among them (explicit modes, checked and monitor mode): it
+        // completes with the GEMM, so nothing is left for it to overlap with, and
         // it is released on the GEMM's own stream, where stream order stands in for the wait
         // kernel (the counter is settled by the copy launch itself), and the groups before it,
         // finished long ago on the communication stream, are joined behind it.  A last group
@@ -243,7 +275,53 @@ void OverlapImpl::consume_groups(const at::Tensor& C, void* dst, int64_t tile_el
         acc += comm;
     }
     // The caller's stream continues only after every group is consumed (src/overlap_impl.cu:267-270).
-    if (G > 1) FO_CALL(fo_stream_join(comm_stream_, gemm_stream_));
+    if (waited > 1 || waited < G) FO_CALL(fo_stream_join(comm_stream_, gemm_stream_));
+}
+
+// What the two overlapped calls share: the GEMM (call.mode, RE and nslices say which) and the
+// release of its groups into dst.
+void OverlapImpl::overlapped_call(fo_gemm_call& call, const fo_host::SignalShape& g, const at::Tensor& C, void* dst,
+                                  const at::Tensor& cseg_cpu, const at::Tensor& cseg_gpu, at::Tensor& MM,
+                                  int64_t slice_stride, const char* who) {
+    prepare_call(MM, who);
+    call.cseg_dev = cseg_gpu.data_ptr<int>();
+    call.G = g.G;
+    call.group_table = group_table_for(cseg_cpu, cseg_gpu, g.T);
+    call.MM = MM.data_ptr<int>();
+    const int64_t kept = (int64_t)call.M * call.N / (slice_stride ? 1 : call.nslices);
+    const int waited = reads_from(call, dst, kept)
+                           ? g.G
+                           : groups_to_wait_for(call, cseg_cpu.data_ptr<int>(), call.nslices, &call.deliver_from);
+    if (waited < g.G) {
+        call.deliver = dst;
+        call.group_start = group_start_.data_ptr<int>();
+        call.slice_first = slice_stride ? 0 : (int)my_rank_;
+        call.slice_count = slice_stride ? call.nslices : 1;
+        call.slice_stride = slice_stride;
+    }
+    fork_comm_stream(waited, g.G);
+    FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+    consume_groups(C, dst, (int64_t)g.BM * g.BN, cseg_cpu, cseg_gpu, MM, waited, call.nslices, slice_stride);
+    raise_on_timeout(MM, who);
+}
+
+static fo_gemm_call describe(int mode, const fo_host::GemmShape& s, int64_t algo, int64_t rLDN, const at::Tensor& A,
+                             const at::Tensor& B, const at::Tensor& C, const at::Tensor& RA, bool monitor) {
+    fo_gemm_call c{};
+    c.mode = mode;
+    c.dtype = s.dtype;
+    c.algo = (int)algo;
+    c.M = s.M;
+    c.N = s.N;
+    c.K = s.K;
+    c.rLDN = (int)rLDN;
+    c.A = A.data_ptr();
+    c.B = B.data_ptr();
+    c.D = C.data_ptr();
+    c.RA = RA.defined() ? RA.data_ptr<int>() : nullptr;
+    c.monitor = monitor ? 1 : 0;
+    c.nslices = 1;
+    return c;
 }
 
 void OverlapImpl::GemmAllReduceOverlap(at::Tensor A, at::Tensor B, at::Tensor C, at::Tensor MM, at::Tensor RA,
@@ -255,15 +333,8 @@ void OverlapImpl::GemmAllReduceOverlap(at::Tensor A, at::Tensor B, at::Tensor C,
         fo_host::check_signal(s, MM, RA, at::Tensor(), rLDN, cSEG_CPU, cSEG_GPU, (int)Algo, if_monitor, 1,
                               "gemm_allreduce_overlap");
     c10::DeviceGuard guard(A.device());
-    prepare_call(MM, "gemm_allreduce_overlap");
-    at::Tensor& staging = staging_like(C);
-    const int* table = group_table_for(cSEG_CPU, cSEG_GPU, g.T);
-    fork_comm_stream(g.G);
-    FO_CALL(fo_gemm_signal(s.dtype, (int)Algo, s.M, s.N, s.K, (int)rLDN, cSEG_GPU.data_ptr<int>(), g.G, table,
-                           A.data_ptr(), B.data_ptr(), C.data_ptr(), MM.data_ptr<int>(), RA.data_ptr<int>(),
-                           if_monitor ? 1 : 0, gemm_stream_));
-    consume_groups(C, staging.data_ptr(), (int64_t)g.BM * g.BN, cSEG_CPU, cSEG_GPU, MM, 1, 0);
-    raise_on_timeout(MM, "gemm_allreduce_overlap");
+    fo_gemm_call call = describe(FO_GEMM_SIGNAL, s, Algo, rLDN, A, B, C, RA, if_monitor);
+    overlapped_call(call, g, C, staging_like(C).data_ptr(), cSEG_CPU, cSEG_GPU, MM, 0, "gemm_allreduce_overlap");
 }
 
 void OverlapImpl::GemmReduceScatterOverlap(at::Tensor A, at::Tensor B, at::Tensor C, at::Tensor D, at::Tensor MM,
@@ -282,20 +353,26 @@ void OverlapImpl::GemmReduceScatterOverlap(at::Tensor A, at::Tensor B, at::Tenso
                 "gemm_reducescatter_overlap: D must hold M*N/world_size = ", total / my_size_, " or M*N = ", total,
                 " elements, got ", D.numel());
     c10::DeviceGuard guard(A.device());
-    prepare_call(MM, "gemm_reducescatter_overlap");
-    const int* table = group_table_for(cSEG_CPU, cSEG_GPU, g.T);
-    fork_comm_stream(g.G);
-    FO_CALL(fo_gemm_scatter(s.dtype, (int)Algo, s.M, s.N, s.K, (int)rLDN, cSEG_GPU.data_ptr<int>(), g.G, table,
-                            A.data_ptr(), B.data_ptr(), C.data_ptr(), MM.data_ptr<int>(), RA.data_ptr<int>(),
-                            RE.data_ptr<int>(), if_monitor ? 1 : 0, gemm_stream_));
+    fo_gemm_call call = describe(FO_GEMM_SCATTER, s, Algo, rLDN, A, B, C, RA, if_monitor);
+    call.RE = RE.data_ptr<int>();
+    call.nslices = (int)my_size_;
     const int64_t stride = (D.numel() == total && my_size_ > 1) ? total / my_size_ : 0;
-    consume_groups(C, D.data_ptr(), (int64_t)g.BM * g.BN, cSEG_CPU, cSEG_GPU, MM, (int)my_size_, stride);
-    raise_on_timeout(MM, "gemm_reducescatter_overlap");
+    overlapped_call(call, g, C, D.data_ptr(), cSEG_CPU, cSEG_GPU, MM, stride, "gemm_reducescatter_overlap");
 }
 
+// The bulk copy that stands in for the collective starts when the GEMM has ended, so the GEMM's
+// epilogue makes it: C is stored twice instead of being read back.
 void OverlapImpl::GemmAllReduce(at::Tensor A, at::Tensor B, at::Tensor C, int64_t Algo) {
-    Gemm(A, B, C, Algo);
-    McclAllReduce(C);
+    require_gemm();
+    const fo_host::GemmShape s = fo_host::check_gemm(A, B, C, "gemm_allreduce");
+    c10::DeviceGuard guard(A.device());
+    fo_gemm_call call = describe(FO_GEMM_PLAIN, s, Algo, 1, A, B, C, at::Tensor(), false);
+    void* dst = staging_like(C).data_ptr();
+    // (rows that are not 16-byte aligned are stored element by element: once is enough)
+    const bool after = reads_from(call, dst, C.numel()) || s.N % 8;
+    if (!after) call.deliver = dst;
+    FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+    if (after) bulk_consume(C.data_ptr(), dst, C.numel() * C.element_size());
 }
 
 void OverlapImpl::GemmReduceScatter(at::Tensor A, at::Tensor B, at::Tensor C, at::Tensor D, int64_t Algo) {

@@ -14,6 +14,8 @@
 #include <cstdint>
 #include <vector>
 
+#include "host_common.h"
+
 class OverlapImpl : public torch::CustomClassHolder {
   public:
     OverlapImpl();
@@ -54,8 +56,8 @@ class OverlapImpl : public torch::CustomClassHolder {
     // caller can own its result like it owns C in the reference.  A call whose C
     // does not match the buffer in size, dtype or device goes back to an internal one.
     void SetStaging(at::Tensor buffer);
-    // 0 = automatic (per-group launches up to 32 groups, one persistent kernel
-    // beyond), 1 = one (wait, consume) launch pair per group like the
+    // 0 = automatic (groups that complete with the GEMM are delivered by its epilogue; the
+    // others: per-group launches up to 32 groups, one persistent kernel beyond), 1 = one (wait, consume) launch pair per group like the
     // reference's host loop, 2 = one persistent wait+consume kernel.
     void SetConsumerMode(int64_t mode);
     // Workgroups of the persistent consumer (default and maximum: one per CU).
@@ -86,15 +88,21 @@ class OverlapImpl : public torch::CustomClassHolder {
     at::Tensor staging_;
     at::Tensor expired_;          // one int32 on the device: expired waits of this object's calls
     at::Tensor group_table_;
-    std::vector<int> table_key_;  // cSeg contents + T the table was built for
+    at::Tensor group_start_;      // first slot of every group (device)
+    std::vector<int> table_key_;  // cSeg contents + T the tables were built for
 
     void require_gemm() const;
     void require_overlap() const;
     at::Tensor& staging_like(const at::Tensor& C);
     const int* group_table_for(const at::Tensor& cseg_cpu, const at::Tensor& cseg_gpu, int T);
-    void fork_comm_stream(int G);
+    void overlapped_call(fo_gemm_call& call, const fo_host::SignalShape& g, const at::Tensor& C, void* dst,
+                         const at::Tensor& cseg_cpu, const at::Tensor& cseg_gpu, at::Tensor& MM, int64_t slice_stride,
+                         const char* who);
+    bool persistent_consumer(int groups) const { return consumer_mode_ == 2 || (consumer_mode_ == 0 && groups > 32); }
+    int groups_to_wait_for(const fo_gemm_call& call, const int* cseg, int nslices, int* first_slot);
+    void fork_comm_stream(int waited, int G);
     void consume_groups(const at::Tensor& C, void* dst, int64_t tile_elems, const at::Tensor& cseg_cpu,
-                        const at::Tensor& cseg_gpu, at::Tensor& MM, int nslices, int64_t slice_stride);
+                        const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int nslices, int64_t slice_stride);
     void bulk_consume(const void* src, void* dst, size_t bytes);
     int* expired_word(const at::Tensor& like);
     void refuse_checked_capture(const char* who);

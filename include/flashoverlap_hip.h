@@ -127,6 +127,49 @@ int fo_gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN,
                           const void* A, const void* B, void* D,
                           int* MM, const int* RA, int monitor, void* stream);
 
+/* The three GEMMs above in one call that takes a description, with what the
+ * plain entry points have no argument for.  No counterpart in the reference.
+ *   deliver   (optional) the buffer that the consumer of the output reads: the
+ *             staging buffer of the AllReduce stand-in, or the receive buffers
+ *             of the ReduceScatter stand-in.  The epilogue stores every tile
+ *             at a slot >= deliver_from (plain GEMM: every element) there as
+ *             well as to D, in the layout that fo_consume_slices would copy it
+ *             to, and does not signal it.  For tiles of which nothing is left
+ *             to overlap with (their groups complete with the GEMM itself) this
+ *             replaces the counter, the wait and the copy that reads D again.
+ *             deliver_from must be the first slot of a group.  The GEMM's stream
+ *             orders a later kernel behind the delivery.
+ *   nslices, slice_first, slice_count, slice_stride, group_start
+ *             (scatter mode only) as in fo_wait_consume; group_start is a device
+ *             array of G ints, the first slot of every group; group_table is
+ *             required.  The layout tile's height must be a multiple of nslices
+ *             (a slice is then a whole number of rows), rLDN 1. */
+enum fo_gemm_mode { FO_GEMM_PLAIN = 0, FO_GEMM_SIGNAL = 1, FO_GEMM_SCATTER = 2 };
+struct fo_gemm_call {
+    int mode, dtype, algo, M, N, K, rLDN;
+    const int* cseg_dev;
+    int G;
+    const int* group_table;
+    const void* A;
+    const void* B;
+    void* D;
+    int* MM;
+    const int* RA;
+    const int* RE;
+    int monitor;
+    void* deliver;
+    int deliver_from;
+    int nslices, slice_first, slice_count;
+    long long slice_stride;   /* elements */
+    const int* group_start;
+};
+int fo_gemm_launch(const struct fo_gemm_call* call, void* stream);
+
+/* First slot (in issue order, i.e. under an RA made from fo_raster_hint) of the
+ * tiles that belong to the last round of workgroups the GPU runs for this shape:
+ * the tiles that finish together, when the GEMM ends. */
+int fo_gemm_last_round(int algo, int M, int N, int* first_slot);
+
 /* group_table[s] = group(s) for s in [0,T), computed on the device from
  * cseg_dev.  No counterpart in the reference, whose epilogue rescans cSeg for
  * every tile (src/overlap/gemm_with_signal.h:188-193); results are identical. */

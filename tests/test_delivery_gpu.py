@@ -1,0 +1,106 @@
+"""The GEMM's epilogue as the last groups' consumer: a call in the automatic mode, which delivers the
+groups that complete with the GEMM, against the same call with every group waited for and copied
+(consumer mode 1).  The same tiles take another way to the same place, so every buffer has to be
+bit-identical, and the counters have to end at zero either way."""
+import ctypes as C
+
+import pytest
+import torch
+
+import flashoverlap_amd
+from flashoverlap_amd import capi, tiling
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def api(dev):
+    flashoverlap_amd.load()
+    capi.check(capi.lib().fo_set_wait_timeout_ms(5000))
+    return torch.classes.flashoverlap_class
+
+
+def _object(api, mode, rank=0, size=1):
+    o = api.OverlapImpl()
+    o.mccl_init(rank, size, torch.ops.flashoverlap_op.generate_mccl_id())
+    o.mutlass_init()
+    o.overlap_init()
+    o.set_consumer_mode(mode)
+    return o
+
+
+def _inputs(dev, dt, M, N, K):
+    g = torch.Generator().manual_seed(M + 3 * N + 7 * K)
+    return tuple((torch.randn(r, K, generator=g) / K ** 0.25).to(dt).to(dev) for r in (M, N))
+
+
+@pytest.mark.parametrize("M,N,K,algo,cseg", [
+    (128, 128, 64, 1, [1]),                      # one tile
+    (384, 640, 328, 1, [4, 0, 11]),              # odd multiples of 128, an empty group, a partial last panel
+    (512, 768, 128, 2, [5, 7]),                  # 128x256 layout tiles: half macro tiles and whole ones
+    (768, 384, 72, 4, [1] * 9),                  # 256x128
+    (8192, 2304, 64, 1, [600, 424, 64, 64]),     # 288 macro tiles of 256: a first round and 32 tiles of a second
+])
+@pytest.mark.parametrize("ws,stacked", [(1, False), (4, False), (8, True)])
+def test_delivered_groups_equal_copied_groups(api, dev, M, N, K, algo, cseg, ws, stacked):
+    print(f"delivery {M}x{N}x{K} algo {algo} ws {ws} stacked {stacked}", flush=True)
+    dt = torch.bfloat16
+    BM, BN, _ = capi.algo_tile(algo)
+    TM, TN = M // BM, N // BN
+    cs = torch.tensor(cseg, dtype=torch.int32)
+    RA = tiling.reorder_indices(TM * TN, tiling.raster_hint(M, N, algo), dev).reshape(TM, TN)
+    RE = tiling.generate_row_remap_array(M, N, BM, BN, cseg, ws, dev) if ws > 1 else None
+    A, B = _inputs(dev, dt, M, N, K)
+    got = []
+    for mode in (1, 0):
+        o = _object(api, mode, ws - 1, ws)
+        mm = torch.zeros(len(cseg), dtype=torch.int32, device=dev)
+        c = torch.full((M, N), 7.0, dtype=dt, device=dev)
+        d = torch.full(((ws if stacked else 1) * M // ws, N), 7.0, dtype=dt, device=dev)
+        torch.cuda.synchronize()
+        for _ in range(2):     # the second call finds the first one's counters
+            if ws > 1:
+                o.gemm_reducescatter_overlap(A, B, c, d, mm, RA, RE, 1, cs, cs.to(dev), algo, False)
+            else:
+                o.set_staging(d)
+                o.gemm_allreduce_overlap(A, B, c, mm, RA, 1, cs, cs.to(dev), algo, False)
+        torch.cuda.synchronize()
+        assert o.wait_timeouts(True) == 0 and not mm.any()
+        got.append((c, d))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (127, 129, 72), (300, 520, 136), (384, 640, 64), (2049, 2056, 64)])
+def test_serial_call_delivers_what_it_stores(api, dev, M, N, K):
+    """gemm_allreduce: C and the staging buffer are both the plain GEMM's result, and nothing around them is touched."""
+    A, B = _inputs(dev, torch.float16, M, N, K)
+    want = torch.empty(M, N, dtype=torch.float16, device=dev)
+    c = torch.empty_like(want)
+    guard = torch.full((64 + M * N + 64,), 7.0, dtype=torch.float16, device=dev)
+    staging = guard[64:64 + M * N]
+    o = _object(api, 0)
+    o.mutlass_gemm(A, B, want, 1)
+    o.set_staging(staging)
+    o.gemm_allreduce(A, B, c, 1)
+    torch.cuda.synchronize()
+    assert torch.equal(c, want) and torch.equal(staging.view(M, N), want)
+    assert (guard[:64] == 7.0).all() and (guard[64 + M * N:] == 7.0).all()
+    # a staging buffer that is also an operand is written only when the GEMM has read it
+    if M * N <= A.numel():
+        o.set_staging(A.view(-1)[:M * N])
+        o.gemm_allreduce(A, B, c, 1)
+        torch.cuda.synchronize()
+        assert torch.equal(c, want) and torch.equal(A.view(-1)[:M * N].view(M, N), want)
+
+
+def test_last_round_of_a_shape(dev):
+    """288 macro tiles on 256 CUs: the last round starts at macro tile 256, layout tile 1024 in issue order."""
+    n = C.c_int()
+    capi.check(capi.lib().fo_gemm_last_round(1, 8192, 2304, C.byref(n)))
+    cus = C.c_int()
+    capi.check(capi.lib().fo_device_info(C.byref(cus), None, None))
+    if cus.value == 256:
+        assert n.value == 1024
+    capi.check(capi.lib().fo_gemm_last_round(1, 1024, 1024, C.byref(n)))
+    assert n.value == 0
+    assert capi.lib().fo_gemm_last_round(1, 100, 1024, C.byref(n)) == capi.FO_ERR_SHAPE
