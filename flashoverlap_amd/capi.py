@@ -23,7 +23,8 @@ class GemmCall(C.Structure):
     _fields_ = [("mode", _i), ("dtype", _i), ("algo", _i), ("M", _i), ("N", _i), ("K", _i), ("rLDN", _i),
                 ("cseg_dev", _vp), ("G", _i), ("group_table", _vp), ("A", _vp), ("B", _vp), ("D", _vp), ("MM", _vp),
                 ("RA", _vp), ("RE", _vp), ("monitor", _i), ("deliver", _vp), ("deliver_from", _i), ("nslices", _i),
-                ("slice_first", _i), ("slice_count", _i), ("slice_stride", _ll), ("group_start", _vp)]
+                ("slice_first", _i), ("slice_count", _i), ("slice_stride", _ll), ("group_start", _vp),
+                ("workspace", _vp), ("workspace_bytes", _sz)]
 
 
 # name -> (restype, argtypes); one entry per declaration in the header.
@@ -38,6 +39,7 @@ SIGNATURES = {
     "fo_gemm_scatter": (_i, [_i, _i, _i, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp]),
     "fo_gemm_signal_static": (_i, [_i, _i, _i, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp]),
     "fo_gemm_launch": (_i, [C.POINTER(GemmCall), _vp]),
+    "fo_gemm_workspace": (_i, [C.POINTER(GemmCall), C.POINTER(_sz)]),
     "fo_gemm_last_round": (_i, [_i, _i, _i, _ip]),
     "fo_build_group_table": (_i, [_vp, _i, _i, _vp, _vp]),
     "fo_raster_hint": (_i, [_i, _i, _i, _ip]),

@@ -99,6 +99,11 @@ int fo_gemm_launch(const struct fo_gemm_call* call, void* stream) {
     return launch_gemm(*call, (hipStream_t)stream);
 }
 
+int fo_gemm_workspace(const struct fo_gemm_call* call, size_t* bytes) {
+    if (!call || !bytes) return fail(FO_ERR_ARG, "fo_gemm_workspace: null argument");
+    return gemm_workspace(*call, bytes);
+}
+
 int fo_gemm_last_round(int algo, int M, int N, int* first_slot) { return last_round(algo, M, N, first_slot); }
 
 int fo_gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg_dev, int G,

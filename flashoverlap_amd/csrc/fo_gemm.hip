@@ -80,23 +80,6 @@
 
 namespace fo {
 
-// Scatter, delivered tiles.  A group's rows are cut into nslices equal parts (fo_wait_consume).
-struct GroupRows {
-    int first, part;   // first row of a group in the permuted view, rows of a slice
-};
-__device__ __forceinline__ GroupRows group_rows(const GemmParams& p, int slot) {
-    const int g = p.gtable[slot];
-    return {p.gstart[g] << p.log_bm, (p.cseg[g] << p.log_bm) / p.nslices};
-}
-// The row of the receive buffers that row q of the permuted view goes to, -1 if this call keeps no
-// buffer for its slice.
-__device__ __forceinline__ int receive_row(const GemmParams& p, int q, GroupRows r) {
-    const unsigned in_group = (unsigned)(q - r.first);
-    const int slice = (int)(in_group / (unsigned)r.part) - p.slice_first;
-    if (slice < 0 || slice >= p.slice_count) return -1;
-    return slice * p.slice_rows + r.first / p.nslices + (int)(in_group % (unsigned)r.part);
-}
-
 // STORE: 0 cached, 1 write-through tile stores; REL: 0 release atomic, 1 relaxed atomic.
 // EDGE (plain GEMM only): M and N are arbitrary; the rows and columns of a macro tile that lie
 // outside the matrix are computed on zeros and not stored.
@@ -121,8 +104,21 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
 
-    const TileCoord mt = raster_map(blockIdx.x, p.GM, p.GN, p.gn_magic);
     const int K = p.K;
+    const int NPK = (K + kBK - 1) / kBK;   // panels of the whole K, the last one possibly partial
+    // A split tile: this workgroup multiplies NP panels from kt0 on.  The workgroups of an XCD
+    // (blockIdx.x % 8; split_from is a multiple of 8) get consecutive numbers, split by split, so that
+    // they work on one range of k and share its panels in their L2.
+    int tile = blockIdx.x, kt0 = 0, NP = NPK, part = -1;
+    if (tile >= p.split_from) {
+        const int q = tile - p.split_from, all = p.split_tiles * p.splits, even = all & ~(kXcds - 1);
+        const int at = q < even ? (q & (kXcds - 1)) * (even / kXcds) + q / kXcds : q;
+        part = at / p.split_tiles;
+        tile = p.split_from + (at - part * p.split_tiles);
+        kt0 = part * p.split_panels;
+        NP = min(p.split_panels, NPK - kt0);
+    }
+    const TileCoord mt = raster_map(tile, p.GM, p.GN, p.gn_magic);
     // M and N are multiples of the layout tile, not necessarily of the macro
     // tile: the last row or column of macro tiles may be half inside.  Such a
     // workgroup runs the full main loop (the waves of the outer half re-read the
@@ -197,7 +193,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
     // their LDS bytes, so the panel is zero-padded and the main loop needs no k
     // mask.  The range (2 GiB, checked against the operand sizes on the host) only
     // has to separate that one offset from the real ones.
-    const int k_rest = K % kBK;
+    const int k_rest = kt0 + NP == NPK ? K % kBK : 0;
     constexpr int kOutOfRange = (int)0x80000000u;
     int tail_off0 = cp_off0, tail_off1 = cp_off1;
     if (k_rest) {
@@ -233,7 +229,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
         constexpr bool ISB = decltype(isb_c)::value;
         constexpr int H = decltype(half_c)::value;
         unsigned char* dst = smem + slot + lds_cp;
-        const unsigned koff = (unsigned)kt * (kBK * 2);
+        const unsigned koff = (unsigned)(kt0 + kt) * (kBK * 2);
 #pragma unroll
         for (int j = H * (LOADS / 2); j < (H + 1) * (LOADS / 2); ++j) {
             const int voff = (j & 1) ? vo1 : vo0;   // LOADS*8 is a multiple of 16: slab parity = j parity
@@ -271,13 +267,12 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
     // the k-step and NH..NB-1 for the second.
     frag fa[2][NB], fb[2][NB];   // [k half][block]
 
-    const int NP = (K + kBK - 1) / kBK;   // panels, the last one possibly partial
     // One copy instruction (slab j of the A or B unit of panel kt) into slot `slot`.
     auto issue_one = [&](int kt, int slot, auto isb_c, auto j_c) {
         constexpr bool ISB = decltype(isb_c)::value;
         constexpr int j = decltype(j_c)::value;
         unsigned char* dst = smem + slot + lds_cp;
-        const unsigned koff = (unsigned)kt * (kBK * 2);
+        const unsigned koff = (unsigned)(kt0 + kt) * (kBK * 2);
         const int voff = (j & 1) ? vo1 : vo0;
         const unsigned rows = (ISB ? baseB : baseA) + j * slab_bytes;
         if constexpr (ISB)
@@ -443,16 +438,30 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
     __builtin_amdgcn_s_setprio(0);
     settle_mfma();
     __builtin_amdgcn_sched_barrier(0);   // no accumulator read is scheduled ahead of the delay
+    if (part >= 0) {   // a part of a split tile: the sums as they are
+        f32x4* out = (f32x4*)p.partial + partial_at(p, tile - p.split_from, part, wave, NB * NB) + lane;
+#pragma unroll
+        for (int b = 0; b < NB * NB; b += 4)
+            if (live && 16 * (b / NB) < valid_m - wm * WT) {   // not the blocks below the matrix
+                f32x4 v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[k][r] = acc_read(acc[(b + k) / NB][(b + k) % NB][r]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) out[(b + k) * 64] = v[k];
+                // (the next reads are assembly the compiler cannot see into: not into the registers of a store just issued)
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_nop 1");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        return;
+    }
     __syncthreads();  // every wave is done with the panel buffers
     if constexpr (MODE == kScatter)
         if (deliver) {
-            // the row map permutes rows inside a group; a row that it sends elsewhere looks its group up
-            auto row_of = [&](int q) {
-                const bool same = (unsigned)(q - tile_group.first) < (unsigned)(tile_group.part * p.nslices);
-                return receive_row(p, q, same ? tile_group : group_rows(p, q >> p.log_bm));
-            };
-            dl_lo = row_of(re_lo);
-            if constexpr (WT > 64) dl_hi = row_of(re_hi);
+            dl_lo = receive_row(p, re_lo, tile_group);
+            if constexpr (WT > 64) dl_hi = receive_row(p, re_hi, tile_group);
         }
     constexpr int PITCH = WT * 2 + 16;                  // strip row pitch in bytes
     constexpr int ROWCH = WT / 8;                       // 16-byte chunks per strip row
@@ -494,7 +503,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
             if constexpr (EDGE) {
                 const int gcol = col0 + cc * 8;
                 if (row >= p.M || gcol >= p.N) continue;
-                if (p.N & 7) {     // rows of D are not 16-byte aligned: element by element
+                if (p.N & 7) {     // rows of D are not 16-byte aligned
                     const T* e = (const T*)&v;
 #pragma unroll
                     for (int k = 0; k < 8; ++k)
@@ -568,10 +577,11 @@ static int launch_one(const GemmParams& p, const LaunchTimer& timer, hipStream_t
         FO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem_bytes));
         configured.fetch_or(bit, std::memory_order_release);
     }
+    const int grid = p.split_from + p.split_tiles * p.splits;
     if (timer.start) {
-        hipExtLaunchKernelGGL(kern, dim3(p.GM * p.GN), dim3(256), smem_bytes, stream, timer.start, timer.stop, 0, p);
+        hipExtLaunchKernelGGL(kern, dim3(grid), dim3(256), smem_bytes, stream, timer.start, timer.stop, 0, p);
     } else {
-        hipLaunchKernelGGL(kern, dim3(p.GM * p.GN), dim3(256), smem_bytes, stream, p);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), smem_bytes, stream, p);
     }
     FO_HIP(hipGetLastError());
     return FO_OK;
@@ -610,6 +620,54 @@ int choose_macro_tile(int BM, int BN, int M, int N, bool any_shape) {
         if (wg256 <= 128) return 128;
     }
     return 256;
+}
+
+// Which macro tiles of a shape are split over K, and into how many parts: those of the last round of
+// workgroups, if they occupy at most half of what the GPU runs at a time and the parts stay worth
+// their sums (a part writes MT * MT floats and the reduction reads them again).
+struct SplitPlan {
+    int from, tiles, splits, panels;   // tiles == 0: none
+    size_t bytes;
+};
+static SplitPlan plan_split(int macro, int M, int N, int K, int cus) {
+    const int total = ((M + macro - 1) / macro) * ((N + macro - 1) / macro), panels = (K + kBK - 1) / kBK;
+    const int rest = total % cus ? total % cus : cus;
+    SplitPlan s{total, 0, 1, panels, 0};
+    if (rest * 2 > cus || (macro == 128 && total > rest)) return s;
+    const double panel_us = macro == 256 ? 1.4 : 0.46;                      // a k-step of one workgroup
+    const double part_us = (double)macro * macro * 8 / 6e6;                 // a part written and read at 6 TB/s
+    double best = panels * panel_us;
+    for (int n = 2; n <= cus / rest && n <= 16; ++n) {
+        const int per = (panels + n - 1) / n, parts = (panels + per - 1) / per;
+        if (per < 3) break;
+        const double us = per * panel_us + rest * parts * part_us + 4.5;   // + the reduction's launch
+        if (us < best * 0.95) {
+            best = us;
+            s = {total - rest, rest, parts, per, FO_WORKSPACE_ZEROED + (size_t)rest * parts * macro * macro * sizeof(float)};
+        }
+    }
+    return s;
+}
+
+static int plan_for(const fo_gemm_call& c, int macro, SplitPlan* s) {
+    const DeviceFacts* facts;
+    if (int e = device_facts(&facts)) return e;
+    *s = plan_split(macro, c.M, c.N, c.K, facts->cus);
+    if (c.mode != kPlain && c.monitor) *s = {s->from + s->tiles, 0, 1, 0, 0};   // tickets are taken in the GEMM's epilogue
+    return FO_OK;
+}
+
+int gemm_workspace(const fo_gemm_call& c, size_t* bytes) {
+    int BM, BN, BK;
+    *bytes = 0;
+    if (algo_tile(c.algo, &BM, &BN, &BK) != FO_OK) return fail(FO_ERR_ARG, "fo_gemm_workspace: Algo %d out of range", c.algo);
+    if (c.M <= 0 || c.N <= 0 || c.K <= 0) return fail(FO_ERR_SHAPE, "fo_gemm_workspace: empty problem %dx%dx%d", c.M, c.N, c.K);
+    const int macro = choose_macro_tile(BM, BN, c.M, c.N, c.mode == kPlain);
+    if (!macro) return fail(FO_ERR_SHAPE, "fo_gemm_workspace: M=%d N=%d not multiples of the %dx%d tile", c.M, c.N, BM, BN);
+    SplitPlan s;
+    if (int e = plan_for(c, macro, &s)) return e;
+    *bytes = s.bytes;
+    return FO_OK;
 }
 
 int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
@@ -687,10 +745,25 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
         }
     }
     if ((uintptr_t)c.deliver & 15) return fail(FO_ERR_ARG, "fo_gemm: operands must be 16-byte aligned");
+    p.split_from = p.GM * p.GN;
+    p.splits = 1;
+    if (c.workspace && !timer.start) {
+        SplitPlan s;
+        if (int e = plan_for(c, macro, &s)) return e;
+        if (s.tiles && c.workspace_bytes >= s.bytes) {
+            if ((uintptr_t)c.workspace & 15) return fail(FO_ERR_ARG, "fo_gemm: the workspace must be 16-byte aligned");
+            p.split_from = s.from; p.split_tiles = s.tiles; p.splits = s.splits; p.split_panels = s.panels;
+            p.arrived = (int*)c.workspace;
+            p.partial = (float*)((char*)c.workspace + FO_WORKSPACE_ZEROED);
+        }
+    }
+    int rc;
     if (dtype == FO_F16)
-        return macro == 256 ? launch_mt<_Float16, 256>(mode, edge, p, timer, stream)
-                            : launch_mt<_Float16, 128>(mode, edge, p, timer, stream);
-    return macro == 256 ? launch_mt<__bf16, 256>(mode, edge, p, timer, stream) : launch_mt<__bf16, 128>(mode, edge, p, timer, stream);
+        rc = macro == 256 ? launch_mt<_Float16, 256>(mode, edge, p, timer, stream) : launch_mt<_Float16, 128>(mode, edge, p, timer, stream);
+    else
+        rc = macro == 256 ? launch_mt<__bf16, 256>(mode, edge, p, timer, stream) : launch_mt<__bf16, 128>(mode, edge, p, timer, stream);
+    if (rc == FO_OK && p.split_tiles) rc = launch_split_reduce(mode, dtype, macro, p, stream);
+    return rc;
 }
 
 int last_round(int algo, int M, int N, int* first_slot) {

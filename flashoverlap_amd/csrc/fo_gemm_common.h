@@ -88,7 +88,38 @@ struct GemmParams {
     const int* gstart;                          // scatter: first slot of every group
     int nslices, slice_first, slice_count;      // scatter: BM is a multiple of nslices
     int slice_rows;                             // scatter: rows of BN elements between the receive buffers
+    // Tiles split over K: workgroups split_from .. split_from + split_tiles * splits - 1 compute a part
+    // of `split_panels` panels of the macro tiles split_from .. split_from + split_tiles - 1 each and
+    // leave it in `partial`; the reduction adds the parts up and stores the tiles.
+    int split_from, split_tiles, splits, split_panels;
+    float* partial;
+    int* arrived;                               // reduction: strips of each layout tile that are stored
 };
+
+// Where a part of a split tile lies in `partial`: [tile][split][wave][block i * NB + j][lane] vectors of
+// four floats, i.e. as the accumulators lie in the wavefronts; every access is a contiguous KiB.
+__device__ __forceinline__ size_t partial_at(const GemmParams& p, int tile, int split, int wave, int blocks) {
+    return ((size_t)(tile * p.splits + split) * 4 + wave) * blocks * 64;
+}
+
+// Scatter, delivered tiles.  A group's rows are cut into nslices equal parts (fo_wait_consume).
+struct GroupRows {
+    int first, part;   // first row of a group in the permuted view, rows of a slice
+};
+__device__ __forceinline__ GroupRows group_rows(const GemmParams& p, int slot) {
+    const int g = p.gtable[slot];
+    return {p.gstart[g] << p.log_bm, (p.cseg[g] << p.log_bm) / p.nslices};
+}
+// The row of the receive buffers that row q of the permuted view goes to, -1 if this call keeps no
+// buffer for its slice.  The row map permutes rows inside a group; a row that it sends out of its
+// tile's group looks its own group up.
+__device__ __forceinline__ int receive_row(const GemmParams& p, int q, GroupRows r) {
+    if ((unsigned)(q - r.first) >= (unsigned)(r.part * p.nslices)) r = group_rows(p, q >> p.log_bm);
+    const unsigned in_group = (unsigned)(q - r.first);
+    const int slice = (int)(in_group / (unsigned)r.part) - p.slice_first;
+    if (slice < 0 || slice >= p.slice_count) return -1;
+    return slice * p.slice_rows + r.first / p.nslices + (int)(in_group % (unsigned)r.part);
+}
 
 typedef __attribute__((address_space(3))) void lds_void;
 
@@ -118,6 +149,25 @@ __device__ __forceinline__ int scan_group(const int* cseg, int slot) {
 // holds k-chunk cc ^ swz(row).  Any 8 (or, two rows per 256 bytes, any 16)
 // consecutive rows then hit distinct banks when they read the same k-chunk.
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+
+// Eight elements of a row of which `left` lie inside the matrix, at an address that is a multiple of
+// the element size only (N need not be a multiple of 8): one 16-byte store where all eight do - the
+// compiler knows that global memory takes it at any alignment - and the elements one by one where
+// the row ends.
+template <typename T>
+__device__ __forceinline__ void store_edge_chunk(T* to, u32x4 v, int left) {
+    struct __attribute__((packed, aligned(2))) chunk {
+        u32x4 v;
+    };
+    if (left >= 8) {
+        ((chunk*)to)->v = v;
+        return;
+    }
+    const T* e = (const T*)&v;
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+        if (k < left) to[k] = e[k];
+}
 
 template <int N>
 using template_int = std::integral_constant<int, N>;

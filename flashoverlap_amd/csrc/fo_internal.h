@@ -32,9 +32,14 @@ extern thread_local LaunchTimer t_launch_timer;
 // fo_gemm.hip
 int choose_macro_tile(int BM, int BN, int M, int N, bool any_shape);
 int launch_gemm(const fo_gemm_call& c, hipStream_t stream);
+int gemm_workspace(const fo_gemm_call& c, size_t* bytes);
 int last_round(int algo, int M, int N, int* first_slot);
 int raster_hint(int algo, int M, int N, int* hint);
 int tune(const char* key, int value);
+
+// fo_splitk.hip: sums the parts of the split tiles and stores the tiles as the GEMM's epilogue would
+struct GemmParams;
+int launch_split_reduce(int mode, int dtype, int macro, const GemmParams& p, hipStream_t stream);
 
 // fo_static.hip
 int gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg, int G, const void* A,

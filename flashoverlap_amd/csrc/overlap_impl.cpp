@@ -8,6 +8,8 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <map>
+
 #include "host_common.h"
 
 // Copies made while the GEMM runs use non-temporal stores once a call makes this many bytes
@@ -156,6 +158,86 @@ void OverlapImpl::bulk_consume(const void* src, void* dst, size_t bytes) {
     FO_CALL(fo_consume(src, dst, bytes, gemm_stream_));
 }
 
+static fo_gemm_call describe(int mode, const fo_host::GemmShape& s, int64_t algo, int64_t rLDN, const at::Tensor& A,
+                             const at::Tensor& B, const at::Tensor& C, const at::Tensor& RA, bool monitor) {
+    fo_gemm_call c{};
+    c.mode = mode;
+    c.dtype = s.dtype;
+    c.algo = (int)algo;
+    c.M = s.M;
+    c.N = s.N;
+    c.K = s.K;
+    c.rLDN = (int)rLDN;
+    c.A = A.data_ptr();
+    c.B = B.data_ptr();
+    c.D = C.data_ptr();
+    c.RA = RA.defined() ? RA.data_ptr<int>() : nullptr;
+    c.monitor = monitor ? 1 : 0;
+    c.nslices = 1;
+    return c;
+}
+
+std::shared_ptr<SplitWorkspace> SplitWorkspace::of_stream(int device, void* stream) {
+    static std::mutex mutex;
+    static std::map<std::pair<int, void*>, std::weak_ptr<SplitWorkspace>> pool;
+    std::lock_guard<std::mutex> lock(mutex);
+    for (auto it = pool.begin(); it != pool.end();) it = it->second.expired() ? pool.erase(it) : std::next(it);
+    std::weak_ptr<SplitWorkspace>& slot = pool[{device, stream}];
+    std::shared_ptr<SplitWorkspace> w = slot.lock();
+    if (!w) slot = w = std::make_shared<SplitWorkspace>();
+    return w;
+}
+
+// The GEMM, with a workspace if its shape can use one.  `signals`: some of its tiles are signalled
+// (the workspace's counters are then used, and have to start at zero).
+void OverlapImpl::launch_gemm(fo_gemm_call& call, const at::Tensor& like, bool signals) {
+    size_t need = 0;
+    FO_CALL(fo_gemm_workspace(&call, &need));
+    int step = 0;
+    while (step < 3 && need > ((size_t)4 << 20 << 2 * step)) ++step;
+    if (need == 0 || step == 3) {
+        FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+        return;
+    }
+    const int64_t bytes = (int64_t)4 << 20 << 2 * step;
+    int capturing = 0;
+    FO_CALL(fo_stream_is_capturing(gemm_stream_, &capturing));
+    if (capturing) {
+        // A graph gets memory of its own (it may be replayed beside later calls on this stream): torch's
+        // allocator takes it from the graph's pool.  Captures that torch does not see run unsplit.
+        if ((void*)c10::hip::getCurrentHIPStream().stream() == gemm_stream_) {
+            at::Tensor own = at::empty({(int64_t)need}, like.options().dtype(at::kByte));
+            if (signals) own.narrow(0, 0, FO_WORKSPACE_ZEROED).zero_();
+            call.workspace = own.data_ptr();
+            call.workspace_bytes = need;
+            FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+            return;
+        }
+        FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+        return;
+    }
+    const int device = like.device().index();
+    if (!workspace_ || workspace_device_ != device || workspace_stream_ != gemm_stream_) {
+        workspace_ = SplitWorkspace::of_stream(device, gemm_stream_);
+        workspace_device_ = device;
+        workspace_stream_ = gemm_stream_;
+    }
+    std::lock_guard<std::mutex> lock(workspace_->mutex);
+    at::Tensor& buffer = workspace_->buffer[step];
+    if (!buffer.defined()) {
+        buffer = at::empty({bytes}, like.options().dtype(at::kByte));
+        buffer.narrow(0, 0, FO_WORKSPACE_ZEROED).zero_();
+        const auto current = c10::hip::getCurrentHIPStream();
+        if ((void*)current.stream() != gemm_stream_) {   // once per buffer: filled on one stream, used on another
+            current.synchronize();
+            buffer.record_stream(c10::hip::getStreamFromExternal((hipStream_t)gemm_stream_, (c10::DeviceIndex)device));
+        }
+    }
+    call.workspace = buffer.data_ptr();
+    call.workspace_bytes = (size_t)bytes;
+    FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+}
+
 // Whether a receive buffer shares memory with an operand: then it cannot be written while the GEMM reads.
 static bool reads_from(const fo_gemm_call& c, const void* dst, int64_t dst_elems) {
     const auto hits = [&](const void* p, int64_t elems) {
@@ -168,7 +250,8 @@ void OverlapImpl::Gemm(at::Tensor A, at::Tensor B, at::Tensor C, int64_t Algo) {
     require_gemm();
     const fo_host::GemmShape s = fo_host::check_gemm(A, B, C, "mutlass_gemm");
     c10::DeviceGuard guard(A.device());
-    FO_CALL(fo_gemm(s.dtype, (int)Algo, s.M, s.N, s.K, A.data_ptr(), B.data_ptr(), C.data_ptr(), gemm_stream_));
+    fo_gemm_call call = describe(FO_GEMM_PLAIN, s, Algo, 1, A, B, C, at::Tensor(), false);
+    launch_gemm(call, C, false);
 }
 
 // Called before the GEMM is enqueued.  While the caller's stream is being captured into a
@@ -300,28 +383,9 @@ void OverlapImpl::overlapped_call(fo_gemm_call& call, const fo_host::SignalShape
         call.slice_stride = slice_stride;
     }
     fork_comm_stream(waited, g.G);
-    FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+    launch_gemm(call, C, waited > 0);
     consume_groups(C, dst, (int64_t)g.BM * g.BN, cseg_cpu, cseg_gpu, MM, waited, call.nslices, slice_stride);
     raise_on_timeout(MM, who);
-}
-
-static fo_gemm_call describe(int mode, const fo_host::GemmShape& s, int64_t algo, int64_t rLDN, const at::Tensor& A,
-                             const at::Tensor& B, const at::Tensor& C, const at::Tensor& RA, bool monitor) {
-    fo_gemm_call c{};
-    c.mode = mode;
-    c.dtype = s.dtype;
-    c.algo = (int)algo;
-    c.M = s.M;
-    c.N = s.N;
-    c.K = s.K;
-    c.rLDN = (int)rLDN;
-    c.A = A.data_ptr();
-    c.B = B.data_ptr();
-    c.D = C.data_ptr();
-    c.RA = RA.defined() ? RA.data_ptr<int>() : nullptr;
-    c.monitor = monitor ? 1 : 0;
-    c.nslices = 1;
-    return c;
 }
 
 void OverlapImpl::GemmAllReduceOverlap(at::Tensor A, at::Tensor B, at::Tensor C, at::Tensor MM, at::Tensor RA,
@@ -371,7 +435,7 @@ void OverlapImpl::GemmAllReduce(at::Tensor A, at::Tensor B, at::Tensor C, int64_
     // (rows that are not 16-byte aligned are stored element by element: once is enough)
     const bool after = reads_from(call, dst, C.numel()) || s.N % 8;
     if (!after) call.deliver = dst;
-    FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+    launch_gemm(call, C, false);
     if (after) bulk_consume(C.data_ptr(), dst, C.numel() * C.element_size());
 }
 

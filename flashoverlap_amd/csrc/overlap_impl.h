@@ -12,9 +12,22 @@
 #include <torch/custom_class.h>
 
 #include <cstdint>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "host_common.h"
+
+// Device memory for the parts of tiles that a GEMM splits over K (fo_gemm_call::workspace).  One per
+// GEMM stream, shared by the objects that launch on it and given back with the last of them: calls on
+// one stream follow each other, and the mutex keeps a call's two launches together when several
+// threads enqueue.  Grows in three steps to at most 64 MiB; a smaller buffer that launches may still
+// be using is kept beside the larger one.
+struct SplitWorkspace {
+    std::mutex mutex;
+    at::Tensor buffer[3];   // 4, 16 and 64 MiB, made when first needed
+    static std::shared_ptr<SplitWorkspace> of_stream(int device, void* stream);
+};
 
 class OverlapImpl : public torch::CustomClassHolder {
   public:
@@ -87,6 +100,9 @@ class OverlapImpl : public torch::CustomClassHolder {
 
     at::Tensor staging_;
     at::Tensor expired_;          // one int32 on the device: expired waits of this object's calls
+    std::shared_ptr<SplitWorkspace> workspace_;
+    int workspace_device_ = -1;
+    void* workspace_stream_ = nullptr;
     at::Tensor group_table_;
     at::Tensor group_start_;      // first slot of every group (device)
     std::vector<int> table_key_;  // cSeg contents + T the tables were built for
@@ -104,6 +120,7 @@ class OverlapImpl : public torch::CustomClassHolder {
     void consume_groups(const at::Tensor& C, void* dst, int64_t tile_elems, const at::Tensor& cseg_cpu,
                         const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int nslices, int64_t slice_stride);
     void bulk_consume(const void* src, void* dst, size_t bytes);
+    void launch_gemm(fo_gemm_call& call, const at::Tensor& like, bool signals);
     int* expired_word(const at::Tensor& like);
     void refuse_checked_capture(const char* who);
     void prepare_call(const at::Tensor& MM, const char* who);

@@ -143,7 +143,17 @@ int fo_gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN,
  *             (scatter mode only) as in fo_wait_consume; group_start is a device
  *             array of G ints, the first slot of every group; group_table is
  *             required.  The layout tile's height must be a multiple of nslices
- *             (a slice is then a whole number of rows), rLDN 1. */
+ *             (a slice is then a whole number of rows), rLDN 1.
+ *   workspace (optional) device memory in which the sums of tiles can be kept
+ *             that are split over K, because there are too few tiles to fill the
+ *             GPU in their round: fo_gemm_workspace says how many bytes this
+ *             shape can use (0: none).  Less is as good as none: the tiles are
+ *             then not split.  Its first FO_WORKSPACE_ZEROED bytes must be zero
+ *             before the first call; every call leaves them zero.  Calls that can
+ *             run at the same time need workspaces of their own.  Results differ
+ *             from those without a workspace by the order of fp32 additions;
+ *             for one shape they are always the same. */
+#define FO_WORKSPACE_ZEROED 4096
 enum fo_gemm_mode { FO_GEMM_PLAIN = 0, FO_GEMM_SIGNAL = 1, FO_GEMM_SCATTER = 2 };
 struct fo_gemm_call {
     int mode, dtype, algo, M, N, K, rLDN;
@@ -162,8 +172,14 @@ struct fo_gemm_call {
     int nslices, slice_first, slice_count;
     long long slice_stride;   /* elements */
     const int* group_start;
+    void* workspace;
+    size_t workspace_bytes;
 };
 int fo_gemm_launch(const struct fo_gemm_call* call, void* stream);
+
+/* Bytes of workspace that a GEMM of this call's mode, algo, M, N and K can use
+ * (pointers are not looked at). */
+int fo_gemm_workspace(const struct fo_gemm_call* call, size_t* bytes);
 
 /* First slot (in issue order, i.e. under an RA made from fo_raster_hint) of the
  * tiles that belong to the last round of workgroups the GPU runs for this shape:
