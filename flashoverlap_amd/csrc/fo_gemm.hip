@@ -504,13 +504,8 @@ __global__ void __launch_bounds__(256) gemm_kernel(const GemmParams p) {
                 const int gcol = col0 + cc * 8;
                 if (row >= p.M || gcol >= p.N) continue;
                 if (p.N & 7) {     // rows of D are not 16-byte aligned
-                    const T* e = (const T*)&v;
-#pragma unroll
-                    for (int k = 0; k < 8; ++k)
-                        if (gcol + k < p.N) {
-                            D[off + k] = e[k];
-                            if (deliver) D2[off + k] = e[k];
-                        }
+                    store_edge_chunk(D + off, v, p.N - gcol);
+                    if (deliver) store_edge_chunk(D2 + off, v, p.N - gcol);
                     continue;
                 }
             }

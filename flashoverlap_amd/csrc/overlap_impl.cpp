@@ -432,8 +432,7 @@ void OverlapImpl::GemmAllReduce(at::Tensor A, at::Tensor B, at::Tensor C, int64_
     c10::DeviceGuard guard(A.device());
     fo_gemm_call call = describe(FO_GEMM_PLAIN, s, Algo, 1, A, B, C, at::Tensor(), false);
     void* dst = staging_like(C).data_ptr();
-    // (rows that are not 16-byte aligned are stored element by element: once is enough)
-    const bool after = reads_from(call, dst, C.numel()) || s.N % 8;
+    const bool after = reads_from(call, dst, C.numel());
     if (!after) call.deliver = dst;
     launch_gemm(call, C, false);
     if (after) bulk_consume(C.data_ptr(), dst, C.numel() * C.element_size());
