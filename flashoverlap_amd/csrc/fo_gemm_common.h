@@ -7,6 +7,7 @@
 #include <type_traits>
 
 #include "fo_internal.h"
+#include "fo_raster.h"
 
 namespace fo {
 
@@ -95,6 +96,13 @@ struct GemmParams {
     float* partial;
     int* arrived;                               // reduction: strips of each layout tile that are stored
 };
+
+// The macro tile that workgroup `tile` of the grid (or the reduction's split tile) computes.
+template <int MTM, int MTN>
+__device__ __forceinline__ TileCoord macro_tile_at(const GemmParams& p, int tile) {
+    if constexpr (MTM > MTN) return raster_map<kGroupM / 2, kUnitN * 2>(tile, p.GM, p.GN, p.gn_magic);
+    else return raster_map(tile, p.GM, p.GN, p.gn_magic);
+}
 
 // Where a part of a split tile lies in `partial`: [tile][split][wave][block i * NB + j][lane] vectors of
 // four floats, i.e. as the accumulators lie in the wavefronts; every access is a contiguous KiB.

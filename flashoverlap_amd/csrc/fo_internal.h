@@ -30,15 +30,17 @@ struct LaunchTimer {
 extern thread_local LaunchTimer t_launch_timer;
 
 // fo_gemm.hip
-int choose_macro_tile(int BM, int BN, int M, int N, bool any_shape);
 int launch_gemm(const fo_gemm_call& c, hipStream_t stream);
 int gemm_workspace(const fo_gemm_call& c, size_t* bytes);
 int last_round(int algo, int M, int N, int* first_slot);
 int raster_hint(int algo, int M, int N, int* hint);
 int tune(const char* key, int value);
 
-// fo_splitk.hip: sums the parts of the split tiles and stores the tiles as the GEMM's epilogue would
+// fo_gemm_tall.hip
 struct GemmParams;
+int launch_gemm_tall(int mode, int dtype, bool edge, const GemmParams& p, const LaunchTimer& timer, hipStream_t stream);
+
+// fo_splitk.hip: sums the parts of the split tiles and stores the tiles as the GEMM's epilogue would
 int launch_split_reduce(int mode, int dtype, int macro, const GemmParams& p, hipStream_t stream);
 
 // fo_static.hip

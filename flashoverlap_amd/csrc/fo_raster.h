@@ -37,7 +37,9 @@ FO_HD int raster_div(int n, unsigned magic) {
     return magic ? (int)(((unsigned long long)(unsigned)n * magic) >> 32) : n;
 }
 
-// pid in [0, GM*GN) -> macro tile coordinate; gn_magic = raster_magic(GN).
+// pid in [0, GM*GN) -> macro tile coordinate; gn_magic = raster_magic(GN).  kGroupM x kUnitN: the
+// unit, 8 x 4 square macro tiles, 4 x 8 of those that are twice as high as wide.
+template <int kGroupM = fo::kGroupM, int kUnitN = fo::kUnitN>
 FO_HD TileCoord raster_map(int pid, int GM, int GN, unsigned gn_magic) {
     const int total = GM * GN;
     const int xcd = pid % kXcds, local = pid / kXcds;

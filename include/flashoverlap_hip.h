@@ -219,9 +219,9 @@ int fo_raster_hint(int algo, int M, int N, int* hint_host);
  *                  for the kernel that reads it next); 1: non-temporal
  *                  everywhere; 0: ordinary everywhere.
  *   "macro_tile"   the tile one workgroup computes.  0 (default): chosen per
- *                  shape (128x128 for outputs of up to 128 tiles of 256x256,
- *                  else 256x256); 128 or 256: forced, 128 only where the
- *                  layout tile is 128x128 or the GEMM is the plain one.  The
+ *                  shape (128x128, 256x128 or 256x256, whichever keeps the GPU
+ *                  busier); 128, 256 or 256128 (256x128): forced, where the
+ *                  layout tile divides it or the GEMM is the plain one.  The
  *                  issue order fo_raster_hint reports follows the setting. */
 int fo_tune(const char* key, int value);
 

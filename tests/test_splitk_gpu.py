@@ -106,3 +106,53 @@ def test_split_signal_and_scatter(dev, M, N, K, algo, ws):
                 assert (mine == 7.0).all()
             else:
                 assert torch.equal(mine, rows[r0 + k * nr // ws:r0 + (k + 1) * nr // ws])
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 128, 64), (384, 256, 72), (8, 136, 128), (600, 385, 200), (1536, 2048, 192)])
+def test_tall_tile_gives_the_bits_of_the_square_one(dev, M, N, K):
+    """The 256x128 macro tile on one, two and three panels, half and ragged tiles: the order of additions is the same."""
+    L = capi.lib()
+    g = torch.Generator().manual_seed(M + N + K)
+    A, B = (torch.randn(r, K, generator=g).to(torch.bfloat16).to(dev) for r in (M, N))
+    got = []
+    try:
+        for macro in (128, 256128):
+            capi.check(L.fo_tune(b"macro_tile", macro))
+            D = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=dev)
+            capi.check(L.fo_gemm(capi.FO_BF16, 1, M, N, K, A.data_ptr(), B.data_ptr(), D.data_ptr(), None))
+            torch.cuda.synchronize()
+            got.append(D)
+    finally:
+        capi.check(L.fo_tune(b"macro_tile", 0))
+    assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("M,N,algo", [(512, 512, 1), (384, 640, 1), (512, 384, 4), (640, 512, 0)])
+@pytest.mark.parametrize("ws", [1, 4])
+def test_tall_tile_signals_and_places(dev, M, N, algo, ws):
+    L = capi.lib()
+    K, dt = 136, torch.float16
+    BM, BN, _ = capi.algo_tile(algo)
+    TM, TN = M // BM, N // BN
+    A, B, want = _operands(dev, dt, M, N, K)
+    cseg = tiling.uniform_cseg(TM * TN, 3)
+    RA = torch.randperm(TM * TN, generator=torch.Generator().manual_seed(3)).int().to(dev)
+    RE = tiling.generate_row_remap_array(M, N, BM, BN, cseg, ws, dev)
+    cs = torch.tensor(cseg, dtype=torch.int32, device=dev)
+    mm = torch.zeros(len(cseg), dtype=torch.int32, device=dev)
+    D = torch.full((M * N // BN, BN), 7.0, dtype=dt, device=dev)
+    c = capi.GemmCall(mode=2 if ws > 1 else 1, dtype=capi.dtype_code(dt), algo=algo, M=M, N=N, K=K, rLDN=1,
+                      cseg_dev=cs.data_ptr(), G=len(cseg), A=A.data_ptr(), B=B.data_ptr(), D=D.data_ptr(),
+                      MM=mm.data_ptr(), RA=RA.data_ptr(), RE=RE.data_ptr(), nslices=ws)
+    try:
+        capi.check(L.fo_tune(b"macro_tile", 256128))
+        capi.check(L.fo_gemm_launch(C.byref(c), None))
+        torch.cuda.synchronize()
+    finally:
+        capi.check(L.fo_tune(b"macro_tile", 0))
+    assert mm.cpu().tolist() == cseg
+    rows = torch.empty(TM * TN, BM, BN, dtype=dt, device=dev)
+    rows[RA.long()] = want.view(TM, BM, TN, BN).permute(0, 2, 1, 3).reshape(TM * TN, BM, BN)
+    out = torch.empty(TM * TN * BM, BN, dtype=dt, device=dev)
+    out[RE.long() if ws > 1 else slice(None)] = rows.view(-1, BN)
+    assert torch.equal(D, out)
