@@ -126,9 +126,13 @@ static int plan_for(const fo_gemm_call& c, bool workspace, Plan* plan) {
     return FO_OK;
 }
 
+// A few rows of A: a kernel of its own, unless a macro tile is asked for.
+static bool is_skinny(const fo_gemm_call& c) { return c.mode == kPlain && c.M <= kSkinnyRows && !knob(knobs().macro_tile); }
+
 int gemm_workspace(const fo_gemm_call& c, size_t* bytes) {
     *bytes = 0;
     if (c.M <= 0 || c.N <= 0 || c.K <= 0) return fail(FO_ERR_SHAPE, "fo_gemm_workspace: empty problem %dx%dx%d", c.M, c.N, c.K);
+    if (is_skinny(c)) return FO_OK;
     Plan plan;
     if (int e = plan_for(c, true, &plan)) return e;
     *bytes = plan.bytes;
@@ -206,6 +210,7 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
         }
     }
     if ((uintptr_t)c.deliver & 15) return fail(FO_ERR_ARG, "fo_gemm: operands must be 16-byte aligned");
+    if (is_skinny(c)) return launch_skinny(dtype, M, N, K, A, B, D, c.deliver, timer, stream);
     Plan plan;
     if (int e = plan_for(c, c.workspace && !timer.start, &plan)) return e;
     if (c.workspace_bytes < plan.bytes)

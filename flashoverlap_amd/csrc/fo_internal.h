@@ -40,6 +40,11 @@ int tune(const char* key, int value);
 struct GemmParams;
 int launch_gemm_tall(int mode, int dtype, bool edge, const GemmParams& p, const LaunchTimer& timer, hipStream_t stream);
 
+// fo_skinny.hip: the plain GEMM for M <= kSkinnyRows
+constexpr int kSkinnyRows = 32;
+int launch_skinny(int dtype, int M, int N, int K, const void* A, const void* B, void* D, void* D2, const LaunchTimer& timer,
+                  hipStream_t stream);
+
 // fo_splitk.hip: sums the parts of the split tiles and stores the tiles as the GEMM's epilogue would
 int launch_split_reduce(int mode, int dtype, int macro, const GemmParams& p, hipStream_t stream);
 
