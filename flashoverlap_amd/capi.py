@@ -40,7 +40,9 @@ SIGNATURES = {
     "fo_gemm_signal_static": (_i, [_i, _i, _i, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp]),
     "fo_gemm_launch": (_i, [C.POINTER(GemmCall), _vp]),
     "fo_gemm_workspace": (_i, [C.POINTER(GemmCall), C.POINTER(_sz)]),
-    "fo_gemm_last_round": (_i, [_i, _i, _i, _ip]),
+    "fo_gemm_rounds": (_i, [_i, _i, _i, _ip, _ip]),
+    "fo_wait_groups": (_i, [_vp, _i, _i, _vp, _vp, _vp]),
+    "fo_consume_groups": (_i, [_vp, _vp, _i, _i, _vp, _vp, _ll, _i, _i, _i, _ll, _i, _sz, _vp]),
     "fo_build_group_table": (_i, [_vp, _i, _i, _vp, _vp]),
     "fo_raster_hint": (_i, [_i, _i, _i, _ip]),
     "fo_tune": (_i, [C.c_char_p, _i]),

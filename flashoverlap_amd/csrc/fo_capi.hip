@@ -104,7 +104,9 @@ int fo_gemm_workspace(const struct fo_gemm_call* call, size_t* bytes) {
     return gemm_workspace(*call, bytes);
 }
 
-int fo_gemm_last_round(int algo, int M, int N, int* first_slot) { return last_round(algo, M, N, first_slot); }
+int fo_gemm_rounds(int algo, int M, int N, int* per_round, int* last_first) {
+    return gemm_rounds(algo, M, N, per_round, last_first);
+}
 
 int fo_gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg_dev, int G,
                           const void* A, const void* B, void* D, int* MM, const int* RA, int monitor, void* stream) {
@@ -128,6 +130,17 @@ int fo_wait_consume(const int* cseg_dev, int G, int* MM, const void* src, void* 
                     int nblocks, int* expired, void* stream) {
     return launch_wait_consume(cseg_dev, G, MM, src, dst, tile_elems, nslices, slice_first, slice_count,
                                slice_stride, order_log, nblocks, expired, (hipStream_t)stream);
+}
+
+int fo_wait_groups(const int* cseg_dev, int group_first, int groups, int* MM, int* expired, void* stream) {
+    return launch_wait_groups(cseg_dev, group_first, groups, MM, expired, (hipStream_t)stream);
+}
+
+int fo_consume_groups(const int* cseg_dev, const int* group_start, int group_first, int groups, const void* src, void* dst,
+                      long long tile_elems, int nslices, int slice_first, int slice_count, long long slice_stride,
+                      int store_policy, size_t total_bytes, void* stream) {
+    return launch_consume_groups(cseg_dev, group_start, group_first, groups, src, dst, tile_elems, nslices, slice_first,
+                                 slice_count, slice_stride, store_policy, total_bytes, (hipStream_t)stream);
 }
 
 int fo_set_wait_timeout_ms(int ms) { return set_wait_timeout_ms(ms); }

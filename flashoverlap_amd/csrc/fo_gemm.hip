@@ -234,19 +234,19 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
     return rc;
 }
 
-int last_round(int algo, int M, int N, int* first_slot) {
+int gemm_rounds(int algo, int M, int N, int* per_round, int* last_first) {
     int BM, BN, BK;
-    if (!first_slot) return fail(FO_ERR_ARG, "fo_gemm_last_round: null output");
-    if (algo_tile(algo, &BM, &BN, &BK) != FO_OK) return fail(FO_ERR_ARG, "fo_gemm_last_round: Algo %d out of range", algo);
-    if (M <= 0 || N <= 0 || M % BM || N % BN) return fail(FO_ERR_SHAPE, "fo_gemm_last_round: M=%d N=%d vs tile %dx%d", M, N, BM, BN);
+    if (!per_round || !last_first) return fail(FO_ERR_ARG, "fo_gemm_rounds: null output");
+    if (algo_tile(algo, &BM, &BN, &BK) != FO_OK) return fail(FO_ERR_ARG, "fo_gemm_rounds: Algo %d out of range", algo);
+    if (M <= 0 || N <= 0 || M % BM || N % BN) return fail(FO_ERR_SHAPE, "fo_gemm_rounds: M=%d N=%d vs tile %dx%d", M, N, BM, BN);
     const DeviceFacts* facts;
     if (int e = device_facts(&facts)) return e;
     const Macro t = hint_macro(BM, BN, M, N);
     const long long total = (long long)((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
     const long long at_once = (long long)facts->cus * (t.m == 256 ? 1 : 2);   // workgroups a CU holds: LDS
-    const long long before = (total - 1) / at_once * at_once;
-    const long long T = (long long)(M / BM) * (N / BN);
-    *first_slot = (int)((T * before + total - 1) / total);   // half macro tiles at the edges make it approximate: it is a hint
+    const long long T = (long long)(M / BM) * (N / BN);   // half macro tiles at the edges make the slots approximate: hints
+    *per_round = (int)((T * at_once + total - 1) / total);
+    *last_first = (int)((T * ((total - 1) / at_once * at_once) + total - 1) / total);
     return FO_OK;
 }
 

@@ -32,7 +32,7 @@ extern thread_local LaunchTimer t_launch_timer;
 // fo_gemm.hip
 int launch_gemm(const fo_gemm_call& c, hipStream_t stream);
 int gemm_workspace(const fo_gemm_call& c, size_t* bytes);
-int last_round(int algo, int M, int N, int* first_slot);
+int gemm_rounds(int algo, int M, int N, int* per_round, int* last_first);
 int raster_hint(int algo, int M, int N, int* hint);
 int tune(const char* key, int value);
 
@@ -60,6 +60,10 @@ int launch_wait_consume(const int* cseg, int G, int* MM, const void* src, void* 
                         int nblocks, int* expired, hipStream_t stream);
 int launch_consume(const void* src, void* dst, size_t bytes, hipStream_t stream, int that = 0, int* addr = nullptr,
                    int nslices = 1, size_t dst_stride_bytes = 0, int policy = FO_COPY_AUTO, int* expired = nullptr);
+int launch_wait_groups(const int* cseg, int first, int groups, int* MM, int* expired, hipStream_t stream);
+int launch_consume_groups(const int* cseg, const int* gstart, int first, int groups, const void* src, void* dst,
+                          long long tile_elems, int nslices, int slice_first, int slice_count, long long slice_stride,
+                          int policy, size_t total_bytes, hipStream_t stream);
 int set_wait_timeout_ms(int ms);
 int wait_timeouts(int* count, int reset);
 

@@ -59,6 +59,19 @@ __global__ void wait_kernel(int that, int* addr, long long ticks, int* expired) 
         count_expired(expired);
 }
 
+// The same for several groups that complete together, a lane to a group.
+__global__ void wait_groups_kernel(const int* __restrict__ cseg, int groups, int* MM, long long ticks, int* expired) {
+    for (int g = threadIdx.x; g < groups; g += blockDim.x) {
+        const int need = cseg[g];
+        if (bounded_poll(MM + g, ticks, [need](int v) { return v == need; })) {
+            __hip_atomic_store(MM + g, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            count_expired(expired);
+            ticks = -1;   // this lane's later groups are looked at once
+        }
+    }
+}
+
 constexpr int kCopyThreads = 512;  // workgroup size of the per-group copy kernel
 constexpr int kCopyUnroll = 8;     // 16-byte units in flight per thread
 constexpr int kWavesPerBlock = 4;  // persistent consumer: one wavefront per SIMD
@@ -254,6 +267,18 @@ __global__ void __launch_bounds__(kCopyThreads) consume_kernel(const uint4* __re
     if (blockIdx.x == 0 && (int)threadIdx.x < tail) dst_tail[threadIdx.x] = src_tail[threadIdx.x];   // one slice only
 }
 
+// The copies of several groups: blockIdx.y is (group, slice).
+template <bool STREAM>
+__global__ void __launch_bounds__(kCopyThreads) consume_groups_kernel(const int* __restrict__ cseg, const int* __restrict__ gstart,
+                                                                      int first, const uint4* __restrict__ src,
+                                                                      uint4* __restrict__ dst, long long tile_units, int nslices,
+                                                                      int slice_first, int slice_count, long long stride_units) {
+    const int g = first + blockIdx.y / slice_count, k = blockIdx.y % slice_count;
+    const long long part = tile_units * cseg[g] / nslices, lo = tile_units * gstart[g];
+    team_copy<kCopyThreads, STREAM>(src + lo + (slice_first + k) * part, dst + k * stride_units + lo / nslices, part, blockIdx.x,
+                                    gridDim.x, threadIdx.x);
+}
+
 // table[s] = number of inclusive prefix sums of cseg that are <= s, i.e. what
 // the linear scan in src/overlap/gemm_with_signal.h:188-193 returns.  One
 // workgroup: per-thread run sums, a block scan, then each thread fills the
@@ -337,6 +362,17 @@ int launch_wait(int that, int* addr, int* expired, hipStream_t stream) {
     return FO_OK;
 }
 
+int launch_wait_groups(const int* cseg, int first, int groups, int* MM, int* expired, hipStream_t stream) {
+    if (!cseg || !MM) return fail(FO_ERR_ARG, "fo_wait_groups: null argument");
+    if (first < 0 || groups <= 0) return fail(FO_ERR_ARG, "fo_wait_groups: groups [%d, %d)", first, first + groups);
+    long long ticks;
+    if (int e = ticks_for_timeout(&ticks)) return e;
+    hipLaunchKernelGGL(wait_groups_kernel, dim3(1), dim3(groups <= 64 ? 64 : 256), 0, stream, cseg + first, groups, MM + first,
+                       ticks, expired);
+    FO_HIP(hipGetLastError());
+    return FO_OK;
+}
+
 int launch_wait_consume(const int* cseg, int G, int* MM, const void* src, void* dst, long long tile_elems,
                         int nslices, int slice_first, int slice_count, long long slice_stride, int* order_log,
                         int nblocks, int* expired, hipStream_t stream) {
@@ -364,6 +400,8 @@ int launch_wait_consume(const int* cseg, int G, int* MM, const void* src, void* 
     return FO_OK;
 }
 
+constexpr size_t kStreamFrom = 48u << 20;   // FO_COPY_AUTO: launches of this size store past the caches
+
 int launch_consume(const void* src, void* dst, size_t bytes, hipStream_t stream, int that, int* addr, int nslices,
                    size_t dst_stride_bytes, int policy, int* expired) {
     const char* who = nslices > 1 ? "fo_consume_slices" : "fo_consume";
@@ -388,7 +426,6 @@ int launch_consume(const void* src, void* dst, size_t bytes, hipStream_t stream,
     // that knows the whole call says which it wants; left to itself a launch goes by its own size, and
     // one that settles its own counter follows its GEMM and is read next, so it stores normally.
     if (policy < FO_COPY_AUTO || policy > FO_COPY_CACHED) return fail(FO_ERR_ARG, "%s: store policy %d", who, policy);
-    constexpr size_t kStreamFrom = 48u << 20;
     bool stream_stores = policy == FO_COPY_STREAM ||
                          (policy == FO_COPY_AUTO && !addr && bytes * (size_t)nslices >= kStreamFrom);
     if (const int forced = knob(knobs().copy_streaming_stores); forced != 2) stream_stores = forced == 1;   // fo_tune
@@ -397,6 +434,34 @@ int launch_consume(const void* src, void* dst, size_t bytes, hipStream_t stream,
                        (uint4*)dst, (long long)units, (long long)(dst_stride_bytes / 16),
                        (const unsigned short*)((const char*)src + units * 16),
                        (unsigned short*)((char*)dst + units * 16), tail, that, addr, expired);
+    FO_HIP(hipGetLastError());
+    return FO_OK;
+}
+
+int launch_consume_groups(const int* cseg, const int* gstart, int first, int groups, const void* src, void* dst,
+                          long long tile_elems, int nslices, int slice_first, int slice_count, long long slice_stride,
+                          int policy, size_t total_bytes, hipStream_t stream) {
+    const char* who = "fo_consume_groups";
+    if (!cseg || !gstart || !src || !dst) return fail(FO_ERR_ARG, "%s: null argument", who);
+    if (first < 0 || groups <= 0 || nslices <= 0 || tile_elems <= 0)
+        return fail(FO_ERR_ARG, "%s: groups [%d, %d) nslices=%d tile_elems=%lld", who, first, first + groups, nslices, tile_elems);
+    if (tile_elems % (8LL * nslices)) return fail(FO_ERR_SHAPE, "%s: a tile (%lld elements) must split into %d slices of whole 16-byte units", who, tile_elems, nslices);
+    if (slice_first < 0 || slice_count <= 0 || slice_first + slice_count > nslices)
+        return fail(FO_ERR_ARG, "%s: slices [%d, %d) outside 0..%d", who, slice_first, slice_first + slice_count, nslices);
+    if (slice_count > 1 && slice_stride % 8) return fail(FO_ERR_SHAPE, "%s: slice_stride=%lld not a multiple of 8 elements", who, slice_stride);
+    if ((long long)groups * slice_count > 65535) return fail(FO_ERR_LIMIT, "%s: %d groups of %d slices", who, groups, slice_count);
+    if (((uintptr_t)src | (uintptr_t)dst) & 15) return fail(FO_ERR_ARG, "%s: buffers must be 16-byte aligned", who);
+    if (policy < FO_COPY_AUTO || policy > FO_COPY_CACHED) return fail(FO_ERR_ARG, "%s: store policy %d", who, policy);
+    bool stream_stores = policy == FO_COPY_STREAM || (policy == FO_COPY_AUTO && total_bytes >= kStreamFrom);
+    if (const int forced = knob(knobs().copy_streaming_stores); forced != 2) stream_stores = forced == 1;   // fo_tune
+    // workgroups per group: about 1024 in all, no more than the bytes of an average group are worth
+    const size_t ranges = (size_t)groups * slice_count, per_block = (size_t)kCopyThreads * kCopyUnroll * 16;
+    size_t blocks = total_bytes ? (total_bytes / ranges + per_block - 1) / per_block : 8;
+    if (blocks > 1024 / ranges) blocks = 1024 / ranges;
+    if (blocks == 0) blocks = 1;
+    auto kern = stream_stores ? consume_groups_kernel<true> : consume_groups_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)ranges), dim3(kCopyThreads), 0, stream, cseg, gstart, first,
+                       (const uint4*)src, (uint4*)dst, tile_elems / 8, nslices, slice_first, slice_count, slice_stride / 8);
     FO_HIP(hipGetLastError());
     return FO_OK;
 }

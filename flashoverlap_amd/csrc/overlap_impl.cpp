@@ -280,7 +280,7 @@ void OverlapImpl::refuse_checked_capture(const char* who) {
 }
 
 void OverlapImpl::fork_comm_stream(int waited, int G) {
-    if (waited == 0 || (waited == G && G <= 1 && !persistent_consumer(waited))) return;   // the second stream is not used
+    if (waited == 0 || (waited == G && G <= 1 && consumer_mode_ != 2)) return;   // the second stream is not used
     int capturing = 0;
     FO_CALL(fo_stream_is_capturing(gemm_stream_, &capturing));
     if (capturing) FO_CALL(fo_stream_join(gemm_stream_, comm_stream_));
@@ -294,32 +294,39 @@ void OverlapImpl::fork_comm_stream(int waited, int G) {
 // behind a GEMM of 97).  The epilogue has these tiles in registers and stores them twice instead.
 // Checked mode and monitor mode keep every group on its counter (the first reports a count that
 // does not come out, the second takes its tickets from the signals), and so do the explicit modes.
-int OverlapImpl::groups_to_wait_for(const fo_gemm_call& call, const int* cseg, int nslices, int* first_slot) {
+int OverlapImpl::groups_to_wait_for(const fo_gemm_call& call, const int* cseg, int nslices, int* first_slot,
+                                    int* per_round) {
     int BM, BN, BK, late = 0;
     FO_CALL(fo_algo_tile(call.algo, &BM, &BN, &BK));
     if (consumer_mode_ != 0 || check_timeouts_ || call.monitor || BM % nslices) return call.G;
-    FO_CALL(fo_gemm_last_round(call.algo, call.M, call.N, &late));
+    FO_CALL(fo_gemm_rounds(call.algo, call.M, call.N, per_round, &late));
     int g = 0, slot = 0;
     while (g + 1 < call.G && slot < late) slot += cseg[g++];
     *first_slot = slot;
     return g;
 }
 
-// Per-group release: either the reference's host loop (one wait kernel and one
-// consumer launch per group, src/overlap_impl.cu:257-265 / 312-323) or one
-// persistent kernel that does the same walk on the device.  On return the GEMM
-// stream is ordered behind every group's copy.  The first `waited` groups are
-// released here; the others have been delivered by the GEMM itself.
+// Release of the first `waited` groups (the others have been delivered by the GEMM itself): the
+// reference's host loop (one wait kernel and one consumer launch per group,
+// src/overlap_impl.cu:257-265 / 312-323), the same with one pair of launches for the groups of a round
+// (per_round slots), or one persistent kernel that does the walk on the device.  On return the GEMM
+// stream is ordered behind every group's copy.
+//
+// Groups of one round fill their counters at the same moment, and a pair of launches of their own
+// each then only queues up, on the host too: 15104x1280x2936 fp16 in 13 groups of 98 tiles took 222 us
+// with its norm, 133 of them of the host, and takes 165; 7424x6016x640 in 5 of 302 148 -> 130, 9856x6400x1408
+// in 14 of 275 253 -> 230.  It also leaves the automatic mode without the persistent kernel, of which
+// two (of two objects, on two streams) can hold the registers that a GEMM they wait for needs.
 void OverlapImpl::consume_groups(const at::Tensor& C, void* dst, int64_t tile_elems, const at::Tensor& cseg_cpu,
-                                 const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int nslices,
-                                 int64_t slice_stride) {
+                                 const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int per_round,
+                                 int nslices, int64_t slice_stride) {
     const int G = (int)cseg_cpu.numel();
     const int* cseg = cseg_cpu.data_ptr<int>();
     const int slice_first = slice_stride ? 0 : (int)my_rank_;      // stride 0: only this rank's slice
     const int slice_count = slice_stride ? nslices : 1;
     int* expired = expired_.data_ptr<int>();   // this object's own count of expired waits (prepare_call)
     if (waited == 0) return;
-    if (persistent_consumer(waited)) {
+    if (consumer_mode_ == 2) {
         FO_CALL(fo_wait_consume(cseg_gpu.data_ptr<int>(), waited, MM.data_ptr<int>(), C.data_ptr(), dst, tile_elems,
                                 nslices, slice_first, slice_count, slice_stride, nullptr, consumer_blocks(),
                                 expired, comm_stream_));
@@ -347,6 +354,22 @@ void OverlapImpl::consume_groups(const at::Tensor& C, void* dst, int64_t tile_el
         const bool last = g == G - 1;
         void* stream = last ? gemm_stream_ : comm_stream_;
         const int64_t comm = tile_elems * cseg[g];
+        // the groups up to `end` complete in the round in which this one does
+        int end = g + 1;
+        int64_t tiles = cseg[g];
+        if (per_round)
+            while (end < waited && end + 1 < G && (int64_t)(end - g + 1) * slice_count < 65536 &&
+                   (acc / tile_elems + tiles + cseg[end] - 1) / per_round == (acc / tile_elems + cseg[g] - 1) / per_round)
+                tiles += cseg[end++];
+        if (end > g + 1) {
+            FO_CALL(fo_wait_groups(cseg_gpu.data_ptr<int>(), g, end - g, MM.data_ptr<int>(), expired, stream));
+            FO_CALL(fo_consume_groups(cseg_gpu.data_ptr<int>(), group_start_.data_ptr<int>(), g, end - g, src, dst, tile_elems,
+                                      nslices, slice_first, slice_count, slice_stride, beside_policy,
+                                      tile_elems * tiles * esz / nslices * slice_count, stream));
+            acc += tile_elems * tiles;
+            g = end - 1;
+            continue;
+        }
         if (!last) FO_CALL(fo_wait(cseg[g], MM.data_ptr<int>() + g, expired, stream));
         // One launch per group, like the one collective call per group of the reference: this
         // rank's slice of the group, or all ranks' slices into their receive buffers side by side.
@@ -372,9 +395,10 @@ void OverlapImpl::overlapped_call(fo_gemm_call& call, const fo_host::SignalShape
     call.group_table = group_table_for(cseg_cpu, cseg_gpu, g.T);
     call.MM = MM.data_ptr<int>();
     const int64_t kept = (int64_t)call.M * call.N / (slice_stride ? 1 : call.nslices);
-    const int waited = reads_from(call, dst, kept)
-                           ? g.G
-                           : groups_to_wait_for(call, cseg_cpu.data_ptr<int>(), call.nslices, &call.deliver_from);
+    int per_round = 0;
+    const int waited = reads_from(call, dst, kept) ? g.G
+                                                   : groups_to_wait_for(call, cseg_cpu.data_ptr<int>(), call.nslices,
+                                                                        &call.deliver_from, &per_round);
     if (waited < g.G) {
         call.deliver = dst;
         call.group_start = group_start_.data_ptr<int>();
@@ -384,7 +408,7 @@ void OverlapImpl::overlapped_call(fo_gemm_call& call, const fo_host::SignalShape
     }
     fork_comm_stream(waited, g.G);
     launch_gemm(call, C, waited > 0);
-    consume_groups(C, dst, (int64_t)g.BM * g.BN, cseg_cpu, cseg_gpu, MM, waited, call.nslices, slice_stride);
+    consume_groups(C, dst, (int64_t)g.BM * g.BN, cseg_cpu, cseg_gpu, MM, waited, per_round, call.nslices, slice_stride);
     raise_on_timeout(MM, who);
 }
 

@@ -69,8 +69,9 @@ class OverlapImpl : public torch::CustomClassHolder {
     // caller can own its result like it owns C in the reference.  A call whose C
     // does not match the buffer in size, dtype or device goes back to an internal one.
     void SetStaging(at::Tensor buffer);
-    // 0 = automatic (groups that complete with the GEMM are delivered by its epilogue; the
-    // others: per-group launches up to 32 groups, one persistent kernel beyond), 1 = one (wait, consume) launch pair per group like the
+    // 0 = automatic (groups that complete with the GEMM are delivered by its epilogue; of the
+    // others, those that complete in one round of workgroups are released together, with one
+    // wait and one copy launch), 1 = one (wait, consume) launch pair per group like the
     // reference's host loop, 2 = one persistent wait+consume kernel.
     void SetConsumerMode(int64_t mode);
     // Workgroups of the persistent consumer (default and maximum: one per CU).
@@ -114,11 +115,10 @@ class OverlapImpl : public torch::CustomClassHolder {
     void overlapped_call(fo_gemm_call& call, const fo_host::SignalShape& g, const at::Tensor& C, void* dst,
                          const at::Tensor& cseg_cpu, const at::Tensor& cseg_gpu, at::Tensor& MM, int64_t slice_stride,
                          const char* who);
-    bool persistent_consumer(int groups) const { return consumer_mode_ == 2 || (consumer_mode_ == 0 && groups > 32); }
-    int groups_to_wait_for(const fo_gemm_call& call, const int* cseg, int nslices, int* first_slot);
+    int groups_to_wait_for(const fo_gemm_call& call, const int* cseg, int nslices, int* first_slot, int* per_round);
     void fork_comm_stream(int waited, int G);
     void consume_groups(const at::Tensor& C, void* dst, int64_t tile_elems, const at::Tensor& cseg_cpu,
-                        const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int nslices, int64_t slice_stride);
+                        const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int per_round, int nslices, int64_t slice_stride);
     void bulk_consume(const void* src, void* dst, size_t bytes);
     void launch_gemm(fo_gemm_call& call, const at::Tensor& like, bool signals);
     int* expired_word(const at::Tensor& like);

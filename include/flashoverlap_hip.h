@@ -181,10 +181,11 @@ int fo_gemm_launch(const struct fo_gemm_call* call, void* stream);
  * (pointers are not looked at). */
 int fo_gemm_workspace(const struct fo_gemm_call* call, size_t* bytes);
 
-/* First slot (in issue order, i.e. under an RA made from fo_raster_hint) of the
- * tiles that belong to the last round of workgroups the GPU runs for this shape:
- * the tiles that finish together, when the GEMM ends. */
-int fo_gemm_last_round(int algo, int M, int N, int* first_slot);
+/* The rounds of workgroups in which the GPU computes this shape, in slots (in
+ * issue order, i.e. under an RA made from fo_raster_hint): tiles of one round
+ * finish together.  per_round: slots of a round; last_first: first slot of the
+ * last round, whose tiles finish when the GEMM ends. */
+int fo_gemm_rounds(int algo, int M, int N, int* per_round, int* last_first);
 
 /* group_table[s] = group(s) for s in [0,T), computed on the device from
  * cseg_dev.  No counterpart in the reference, whose epilogue rescans cSeg for
@@ -269,6 +270,21 @@ int fo_wait_consume(const int* cseg_dev, int G, int* MM,
                     const void* src, void* dst, long long tile_elems,
                     int nslices, int slice_first, int slice_count, long long slice_stride,
                     int* order_log, int nblocks, int* expired, void* stream);
+
+/* fo_wait for the groups [group_first, group_first + groups) in one launch, and
+ * the copies behind such a wait in another: groups that complete together (in one
+ * round of workgroups, fo_gemm_rounds) need no launches of their own.
+ * fo_wait_groups returns once MM[g] == cseg_dev[g] for all of them and leaves
+ * zeros; a group whose wait expires is left as it is and counted, and the ones
+ * after it are looked at once.  fo_consume_groups copies the slices of each group
+ * as fo_wait_consume does (cseg_dev, group_start: device arrays of all groups;
+ * store_policy as in fo_consume_slices, total_bytes: of all its copies together,
+ * or 0 for what FO_COPY_AUTO need not know).  No counterpart in the reference,
+ * which launches a wait and a collective per group (src/overlap_impl.cu:257-265). */
+int fo_wait_groups(const int* cseg_dev, int group_first, int groups, int* MM, int* expired, void* stream);
+int fo_consume_groups(const int* cseg_dev, const int* group_start, int group_first, int groups, const void* src, void* dst,
+                      long long tile_elems, int nslices, int slice_first, int slice_count, long long slice_stride,
+                      int store_policy, size_t total_bytes, void* stream);
 
 int fo_set_wait_timeout_ms(int ms);
 /* Number of bounded waits that were given no `expired` word of their own and

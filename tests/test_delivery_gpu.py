@@ -93,14 +93,46 @@ def test_serial_call_delivers_what_it_stores(api, dev, M, N, K):
         assert torch.equal(c, want) and torch.equal(A.view(-1)[:M * N].view(M, N), want)
 
 
-def test_last_round_of_a_shape(dev):
+def test_rounds_of_a_shape(dev):
     """288 macro tiles on 256 CUs: the last round starts at macro tile 256, layout tile 1024 in issue order."""
-    n = C.c_int()
-    capi.check(capi.lib().fo_gemm_last_round(1, 8192, 2304, C.byref(n)))
-    cus = C.c_int()
+    per, late, cus = C.c_int(), C.c_int(), C.c_int()
+    rounds = capi.lib().fo_gemm_rounds
     capi.check(capi.lib().fo_device_info(C.byref(cus), None, None))
+    capi.check(rounds(1, 8192, 2304, C.byref(per), C.byref(late)))
     if cus.value == 256:
-        assert n.value == 1024
-    capi.check(capi.lib().fo_gemm_last_round(1, 1024, 1024, C.byref(n)))
-    assert n.value == 0
-    assert capi.lib().fo_gemm_last_round(1, 100, 1024, C.byref(n)) == capi.FO_ERR_SHAPE
+        assert (per.value, late.value) == (1024, 1024)
+    capi.check(rounds(1, 1024, 1024, C.byref(per), C.byref(late)))
+    assert late.value == 0
+    assert rounds(1, 100, 1024, C.byref(per), C.byref(late)) == capi.FO_ERR_SHAPE
+
+
+@pytest.mark.parametrize("ws,stacked", [(1, False), (4, False), (4, True)])
+@pytest.mark.parametrize("group", [13, 100, 700])
+def test_groups_of_a_round_released_together(api, dev, ws, stacked, group):
+    """Two whole rounds and a bit: the groups of a round take one wait and one copy launch; with 13 tiles
+    to a group there are more groups to a round than lanes to a wavefront."""
+    M, N, K, algo, dt = 8192, 4352, 64, 1, torch.float16
+    BM, BN, _ = capi.algo_tile(algo)
+    TM, TN = M // BM, N // BN
+    cseg = tiling.uniform_cseg(TM * TN, group)
+    cs = torch.tensor(cseg, dtype=torch.int32)
+    RA = tiling.reorder_indices(TM * TN, tiling.raster_hint(M, N, algo), dev).reshape(TM, TN)
+    RE = tiling.generate_row_remap_array(M, N, BM, BN, cseg, ws, dev) if ws > 1 else None
+    A, B = _inputs(dev, dt, M, N, K)
+    got = []
+    for mode in (1, 0):
+        o = _object(api, mode, ws - 2 if ws > 1 else 0, ws)
+        mm = torch.zeros(len(cseg), dtype=torch.int32, device=dev)
+        c = torch.full((M, N), 7.0, dtype=dt, device=dev)
+        d = torch.full(((ws if stacked else 1) * M // ws, N), 7.0, dtype=dt, device=dev)
+        o.set_staging(d)
+        torch.cuda.synchronize()
+        for _ in range(2):
+            if ws > 1:
+                o.gemm_reducescatter_overlap(A, B, c, d, mm, RA, RE, 1, cs, cs.to(dev), algo, False)
+            else:
+                o.gemm_allreduce_overlap(A, B, c, mm, RA, 1, cs, cs.to(dev), algo, False)
+        torch.cuda.synchronize()
+        assert o.wait_timeouts(True) == 0 and not mm.any()
+        got.append((c, d))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
