@@ -71,40 +71,55 @@ struct Plan {
 // Microseconds of a k-step of 64 of a macro tile, and of a round's start and end (launch, first panels,
 // stores).  Measured on shapes from 1024x1024x1024 to 8192x4096x7168, bf16 and fp16: with more than
 // three quarters of the CUs at work the chip comes to its power limit, and the k-steps get longer.
-// 2048x4096x7168 bf16: 114 us in 128x128 tiles, 101 in 256x128, 130 in 256x256; 4096x4096x4096: 116, 101, 90.
-static double panel_us(Macro t, double busy) {   // busy: share of the CUs
+// 2048x4096x7168 bf16: 114 us in 128x128 tiles, 101 in 256x128, 130 in 256x256; 4096x4096x4096: 116, 101, 90;
+// 1024x1024x1024: 9.2 in 64x64, 11.0 in 128x128.
+// straddle: rows that do not start on cache lines (K no multiple of 64) ask the L2 for every line twice,
+// which the smaller tiles feel (2304x1664x5424: 77 us in 256x128 tiles, 55 in 128x128).
+static double panel_us(Macro t, double busy, bool straddle) {   // busy: share of the CUs
     const double hot = busy <= 0.75 ? 0.0 : busy >= 1.0 ? 1.0 : (busy - 0.75) * 4;
     if (t.n == 256) return 1.08 + 0.28 * hot;
-    return t.m == 256 ? 0.61 + 0.25 * hot : 0.46 + 0.06 * hot;
+    if (t.n == 64) return (busy <= 1.0 ? 0.37 : 0.41) + 0.1 * straddle;   // (the copies' latency; of two on a CU each hides the other's)
+    return t.m == 256 ? 0.61 + 0.25 * (straddle ? 1.0 : hot) : 0.46 + 0.06 * hot + 0.13 * straddle;
 }
-static double round_us(Macro t) { return t.n == 256 ? 7.0 : t.m == 256 ? 5.0 : 3.5; }
+static double round_us(Macro t) { return t.n == 256 ? 7.0 : t.m == 256 ? 5.0 : t.n == 128 ? 3.5 : 3.0; }
 
 // The plan whose estimated time is the smallest.  A round of workgroups takes as long if it is not
 // full; of a round that is at most half full the tiles can be split over K instead, if the parts
 // (which write MT * MT floats each, and are read again by a second launch) stay worth it.
-static Plan make_plan(int BM, int BN, int M, int N, int K, bool any_shape, bool may_split, bool may_be_tall, int cus) {
+static Plan make_plan(int BM, int BN, int M, int N, int K, bool any_tile, bool may_split, bool all_tiles, int cus) {
     const int panels = (K + kBK - 1) / kBK;
+    const bool straddle = K % kBK != 0;
     Plan best{};
     double best_us = 1e30;
-    const Macro forced = forced_macro(any_shape, BM, BN);
-    for (const Macro t : {Macro{256, 256}, Macro{256, 128}, Macro{128, 128}}) {
-        if (forced.m ? t.m != forced.m || t.n != forced.n : !any_shape && (t.m % BM || t.n % BN)) continue;
-        if (t.m != t.n && !may_be_tall) continue;
-        const int total = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n), whole = (total - 1) / cus, rest = total - whole * cus;
-        const double whole_us = whole * (panels * panel_us(t, 1.0) + round_us(t));
-        const double us = whole_us + panels * panel_us(t, whole ? 1.0 : (double)rest / cus) + round_us(t);
+    const Macro forced = forced_macro(any_tile, BM, BN);
+    for (const Macro t : {Macro{256, 256}, Macro{256, 128}, Macro{128, 128}, Macro{64, 64}}) {
+        if (forced.m ? t.m != forced.m || t.n != forced.n : !any_tile && (t.m % BM || t.n % BN)) continue;
+        if ((t.m != t.n || t.m == 64) && !all_tiles) continue;
+        const int total = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
+        if (t.m == 64) {   // one round of at most two to a CU, or none
+            const double us = panels * panel_us(t, (double)total / cus, straddle) + round_us(t);
+            if (total <= 2 * cus && us < best_us) {
+                best_us = us;
+                best = {t, total, 0, 1, panels, 0};
+            }
+            continue;
+        }
+        const int whole = (total - 1) / cus, rest = total - whole * cus;
+        const double whole_us = whole * (panels * panel_us(t, 1.0, straddle) + round_us(t));
+        const double us = whole_us + panels * panel_us(t, whole ? 1.0 : (double)rest / cus, straddle) + round_us(t);
         if (us < best_us) {
             best_us = us;
             best = {t, total, 0, 1, panels, 0};
         }
         if (!may_split || t.m != t.n || rest * 2 > cus) continue;
         // A part written and read again, and what the second launch adds (16x4096x7168 in 2, 4, 8, 16
-        // parts: 31.0, 19.7, 15.0, 15.7 us, 54.7 unsplit; 8191x4097x7168: 376, 360, 362 us, 435 unsplit).
-        const double part_us = t.m == 256 ? 0.14 : 0.022, launch_us = 2.0;
+        // parts: 31.0, 19.7, 15.0, 15.7 us, 54.7 unsplit; 2688x1920x4944 in 2: 63, 88 unsplit, 72 in 256x128 tiles;
+        // 8191x4097x7168 in 2, 4, 8: 376, 360, 362, 435 unsplit).
+        const double part_us = t.m == 256 ? 0.09 : 0.022, launch_us = 2.0;
         for (int n = 2; n <= cus / rest && n <= 16; ++n) {
             const int per = (panels + n - 1) / n, parts = (panels + per - 1) / per;
             if (per < 3) break;
-            const double split_us = whole_us + per * panel_us(t, 0.5) + round_us(t) + rest * parts * part_us + launch_us;
+            const double split_us = whole_us + per * panel_us(t, t.m == 256 ? (double)rest * parts / cus : 0.5, straddle) + round_us(t) + rest * parts * part_us + launch_us;
             if (split_us < best_us && split_us < us * 0.97) {
                 best_us = split_us;
                 best = {t, total - rest, rest, parts, per, FO_WORKSPACE_ZEROED + (size_t)rest * parts * t.m * t.n * sizeof(float)};
@@ -119,10 +134,12 @@ static int plan_for(const fo_gemm_call& c, bool workspace, Plan* plan) {
     if (algo_tile(c.algo, &BM, &BN, &BK) != FO_OK) return fail(FO_ERR_ARG, "fo_gemm: Algo %d out of range", c.algo);
     const DeviceFacts* facts;
     if (int e = device_facts(&facts)) return e;
-    // tickets are taken in the GEMM's own epilogue; the signal and store forms behind knobs are built for square tiles
-    const bool plain = c.mode == kPlain, knobs_default = knob(knobs().store_mode) && knob(knobs().release_mode);
-    *plan = make_plan(BM, BN, c.M, c.N, c.K, plain, workspace && (plain || !c.monitor), knobs_default, facts->cus);
-    if (!plan->macro.m) *plan = make_plan(BM, BN, c.M, c.N, c.K, plain, false, true, facts->cus);
+    // Tiles that are signalled take a macro tile of whole layout tiles, tickets are taken in the GEMM's own
+    // epilogue, and the signal and store forms behind knobs are built for the two square tiles.
+    const bool plain = c.mode == kPlain, any_tile = plain || (c.deliver && c.deliver_from == 0);
+    const bool knobs_default = knob(knobs().store_mode) && knob(knobs().release_mode);
+    *plan = make_plan(BM, BN, c.M, c.N, c.K, any_tile, workspace && (plain || !c.monitor), knobs_default, facts->cus);
+    if (!plan->macro.m) *plan = make_plan(BM, BN, c.M, c.N, c.K, any_tile, false, true, facts->cus);
     return FO_OK;
 }
 
@@ -226,6 +243,7 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
     const int macro = plan.macro.m;
     int rc;
     if (plan.macro.n != macro) rc = launch_gemm_tall(mode, dtype, edge, p, timer, stream);
+    else if (macro == 64) rc = launch_gemm_small(mode, dtype, edge, p, timer, stream);
     else if (dtype == FO_F16)
         rc = macro == 256 ? launch_mt<_Float16, 256>(mode, edge, p, timer, stream) : launch_mt<_Float16, 128>(mode, edge, p, timer, stream);
     else

@@ -2,7 +2,7 @@
 // K contiguous, 16-bit inputs (fp16 / bf16), fp32 accumulation on MFMA.
 //
 // One workgroup of 4 wavefronts computes one MTM x MTN macro tile (256 x 256, or
-// 256 x 128 or 128 x 128 where those are too few to fill the GPU); each wavefront
+// 256 x 128, 128 x 128 or 64 x 64 where those are too few to fill the GPU); each wavefront
 // owns an (MTM/2) x (MTN/2) quadrant as 16 x 16 blocks of v_mfma_f32_16x16x32,
 // accumulators in AGPRs.  The 16x16x32
 // form reads and writes a quarter of the accumulator registers per flop of the
@@ -147,8 +147,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     if constexpr (MODE != kPlain) {
         const int tiles_n = MTN >> p.log_bn;          // layout tiles per macro tile, N
         const int tiles_m = MTM >> p.log_bm;
-        const int qm = wm * WM, qn = wn * WN;         // quadrant origin in the macro tile
-        if (live) quad_slot = p.RA[(mt.m * tiles_m + (qm >> p.log_bm)) * p.TN + mt.n * tiles_n + (qn >> p.log_bn)];
+        // (a layout tile may also be larger than the macro tile, if nothing is signalled: no lane then has one to signal)
+        if (live) quad_slot = p.RA[((mt.m * MTM + wm * WM) >> p.log_bm) * p.TN + ((mt.n * MTN + wn * WN) >> p.log_bn)];
         const int sig_m = tiles_n == 2 ? tid >> 1 : tid, sig_n = tiles_n == 2 ? tid & 1 : 0;   // tiles_n is 1 or 2
         sig_lane = tid < tiles_m * tiles_n && (sig_m << p.log_bm) < valid_m && (sig_n << p.log_bn) < valid_n;
         if (sig_lane) sig_slot = p.RA[(mt.m * tiles_m + sig_m) * p.TN + mt.n * tiles_n + sig_n];
@@ -160,8 +160,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     auto resolve_destination = [&]() {
         if constexpr (MODE != kPlain) {
             const int s = __builtin_amdgcn_readfirstlane(quad_slot);
-            row0 = (s / p.rLDN) * p.BM + ((wm * WM) & (p.BM - 1));
-            col0 = (s % p.rLDN) * p.BN + ((wn * WN) & (p.BN - 1));
+            row0 = (s / p.rLDN) * p.BM + ((mt.m * MTM + wm * WM) & (p.BM - 1));
+            col0 = (s % p.rLDN) * p.BN + ((mt.n * MTN + wn * WN) & (p.BN - 1));
             ld = p.rLDN * p.BN;
             // a delivered tile is not signalled: nobody waits for it
             if (sig_lane && !(p.D2 && sig_slot >= p.deliver_from))
@@ -522,6 +522,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
 
     // ---- signal ---------------------------------------------------------------------
     if constexpr (MODE != kPlain) {
+        if (p.D2 && p.deliver_from == 0) return;   // nothing is signalled
         // Every wave's tile stores are acknowledged before the barrier: with
         // write-through stores they are then visible device-wide (REL = 1);
         // otherwise the release on the atomic writes this L2's dirty lines back

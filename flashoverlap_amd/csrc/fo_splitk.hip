@@ -44,8 +44,8 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const GemmParams p) {
     bool deliver = p.D2 != nullptr, signal = false;
     if constexpr (MODE != kPlain) {
         slot = p.RA[((mt.m * MT + wm * WT) >> p.log_bm) * p.TN + ((mt.n * MT + wn * WT) >> p.log_bn)];
-        row0 = (slot / p.rLDN) * p.BM + ((wm * WT) & (p.BM - 1));
-        col0 = (slot % p.rLDN) * p.BN + ((wn * WT) & (p.BN - 1));
+        row0 = (slot / p.rLDN) * p.BM + ((mt.m * MT + wm * WT) & (p.BM - 1));
+        col0 = (slot % p.rLDN) * p.BN + ((mt.n * MT + wn * WT) & (p.BN - 1));
         ld = p.rLDN * p.BN;
         deliver = deliver && slot >= p.deliver_from;
         signal = !deliver;

@@ -37,7 +37,7 @@ def _operands(dev, dt, M, N, K):
 @pytest.mark.parametrize("M,N,K", [
     (128, 128, 8192),      # one tile
     (33, 129, 4104),       # four edge tiles, rows of D unaligned, 8 k in the last panel
-    (100, 1160, 7168), (128, 4096, 2048), (256, 2048, 4160),
+    (100, 1160, 7168), (128, 4096, 4096), (256, 2048, 4160),
     (4352, 4096, 1544),    # 272 macro tiles of 256x256: sixteen behind a whole round
     (4225, 4104, 1984),    # 17 x 17: the tail is ragged in both directions
 ])
@@ -156,3 +156,30 @@ def test_tall_tile_signals_and_places(dev, M, N, algo, ws):
     out = torch.empty(TM * TN * BM, BN, dtype=dt, device=dev)
     out[RE.long() if ws > 1 else slice(None)] = rows.view(-1, BN)
     assert torch.equal(D, out)
+
+
+@pytest.mark.parametrize("M,N,K,algo", [(128, 128, 64, 1), (256, 384, 72, 1), (256, 256, 200, 2), (512, 128, 136, 4)])
+@pytest.mark.parametrize("ws", [1, 8])
+def test_small_tile_delivers_into_larger_layout_tiles(dev, M, N, K, algo, ws):
+    """Nothing signalled: the 64x64 macro tile, four or eight of which share a layout tile."""
+    L, dt = capi.lib(), torch.bfloat16
+    BM, BN, _ = capi.algo_tile(algo)
+    TM, TN = M // BM, N // BN
+    T = TM * TN
+    A, B, want = _operands(dev, dt, M, N, K)
+    RA = torch.randperm(T, generator=torch.Generator().manual_seed(3)).int().to(dev)
+    RE = tiling.generate_row_remap_array(M, N, BM, BN, [T], ws, dev)
+    cs, zero = torch.tensor([T], dtype=torch.int32, device=dev), torch.zeros(T, dtype=torch.int32, device=dev)
+    D, D2 = (torch.full((T * BM, BN), 7.0, dtype=dt, device=dev) for _ in range(2))
+    mm = torch.zeros(1, dtype=torch.int32, device=dev)
+    c = capi.GemmCall(mode=2 if ws > 1 else 1, dtype=capi.dtype_code(dt), algo=algo, M=M, N=N, K=K, rLDN=1,
+                      cseg_dev=cs.data_ptr(), G=1, group_table=zero.data_ptr(), A=A.data_ptr(), B=B.data_ptr(),
+                      D=D.data_ptr(), MM=mm.data_ptr(), RA=RA.data_ptr(), RE=RE.data_ptr(), nslices=ws, slice_count=ws,
+                      slice_stride=M * N // ws, group_start=zero.data_ptr(), deliver=D2.data_ptr())
+    capi.check(L.fo_gemm_launch(C.byref(c), None))
+    torch.cuda.synchronize()
+    rows = torch.empty(T, BM, BN, dtype=dt, device=dev)
+    rows[RA.long()] = want.view(TM, BM, TN, BN).permute(0, 2, 1, 3).reshape(T, BM, BN)
+    out = torch.empty(T * BM, BN, dtype=dt, device=dev)
+    out[RE.long() if ws > 1 else slice(None)] = rows.view(-1, BN)
+    assert torch.equal(D, out) and torch.equal(D2, out) and mm.item() == 0
