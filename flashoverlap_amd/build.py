@@ -23,7 +23,7 @@ LIB = os.path.join(HERE, "lib")
 OBJ = os.path.join(HERE, "build")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-HIP_SOURCES = ["fo_capi.hip", "fo_gemm.hip", "fo_gemm_small.hip", "fo_gemm_tall.hip", "fo_skinny.hip", "fo_splitk.hip",
+HIP_SOURCES = ["fo_capi.hip", "fo_gemm.hip", "fo_gemm_deep.hip", "fo_gemm_tall.hip", "fo_skinny.hip", "fo_splitk.hip",
                "fo_sync.hip", "fo_rmsnorm.hip", "fo_static.hip"]
 BENCH_SOURCES = ["fo_probe.hip"]
 BINDING_SOURCES = ["overlap_impl.cpp", "baseline_impl.cpp", "rmsnorm_op.cpp", "pybind.cpp"]

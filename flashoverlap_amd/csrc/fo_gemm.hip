@@ -129,6 +129,9 @@ static Plan make_plan(int BM, int BN, int M, int N, int K, bool any_tile, bool m
     return best;
 }
 
+// The store and signal forms of the default: the only ones that all macro tiles are built for.
+static bool default_forms() { return knob(knobs().store_mode) && knob(knobs().release_mode); }
+
 static int plan_for(const fo_gemm_call& c, bool workspace, Plan* plan) {
     int BM, BN, BK;
     if (algo_tile(c.algo, &BM, &BN, &BK) != FO_OK) return fail(FO_ERR_ARG, "fo_gemm: Algo %d out of range", c.algo);
@@ -137,8 +140,7 @@ static int plan_for(const fo_gemm_call& c, bool workspace, Plan* plan) {
     // Tiles that are signalled take a macro tile of whole layout tiles, tickets are taken in the GEMM's own
     // epilogue, and the signal and store forms behind knobs are built for the two square tiles.
     const bool plain = c.mode == kPlain, any_tile = plain || (c.deliver && c.deliver_from == 0);
-    const bool knobs_default = knob(knobs().store_mode) && knob(knobs().release_mode);
-    *plan = make_plan(BM, BN, c.M, c.N, c.K, any_tile, workspace && (plain || !c.monitor), knobs_default, facts->cus);
+    *plan = make_plan(BM, BN, c.M, c.N, c.K, any_tile, workspace && (plain || !c.monitor), default_forms(), facts->cus);
     if (!plan->macro.m) *plan = make_plan(BM, BN, c.M, c.N, c.K, any_tile, false, true, facts->cus);
     return FO_OK;
 }
@@ -241,9 +243,14 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
         p.partial = (float*)((char*)c.workspace + FO_WORKSPACE_ZEROED);
     }
     const int macro = plan.macro.m;
+    const DeviceFacts* facts;
+    if (int e = device_facts(&facts)) return e;
+    // A workgroup that has its CU to itself takes the ring of four panels ahead: nothing else hides the latency of
+    // its copies (256x4096x7168, 256 parts: 25.3 us, 22.5; with two on a CU the LDS allows two panels ahead).
+    const bool deep = macro == 64 || (macro == 128 && plan.macro.n == 128 && default_forms() && p.split_from + p.split_tiles * p.splits <= facts->cus);
     int rc;
     if (plan.macro.n != macro) rc = launch_gemm_tall(mode, dtype, edge, p, timer, stream);
-    else if (macro == 64) rc = launch_gemm_small(mode, dtype, edge, p, timer, stream);
+    else if (deep) rc = launch_gemm_deep(macro, mode, dtype, edge, p, timer, stream);
     else if (dtype == FO_F16)
         rc = macro == 256 ? launch_mt<_Float16, 256>(mode, edge, p, timer, stream) : launch_mt<_Float16, 128>(mode, edge, p, timer, stream);
     else

@@ -83,7 +83,8 @@ namespace fo {
 // STORE: 0 cached, 1 write-through tile stores; REL: 0 release atomic, 1 relaxed atomic.
 // EDGE (plain GEMM only): M and N are arbitrary; the rows and columns of a macro tile that lie
 // outside the matrix are computed on zeros and not stored.
-template <typename T, int MTM, int MTN, int MODE, int STORE, int REL, bool EDGE>
+// DEPTH: panels ahead of the one being multiplied that are in LDS or on their way there.
+template <typename T, int MTM, int MTN, int MODE, int STORE, int REL, bool EDGE, int DEPTH = 2>
 __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     static_assert(!EDGE || MODE == kPlain, "only the plain GEMM takes shapes that are not multiples of the layout tile");
     constexpr int WM = MTM / 2, WN = MTN / 2;    // wave quadrant
@@ -97,7 +98,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
 
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
-    static_assert(2 * 4 * 32 * (WN * 2 + 16) <= 5 * PANEL, "epilogue strips must fit in the panel slots");
+    constexpr int SLOTS = 2 * DEPTH + 1;
+    static_assert(2 * 4 * 32 * (WN * 2 + 16) <= SLOTS * PANEL, "epilogue strips must fit in the panel slots");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -222,8 +224,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     const unsigned slab_bytes = 8u * (unsigned)K * 2u;    // bytes between consecutive slabs
     const int lds_cpA = wave * (LOADS_A * 1024), lds_cpB = wave * (LOADS_B * 1024);   // this wave's first slab in a panel
 
-    // The LDS is a ring of five panel slots.  Panel units alternate A(0) B(0)
-    // A(1) B(1) ...; unit u lives in slot u % 5.  `slot` is the byte offset of
+    // The LDS is a ring of SLOTS panel slots.  Panel units alternate A(0) B(0)
+    // A(1) B(1) ...; unit u lives in slot u % SLOTS.  `slot` is the byte offset of
     // the receiving slot; the copies of a unit are issued in two halves.
     auto issue_unit = [&](int kt, int slot, auto isb_c, auto half_c) {
         constexpr bool ISB = decltype(isb_c)::value;
@@ -287,8 +289,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     auto read_a = [&](int slot_a, int h, int i) { fa[h][i] = *(const frag*)(smem + slot_a + ko[h] + a_lane + i * BLK); };
     auto read_b = [&](int slot_b, int h, int j) { fb[h][j] = *(const frag*)(smem + slot_b + ko[h] + b_lane + j * BLK); };
 
-    // One k-step on panel kt.  A(kt) sits in slot sa, the units of panel kt+1 in na and nb (landed
-    // or landing), sp is the free slot; the B fragments of panel kt and the A fragments of its
+    // One k-step on panel kt (at DEPTH 2; of a deeper ring the copies are those of panel kt+DEPTH).
+    // A(kt) sits in slot sa, the units of panel kt+1 in na and nb (landed or landing), sp is the free slot; the B fragments of panel kt and the A fragments of its
     // first NH rows of blocks are in registers, or on their way there, on entry.
     //
     // The two MFMAs that an accumulator gets from a panel (k halves 0 and 1) are issued back to
@@ -305,7 +307,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     //     left; copies B(kt+2) to slot sa.
     // LDS reads return in order.  Half step 0 therefore starts column j as soon as at most
     // 2(NBN-1-j) reads younger than B fragments j are outstanding, plus its own reads issued so far.
-    // NEXT: panel kt+1 exists.  C2: panel kt+2 exists.
+    // NEXT: panel kt+1 exists.  C2: panel kt+DEPTH exists.
     constexpr int COL = 2 * NH;          // MFMAs per column of a half step
     constexpr int NS = COL * NBN;        // MFMAs per half step
     auto half_step = [&](auto hs_c, int kt, int slot_reads_a, int slot_next_b, int slot_copy, auto next_c, auto c2_c) {
@@ -334,7 +336,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
                 }
             }
             if constexpr (C2 && sl % CP_EVERY == CP_EVERY / 2)
-                issue_one(kt + 2, slot_copy, std::integral_constant<bool, hs == 1>{}, template_int<sl / CP_EVERY>{});
+                issue_one(kt + DEPTH, slot_copy, std::integral_constant<bool, hs == 1>{}, template_int<sl / CP_EVERY>{});
             __builtin_amdgcn_sched_barrier(0);   // nothing moves across an MFMA
             // operands swapped (B rows as the MFMA "A" matrix): a lane ends up with 4 consecutive n for one m
             Mma<T>::run(fb[h][j], fa[h][i0 + r], acc[i0 + r][j]);
@@ -346,26 +348,30 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    auto kstep = [&](int kt, int sa, int sb, int na, int nb, int sp, auto next_c, auto c2_c) {
-        constexpr bool NEXT = decltype(next_c)::value;
-        constexpr bool C2 = decltype(c2_c)::value;
+    // after: how many panels follow panel kt, DEPTH if at least that many.
+    auto kstep = [&](int kt, int sa, int na, int nb, int sp, auto after_c) {
+        constexpr int AFTER = decltype(after_c)::value;
+        constexpr bool NEXT = AFTER > 0, C2 = AFTER == DEPTH;
+        const std::bool_constant<NEXT> next_c;
+        const std::bool_constant<C2> c2_c;
         half_step(template_int<0>{}, kt, sa, 0, sp, next_c, c2_c);
         __builtin_amdgcn_sched_barrier(0);
         wait_lds_reads();                 // the A fragments of the second half step; panel kt has been read
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (NEXT) {
-            // Panel kt+1 has landed for every wave (the copies of A(kt+2), the newest
-            // LOADS_A of this wave, may still be in flight: copies complete in issue
-            // order), and every wave has read panel kt for the last time.
-            if constexpr (C2) wait_vmcnt<LOADS_A>(); else wait_vmcnt<0>();
+            // Panel kt+1 has landed for every wave (the copies of the panels behind it and of
+            // A(kt+DEPTH), the newest of this wave, may still be in flight: copies complete in
+            // issue order), and every wave has read panel kt for the last time.
+            wait_vmcnt<C2 ? (DEPTH - 2) * (LOADS_A + LOADS_B) + LOADS_A : (AFTER - 1) * (LOADS_A + LOADS_B)>();
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
         }
         half_step(template_int<1>{}, kt, na, nb, sa, next_c, c2_c);
-        (void)sb;
     };
 
-    // Prologue: panels 0 and 1 go out; wait for panel 0.
+    // Prologue: panels 0 .. DEPTH-1 go out; wait for panel 0.  (Where K has fewer, the last one is
+    // copied again, to slots that nobody reads: without branches the waits that the compiler derives
+    // for the slot lookups count all of these copies.)
     template_int<0> first_half;
     template_int<1> second_half;
     auto last_panel_next = [&](bool is_last) {   // called before the copies of a panel are issued
@@ -374,18 +380,15 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
             vo1 = tail_off1;
         }
     };
-    last_panel_next(NP == 1);
-    issue_unit(0, 0 * PANEL, unit_a, first_half);
-    issue_unit(0, 0 * PANEL, unit_a, second_half);
-    issue_unit(0, 1 * PANEL, unit_b, first_half);
-    issue_unit(0, 1 * PANEL, unit_b, second_half);
-    if (NP > 1) {
-        last_panel_next(NP == 2);
-        issue_unit(1, 2 * PANEL, unit_a, first_half);
-        issue_unit(1, 2 * PANEL, unit_a, second_half);
-        issue_unit(1, 3 * PANEL, unit_b, first_half);
-        issue_unit(1, 3 * PANEL, unit_b, second_half);
-    }
+    static_for<DEPTH>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        const int panel = min(i, NP - 1);
+        last_panel_next(panel == NP - 1);
+        issue_unit(panel, 2 * i * PANEL, unit_a, first_half);
+        issue_unit(panel, 2 * i * PANEL, unit_a, second_half);
+        issue_unit(panel, (2 * i + 1) * PANEL, unit_b, first_half);
+        issue_unit(panel, (2 * i + 1) * PANEL, unit_b, second_half);
+    });
     // The accumulators are cleared here, under the latency of those copies, by MFMAs on zero
     // operands (0 x 0 + 0).  Written as assignments of zero, the compiler places the 256 register
     // writes directly in front of the main loop, behind the wait for the first panel.
@@ -399,7 +402,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
 #pragma unroll
             for (int j = 0; j < NBN; ++j) Mma<T>::clear(zeros, acc[i][j]);
     }
-    if (NP > 1) wait_vmcnt<LOADS_A + LOADS_B>(); else wait_vmcnt<0>();
+    if (NP > 1) wait_vmcnt<(DEPTH - 1) * (LOADS_A + LOADS_B)>(); else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
     // fragments of the first half step, in the order the main loop leaves them for the next k-step
 #pragma unroll
@@ -417,22 +420,29 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     // copied; the issue arbiter should always prefer the wave that feeds the MFMAs.
     __builtin_amdgcn_s_setprio(3);
     int kt = 0;
-    int sa = 0, sb = PANEL, na = 2 * PANEL, nb = 3 * PANEL, sp = 4 * PANEL;
-    auto rotate = [&]() {   // (sa, sb, na, nb, sp) <- (na, nb, sp, sa, sb)
-        const int a0 = sa, b0 = sb;
-        sa = na; sb = nb; na = sp; nb = a0; sp = b0;
+    int ring[SLOTS];   // the slots, from that of A(kt) on
+#pragma unroll
+    for (int u = 0; u < SLOTS; ++u) ring[u] = u * PANEL;
+    auto rotate = [&]() {
+        const int a0 = ring[0], b0 = ring[1];
+#pragma unroll
+        for (int u = 0; u + 2 < SLOTS; ++u) ring[u] = ring[u + 2];
+        ring[SLOTS - 2] = a0;
+        ring[SLOTS - 1] = b0;
     };
-    for (; kt < NP - 2; ++kt) {
-        last_panel_next(kt + 3 == NP);   // this k-step copies panel kt + 2
-        kstep(kt, sa, sb, na, nb, sp, std::true_type{}, std::true_type{});
+    for (; kt < NP - DEPTH; ++kt) {
+        last_panel_next(kt + DEPTH + 1 == NP);   // this k-step copies panel kt + DEPTH
+        kstep(kt, ring[0], ring[2], ring[3], ring[SLOTS - 1], template_int<DEPTH>{});
         rotate();
     }
-    if (NP >= 2) {
-        kstep(kt, sa, sb, na, nb, sp, std::true_type{}, std::false_type{});
-        rotate();
-        ++kt;
-    }
-    kstep(kt, sa, sb, na, nb, sp, std::false_type{}, std::false_type{});
+    static_for<DEPTH>([&](auto t_c) {
+        constexpr int after = DEPTH - 1 - decltype(t_c)::value;
+        if (after == 0 || NP > after) {
+            kstep(kt, ring[0], ring[2], ring[3], ring[SLOTS - 1], template_int<after>{});
+            rotate();
+            ++kt;
+        }
+    });
 
     // ---- epilogue: registers -> LDS strip -> global -------------------------------
     // acc[i][j][r] is element m = 16i + l%16, n = 16j + 4(l/16) + r (fr_g = l/16).
@@ -561,7 +571,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
 }
 
 
-// SMEM: five panel slots (160 KiB at MTM = 256).
+// SMEM: the panel slots (160 KiB at MTM = 256).
 template <auto KERN, int SMEM>
 static int launch_gemm_kernel(const GemmParams& p, const LaunchTimer& timer, hipStream_t stream) {
     // The attribute belongs to the function on one device: set it once per device.

@@ -36,9 +36,9 @@ int gemm_rounds(int algo, int M, int N, int* per_round, int* last_first);
 int raster_hint(int algo, int M, int N, int* hint);
 int tune(const char* key, int value);
 
-// fo_gemm_tall.hip, fo_gemm_small.hip: the 256x128 and the 64x64 macro tile
+// fo_gemm_tall.hip, fo_gemm_deep.hip: the 256x128 macro tile; 64x64, and 128x128 with one workgroup to a CU
 struct GemmParams;
-int launch_gemm_small(int mode, int dtype, bool edge, const GemmParams& p, const LaunchTimer& timer, hipStream_t stream);
+int launch_gemm_deep(int macro, int mode, int dtype, bool edge, const GemmParams& p, const LaunchTimer& timer, hipStream_t stream);
 int launch_gemm_tall(int mode, int dtype, bool edge, const GemmParams& p, const LaunchTimer& timer, hipStream_t stream);
 
 // fo_skinny.hip: the plain GEMM for M <= kSkinnyRows
