@@ -70,22 +70,28 @@ struct Plan {
 
 // Microseconds of a k-step of 64 of a macro tile, and of a round's start and end (launch, first panels,
 // stores).  Measured on shapes from 1024x1024x1024 to 8192x4096x7168, bf16 and fp16: with more than
-// three quarters of the CUs at work the chip comes to its power limit, and the k-steps get longer.
+// two thirds of the CUs at work all the time the chip comes to its power limit, and the k-steps get longer.
 // 2048x4096x7168 bf16: 114 us in 128x128 tiles, 101 in 256x128, 130 in 256x256; 4096x4096x4096: 116, 101, 90;
 // 1024x1024x1024: 9.2 in 64x64, 11.0 in 128x128.
-// straddle: rows that do not start on cache lines (K no multiple of 64) ask the L2 for every line twice,
-// which the smaller tiles feel (2304x1664x5424: 77 us in 256x128 tiles, 55 in 128x128).
+// straddle: rows that do not start on cache lines (K no multiple of 64) ask the L2 for every line twice
+// (2304x1664x5424: 77 us in 256x128 tiles, 55 in 128x128; 5504x1536 in 256x256: 123 with K 6912, 148 with 6944).
 static double panel_us(Macro t, double busy, bool straddle) {   // busy: share of the CUs
-    const double hot = busy <= 0.75 ? 0.0 : busy >= 1.0 ? 1.0 : (busy - 0.75) * 4;
-    if (t.n == 256) return 1.08 + 0.28 * hot;
-    if (t.n == 64) return (busy <= 1.0 ? 0.37 : 0.41) + 0.1 * straddle;   // (the copies' latency; of two on a CU each hides the other's)
-    return t.m == 256 ? 0.61 + 0.25 * (straddle ? 1.0 : hot) : 0.46 + 0.06 * hot + 0.13 * straddle;
+    const double hot = busy <= 0.65 ? 0.0 : busy >= 1.0 ? 1.0 : (busy - 0.65) / 0.35;
+    if (t.n == 256) return 1.08 + 0.28 * hot + 0.2 * straddle * (1.0 - hot);
+    if (t.n == 64) return busy <= 1.0 ? 0.34 + 0.1 * straddle : 0.36 + 0.16 * straddle;   // (of two on a CU each hides the other's latency)
+    return t.m == 256 ? 0.70 + 0.16 * (straddle ? 1.0 : hot) : 0.46 + 0.02 * hot + 0.13 * straddle;
 }
 static double round_us(Macro t) { return t.n == 256 ? 7.0 : t.m == 256 ? 5.0 : t.n == 128 ? 3.5 : 3.0; }
 
 // The plan whose estimated time is the smallest.  A round of workgroups takes as long if it is not
 // full; of a round that is at most half full the tiles can be split over K instead, if the parts
 // (which write MT * MT floats each, and are read again by a second launch) stay worth it.
+// Of the 128x128 tiles a CU holds two, and while one starts or stores the other multiplies: they take
+// k-steps only, however many come to a CU (9856x2048x1216, 4.8 to a CU: 46 us, 56 in 256x256 tiles;
+// 7168x1152x3520: 55, 64; 4608x4096x4096: 147, 119).  That also pairs them up as they come, so the parts of
+// an odd round out can share a CU with a whole tile while another two whole ones share theirs
+// (1407x3088x7360, 275 tiles of which 19 in 13 parts: 94 us, 68 in 256x256 tiles in 3): behind an odd number of
+// whole rounds nothing is split.
 static Plan make_plan(int BM, int BN, int M, int N, int K, bool any_tile, bool may_split, bool all_tiles, int cus) {
     const int panels = (K + kBK - 1) / kBK;
     const bool straddle = K % kBK != 0;
@@ -105,21 +111,24 @@ static Plan make_plan(int BM, int BN, int M, int N, int K, bool any_tile, bool m
             continue;
         }
         const int whole = (total - 1) / cus, rest = total - whole * cus;
-        const double whole_us = whole * (panels * panel_us(t, 1.0, straddle) + round_us(t));
-        const double us = whole_us + panels * panel_us(t, whole ? 1.0 : (double)rest / cus, straddle) + round_us(t);
+        const bool paired = t.m == 128;
+        const double each = panels * panel_us(t, (double)total / (whole * cus + cus), straddle);
+        const double us = (whole + 1) * (each + (paired ? 0.0 : round_us(t))) + (paired ? round_us(t) : 0.0);
         if (us < best_us) {
             best_us = us;
             best = {t, total, 0, 1, panels, 0};
         }
-        if (!may_split || t.m != t.n || rest * 2 > cus) continue;
+        if (!may_split || t.m != t.n || rest * 2 > cus || (paired && whole % 2)) continue;
         // A part written and read again, and what the second launch adds (16x4096x7168 in 2, 4, 8, 16
         // parts: 31.0, 19.7, 15.0, 15.7 us, 54.7 unsplit; 2688x1920x4944 in 2: 63, 88 unsplit, 72 in 256x128 tiles;
-        // 8191x4097x7168 in 2, 4, 8: 376, 360, 362, 435 unsplit).
-        const double part_us = t.m == 256 ? 0.09 : 0.022, launch_us = 2.0;
+        // 8191x4097x7168 in 2, 4, 8: 376, 360, 362, 435 unsplit; 71x856x600 with its norm in 4: 13.4, 10.6 in 64x64 tiles).
+        const double part_us = t.m == 256 ? 0.09 : 0.022, launch_us = 3.0;
         for (int n = 2; n <= cus / rest && n <= 16; ++n) {
             const int per = (panels + n - 1) / n, parts = (panels + per - 1) / per;
             if (per < 3) break;
-            const double split_us = whole_us + per * panel_us(t, t.m == 256 ? (double)rest * parts / cus : 0.5, straddle) + round_us(t) + rest * parts * part_us + launch_us;
+            const double share = (double)rest * parts / cus;   // of the CUs; the parts' way through memory is some 20 k-steps' time
+            const double whole_us = whole * (panels * panel_us(t, (whole * panels + per * share) / (whole * panels + per + 20), straddle) + (paired ? 0.0 : round_us(t)));
+            const double split_us = whole_us + per * panel_us(t, t.m == 256 ? share : 0.5, straddle) + round_us(t) + rest * parts * part_us + launch_us;
             if (split_us < best_us && split_us < us * 0.97) {
                 best_us = split_us;
                 best = {t, total - rest, rest, parts, per, FO_WORKSPACE_ZEROED + (size_t)rest * parts * t.m * t.n * sizeof(float)};
