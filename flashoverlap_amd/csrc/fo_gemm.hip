@@ -294,8 +294,8 @@ int raster_hint(int algo, int M, int N, int* hint) {
     const int tiles_m = t.m / BM, tiles_n = t.n / BN;
     int k = 0;
     for (int pid = 0; pid < GM * GN; ++pid) {
-        const TileCoord c = t.m > t.n ? raster_map<kGroupM / 2, kUnitN * 2>(pid, GM, GN, raster_magic(GN))
-                                      : raster_map(pid, GM, GN, raster_magic(GN));
+        const TileCoord c = t.m > t.n ? raster_order<kGroupM / 2, kUnitN * 2>(pid, GM, GN, raster_magic(GN))
+                                      : raster_order(pid, GM, GN, raster_magic(GN));
         for (int i = 0; i < tiles_m; ++i)
             for (int j = 0; j < tiles_n; ++j) {
                 const int tm = c.m * tiles_m + i, tn = c.n * tiles_n + j;

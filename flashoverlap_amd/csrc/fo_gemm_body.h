@@ -112,15 +112,18 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     // (blockIdx.x % 8; split_from is a multiple of 8) get consecutive numbers, split by split, so that
     // they work on one range of k and share its panels in their L2.
     int tile = blockIdx.x, kt0 = 0, NP = NPK, part = -1;
-    if (tile >= p.split_from) {
+    TileCoord mt;
+    if (MTM == MTN && tile >= p.split_from) {
         const int q = tile - p.split_from, all = p.split_tiles * p.splits, even = all & ~(kXcds - 1);
         const int at = q < even ? (q & (kXcds - 1)) * (even / kXcds) + q / kXcds : q;
         part = at / p.split_tiles;
-        tile = p.split_from + (at - part * p.split_tiles);
+        tile = at - part * p.split_tiles;
+        mt = split_tile_at(p, tile);
         kt0 = part * p.split_panels;
         NP = min(p.split_panels, NPK - kt0);
+    } else {
+        mt = macro_tile_at<MTM, MTN>(p, tile);
     }
-    const TileCoord mt = macro_tile_at<MTM, MTN>(p, tile);
     // M and N are multiples of the layout tile, not necessarily of the macro
     // tile: the last row or column of macro tiles may be half inside.  Such a
     // workgroup runs the full main loop (the waves of the outer half re-read the
@@ -450,7 +453,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     settle_mfma();
     __builtin_amdgcn_sched_barrier(0);   // no accumulator read is scheduled ahead of the delay
     if (part >= 0) {   // a part of a split tile: the sums as they are
-        f32x4* out = (f32x4*)p.partial + partial_at(p, tile - p.split_from, part, wave, NBM * NBN) + lane;
+        f32x4* out = (f32x4*)p.partial + partial_at(p, tile, part, wave, NBM * NBN) + lane;
 #pragma unroll
         for (int b = 0; b < NBM * NBN; b += 4)
             if (live && 16 * (b / NBN) < valid_m - wm * WM) {   // not the blocks below the matrix

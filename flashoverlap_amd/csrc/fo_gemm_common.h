@@ -97,11 +97,18 @@ struct GemmParams {
     int* arrived;                               // reduction: strips of each layout tile that are stored
 };
 
-// The macro tile that workgroup `tile` of the grid (or the reduction's split tile) computes.
+// The macro tile that workgroup `tile` of the grid computes.
 template <int MTM, int MTN>
 __device__ __forceinline__ TileCoord macro_tile_at(const GemmParams& p, int tile) {
     if constexpr (MTM > MTN) return raster_map<kGroupM / 2, kUnitN * 2>(tile, p.GM, p.GN, p.gn_magic);
     else return raster_map(tile, p.GM, p.GN, p.gn_magic);
+}
+
+// Split tile `index`: counted from split_from on, by position if that is where a wave begins (the
+// workgroups of its parts are shared out between the XCDs before they get here).
+__device__ __forceinline__ TileCoord split_tile_at(const GemmParams& p, int index) {
+    const int at = p.split_from + index;
+    return p.split_from % kWave ? raster_map(at, p.GM, p.GN, p.gn_magic) : raster_tile(at, p.GM, p.GN, p.gn_magic, p.GM * p.GN);
 }
 
 // Where a part of a split tile lies in `partial`: [tile][split][wave][block i * NB + j][lane] vectors of
