@@ -44,6 +44,7 @@ SIGNATURES = {
     "fo_wait_groups": (_i, [_vp, _i, _i, _vp, _vp, _vp]),
     "fo_consume_groups": (_i, [_vp, _vp, _i, _i, _vp, _vp, _ll, _i, _i, _i, _ll, _i, _sz, _vp]),
     "fo_build_group_table": (_i, [_vp, _i, _i, _vp, _vp]),
+    "fo_build_group_tables": (_i, [_vp, _i, _i, _vp, _vp, _vp]),
     "fo_raster_hint": (_i, [_i, _i, _i, _ip]),
     "fo_tune": (_i, [C.c_char_p, _i]),
     "fo_wait": (_i, [_i, _vp, _vp, _vp]),

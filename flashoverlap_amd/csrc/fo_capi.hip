@@ -114,7 +114,11 @@ int fo_gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, co
 }
 
 int fo_build_group_table(const int* cseg_dev, int G, int T, int* group_table, void* stream) {
-    return launch_group_table(cseg_dev, G, T, group_table, (hipStream_t)stream);
+    return launch_group_table(cseg_dev, G, T, group_table, nullptr, (hipStream_t)stream);
+}
+
+int fo_build_group_tables(const int* cseg_dev, int G, int T, int* group_table, int* group_start, void* stream) {
+    return launch_group_table(cseg_dev, G, T, group_table, group_start, (hipStream_t)stream);
 }
 
 int fo_raster_hint(int algo, int M, int N, int* hint_host) { return raster_hint(algo, M, N, hint_host); }

@@ -54,7 +54,7 @@ int gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, const
                        const void* B, void* D, int* MM, const int* RA, int monitor, hipStream_t stream);
 
 // fo_sync.hip
-int launch_group_table(const int* cseg, int G, int T, int* table, hipStream_t stream);
+int launch_group_table(const int* cseg, int G, int T, int* table, int* start, hipStream_t stream);
 int launch_wait(int that, int* addr, int* expired, hipStream_t stream);
 int launch_wait_consume(const int* cseg, int G, int* MM, const void* src, void* dst, long long tile_elems,
                         int nslices, int slice_first, int slice_count, long long slice_stride, int* order_log,

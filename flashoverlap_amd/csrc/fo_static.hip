@@ -59,7 +59,7 @@ int gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, const
                     T, kStaticSlots);
     int* table = nullptr;
     if (int e = scratch_for_current_device(&table)) return e;
-    if (int e = launch_group_table(cseg, G, (int)T, table, stream)) return e;
+    if (int e = launch_group_table(cseg, G, (int)T, table, nullptr, stream)) return e;
     t_launch_timer = timer;   // for the GEMM's own dispatch
     fo_gemm_call c{};
     c.mode = FO_GEMM_SIGNAL; c.dtype = dtype; c.algo = algo; c.M = M; c.N = N; c.K = K; c.rLDN = rLDN;

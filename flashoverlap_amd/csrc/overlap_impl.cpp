@@ -145,10 +145,9 @@ const int* OverlapImpl::group_table_for(const at::Tensor& cseg_cpu, const at::Te
     const bool same_device = group_table_.defined() && group_table_.device() == cseg_gpu.device();
     if (!same_device || key != table_key_) {
         group_table_ = at::empty({T}, cseg_gpu.options());
-        FO_CALL(fo_build_group_table(cseg_gpu.data_ptr<int>(), G, T, group_table_.data_ptr<int>(), gemm_stream_));
-        at::Tensor start = at::empty({G}, cseg_cpu.options());
-        for (int g = 0, acc = 0; g < G; acc += host[g++]) start.data_ptr<int>()[g] = acc;
-        group_start_ = start.to(cseg_gpu.device());
+        group_start_ = at::empty({G}, cseg_gpu.options());
+        FO_CALL(fo_build_group_tables(cseg_gpu.data_ptr<int>(), G, T, group_table_.data_ptr<int>(),
+                                      group_start_.data_ptr<int>(), gemm_stream_));
         table_key_ = std::move(key);
     }
     return group_table_.data_ptr<int>();

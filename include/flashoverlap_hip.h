@@ -192,6 +192,10 @@ int fo_gemm_rounds(int algo, int M, int N, int* per_round, int* last_first);
  * every tile (src/overlap/gemm_with_signal.h:188-193); results are identical. */
 int fo_build_group_table(const int* cseg_dev, int G, int T, int* group_table, void* stream);
 
+/* The same, and group_start[g] = the first slot of group g for g in [0,G) (see
+ * fo_gemm_call), in one launch. */
+int fo_build_group_tables(const int* cseg_dev, int G, int T, int* group_table, int* group_start, void* stream);
+
 /* The order in which the GEMM kernels issue layout tiles for this shape:
  * hint[i] = original tile id of the i-th tile issued (T entries, host memory).
  * Feeding it to reorder_indices makes slot order equal issue order.  Replaces
