@@ -122,12 +122,14 @@ static Plan make_plan(int BM, int BN, int M, int N, int K, bool any_tile, bool m
         // A part written and read again, and what the second launch adds (16x4096x7168 in 2, 4, 8, 16
         // parts: 31.0, 19.7, 15.0, 15.7 us, 54.7 unsplit; 2688x1920x4944 in 2: 63, 88 unsplit, 72 in 256x128 tiles;
         // 8191x4097x7168 in 2, 4, 8: 376, 360, 362, 435 unsplit; 71x856x600 with its norm in 4: 13.4, 10.6 in 64x64 tiles).
-        const double part_us = t.m == 256 ? 0.09 : 0.022, launch_us = 3.0;
+        const double part_us = t.m == 256 ? 0.07 : 0.022, launch_us = 3.0;
+        // the k-steps of a chip that is never idle, against some 24 more in which the parts pass through memory
+        const double steps = (double)panels * total / cus;
+        const double whole_us = whole * (panels * panel_us(t, steps / (steps + 24), straddle) + (paired ? 0.0 : round_us(t)));
         for (int n = 2; n <= cus / rest && n <= 16; ++n) {
             const int per = (panels + n - 1) / n, parts = (panels + per - 1) / per;
             if (per < 3) break;
-            const double share = (double)rest * parts / cus;   // of the CUs; the parts' way through memory is some 20 k-steps' time
-            const double whole_us = whole * (panels * panel_us(t, (whole * panels + per * share) / (whole * panels + per + 20), straddle) + (paired ? 0.0 : round_us(t)));
+            const double share = (double)rest * parts / cus;   // of the CUs
             const double split_us = whole_us + per * panel_us(t, t.m == 256 ? share : 0.5, straddle) + round_us(t) + rest * parts * part_us + launch_us;
             if (split_us < best_us && split_us < us * 0.97) {
                 best_us = split_us;

@@ -112,18 +112,19 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
     // (blockIdx.x % 8; split_from is a multiple of 8) get consecutive numbers, split by split, so that
     // they work on one range of k and share its panels in their L2.
     int tile = blockIdx.x, kt0 = 0, NP = NPK, part = -1;
-    TileCoord mt;
+    TilePos at_tile;
     if (MTM == MTN && tile >= p.split_from) {
-        const int q = tile - p.split_from, all = p.split_tiles * p.splits, even = all & ~(kXcds - 1);
-        const int at = q < even ? (q & (kXcds - 1)) * (even / kXcds) + q / kXcds : q;
-        part = at / p.split_tiles;
+        const unsigned q = tile - p.split_from, all = p.split_tiles * p.splits, even = all & ~(kXcds - 1);
+        const unsigned at = q < even ? (q & (kXcds - 1)) * (even / kXcds) + q / kXcds : q;
+        part = at / (unsigned)p.split_tiles;
         tile = at - part * p.split_tiles;
-        mt = split_tile_at(p, tile);
+        at_tile = split_tile_pos(p, tile);
         kt0 = part * p.split_panels;
         NP = min(p.split_panels, NPK - kt0);
     } else {
-        mt = macro_tile_at<MTM, MTN>(p, tile);
+        at_tile = whole_tile_pos(p, tile);
     }
+    const TileCoord mt = macro_tile_at<MTM, MTN>(p, at_tile);
     // M and N are multiples of the layout tile, not necessarily of the macro
     // tile: the last row or column of macro tiles may be half inside.  Such a
     // workgroup runs the full main loop (the waves of the outer half re-read the

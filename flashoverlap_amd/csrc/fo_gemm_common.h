@@ -97,18 +97,23 @@ struct GemmParams {
     int* arrived;                               // reduction: strips of each layout tile that are stored
 };
 
-// The macro tile that workgroup `tile` of the grid computes.
-template <int MTM, int MTN>
-__device__ __forceinline__ TileCoord macro_tile_at(const GemmParams& p, int tile) {
-    if constexpr (MTM > MTN) return raster_map<kGroupM / 2, kUnitN * 2>(tile, p.GM, p.GN, p.gn_magic);
-    else return raster_map(tile, p.GM, p.GN, p.gn_magic);
+// Position of the macro tile of workgroup `tile` of the grid, and of split tile `index`: counted from
+// split_from on if that is where a wave begins (the workgroups of its parts are shared out between the XCDs
+// before they get here).
+struct TilePos {
+    int pos, by_column;   // for raster_tile
+};
+__device__ __forceinline__ TilePos whole_tile_pos(const GemmParams& p, int tile) {
+    const int total = p.GM * p.GN;
+    return {raster_pos(tile, total), raster_whole(total)};
 }
-
-// Split tile `index`: counted from split_from on, by position if that is where a wave begins (the
-// workgroups of its parts are shared out between the XCDs before they get here).
-__device__ __forceinline__ TileCoord split_tile_at(const GemmParams& p, int index) {
-    const int at = p.split_from + index;
-    return p.split_from % kWave ? raster_map(at, p.GM, p.GN, p.gn_magic) : raster_tile(at, p.GM, p.GN, p.gn_magic, p.GM * p.GN);
+__device__ __forceinline__ TilePos split_tile_pos(const GemmParams& p, int index) {
+    return p.split_from % kWave ? whole_tile_pos(p, p.split_from + index) : TilePos{p.split_from + index, p.GM * p.GN};
+}
+template <int MTM, int MTN>
+__device__ __forceinline__ TileCoord macro_tile_at(const GemmParams& p, TilePos at) {
+    if constexpr (MTM > MTN) return raster_tile<kGroupM / 2, kUnitN * 2>(at.pos, p.GM, p.GN, p.gn_magic, at.by_column);
+    else return raster_tile(at.pos, p.GM, p.GN, p.gn_magic, at.by_column);
 }
 
 // Where a part of a split tile lies in `partial`: [tile][split][wave][block i * NB + j][lane] vectors of

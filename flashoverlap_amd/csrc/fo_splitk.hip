@@ -27,7 +27,7 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const GemmParams p) {
     const int tid = threadIdx.x;
     const int strip = blockIdx.x % NB, wave = blockIdx.x / NB % 4, tile = blockIdx.x / (4 * NB);
     const int wm = wave >> 1, wn = wave & 1;
-    const TileCoord mt = split_tile_at(p, tile);
+    const TileCoord mt = macro_tile_at<MT, MT>(p, split_tile_pos(p, tile));
     if (mt.m * MT + wm * WT + 16 * strip >= p.M || mt.n * MT + wn * WT >= p.N) return;   // outside the matrix
 
     f32x4 sum[VECS];
