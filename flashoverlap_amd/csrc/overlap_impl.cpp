@@ -447,6 +447,26 @@ void OverlapImpl::GemmReduceScatterOverlap(at::Tensor A, at::Tensor B, at::Tenso
     overlapped_call(call, g, C, D.data_ptr(), cSEG_CPU, cSEG_GPU, MM, stride, "gemm_reducescatter_overlap");
 }
 
+at::Tensor OverlapImpl::AllReduceLinear(at::Tensor A, at::Tensor B, at::Tensor MM, at::Tensor RA, at::Tensor cSEG_CPU,
+                                        at::Tensor cSEG_GPU, int64_t Algo) {
+    TORCH_CHECK(A.dim() == 2 && B.dim() == 2, "allreduce_linear: A [M,K] and B [N,K] must be 2-D");
+    // C receives the GEMM's tiles; the per-group copies (the collective's stand-in) land in the result
+    at::Tensor C = at::empty({A.size(0), B.size(0)}, A.options());
+    at::Tensor out = at::empty({A.size(0), B.size(0)}, A.options());
+    SetStaging(out);
+    GemmAllReduceOverlap(A, B, C, MM, RA, 1, cSEG_CPU, cSEG_GPU, Algo, false);
+    return out;
+}
+
+at::Tensor OverlapImpl::ReduceScatterLinear(at::Tensor A, at::Tensor B, at::Tensor MM, at::Tensor RA, at::Tensor RE,
+                                            at::Tensor cSEG_CPU, at::Tensor cSEG_GPU, int64_t Algo) {
+    TORCH_CHECK(A.dim() == 2 && B.dim() == 2, "reducescatter_linear: A [M,K] and B [N,K] must be 2-D");
+    at::Tensor C = at::empty({A.size(0), B.size(0)}, A.options());
+    at::Tensor out = at::empty({A.size(0) / my_size_, B.size(0)}, A.options());
+    GemmReduceScatterOverlap(A, B, C, out, MM, RA, RE, 1, cSEG_CPU, cSEG_GPU, Algo, false);
+    return out;
+}
+
 // The bulk copy that stands in for the collective starts when the GEMM has ended, so the GEMM's
 // epilogue makes it: C is stored twice instead of being read back.
 void OverlapImpl::GemmAllReduce(at::Tensor A, at::Tensor B, at::Tensor C, int64_t Algo) {

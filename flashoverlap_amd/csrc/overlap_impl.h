@@ -69,6 +69,14 @@ class OverlapImpl : public torch::CustomClassHolder {
     // caller can own its result like it owns C in the reference.  A call whose C
     // does not match the buffer in size, dtype or device goes back to an internal one.
     void SetStaging(at::Tensor buffer);
+    // The overlapped calls with their buffers made here, for callers that keep only the result (the
+    // nn.Module layers): a fresh staging buffer [M, N], and this rank's receive buffer [M / world_size, N].
+    // Made in Python, three tensors and the arguments of a second method cost some 8 us of a call whose
+    // kernels take 20.
+    at::Tensor AllReduceLinear(at::Tensor A, at::Tensor B, at::Tensor MM, at::Tensor RA, at::Tensor cSEG_CPU,
+                               at::Tensor cSEG_GPU, int64_t Algo);
+    at::Tensor ReduceScatterLinear(at::Tensor A, at::Tensor B, at::Tensor MM, at::Tensor RA, at::Tensor RE,
+                                   at::Tensor cSEG_CPU, at::Tensor cSEG_GPU, int64_t Algo);
     // 0 = automatic (groups that complete with the GEMM are delivered by its epilogue; of the
     // others, those that complete in one round of workgroups are released together, with one
     // wait and one copy launch), 1 = one (wait, consume) launch pair per group like the

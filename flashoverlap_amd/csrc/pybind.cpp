@@ -56,6 +56,8 @@ TORCH_LIBRARY(flashoverlap_class, m) {
         .def("staging", &OverlapImpl::Staging)
         .def("set_consumer_mode", &OverlapImpl::SetConsumerMode)
         .def("set_staging", &OverlapImpl::SetStaging)
+        .def("allreduce_linear", &OverlapImpl::AllReduceLinear)
+        .def("reducescatter_linear", &OverlapImpl::ReduceScatterLinear)
         .def("set_consumer_blocks", &OverlapImpl::SetConsumerBlocks)
         .def("set_wait_timeout_ms", &OverlapImpl::SetWaitTimeoutMs)
         .def("wait_timeouts", &OverlapImpl::WaitTimeouts)
@@ -70,4 +72,5 @@ TORCH_LIBRARY(flashoverlap_op, m) {
     m.def("rmsnorm", &rmsnorm);
     m.def("reorder_rmsnorm_eps", &reorder_rmsnorm_eps);
     m.def("rmsnorm_eps", &rmsnorm_eps);
+    m.def("reorder_rmsnorm_new", &reorder_rmsnorm_new);
 }

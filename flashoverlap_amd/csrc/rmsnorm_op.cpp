@@ -40,6 +40,14 @@ void reorder_rmsnorm_eps(at::Tensor X, at::Tensor RX, at::Tensor RW, int64_t BM,
                                (void*)c10::hip::getCurrentHIPStream().stream()));
 }
 
+at::Tensor reorder_rmsnorm_new(at::Tensor X, at::Tensor RW, int64_t BM, int64_t BN, int64_t rldn, at::Tensor RA,
+                               double eps) {
+    TORCH_CHECK(X.defined() && X.dim() == 2, "reorder_rmsnorm: X must be [rows, dim]");
+    at::Tensor out = at::empty({X.size(0), X.size(1)}, X.options());
+    reorder_rmsnorm_eps(X, out, RW, BM, BN, rldn, RA, eps);
+    return out;
+}
+
 void reorder_rmsnorm(at::Tensor X, at::Tensor RX, at::Tensor RW, int64_t BM, int64_t BN, int64_t rldn,
                      at::Tensor RA) {
     reorder_rmsnorm_eps(X, RX, RW, BM, BN, rldn, RA, 1e-5);

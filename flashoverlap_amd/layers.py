@@ -41,10 +41,8 @@ class ReorderRMSNorm(nn.Module):
         self.reorder_array = tiling.reorder_indices(tm * tn, hint, device).reshape(tm, tn)
 
     def forward(self, x):
-        out = torch.empty((x.size(0), x.size(1)), dtype=x.dtype, device=x.device)
-        torch.ops.flashoverlap_op.reorder_rmsnorm_eps(x, out, self.weight, self.bm, self.bn, 1, self.reorder_array,
-                                                      self.eps)
-        return out
+        return torch.ops.flashoverlap_op.reorder_rmsnorm_new(x, self.weight, self.bm, self.bn, 1, self.reorder_array,
+                                                             self.eps)
 
 
 class RowParallelLayer(nn.Module):
@@ -92,18 +90,8 @@ class OverlapRowParallelLayer(nn.Module):
                           if comm_op == "reduce_scatter" else None)
 
     def forward(self, x):
-        n = self.weight.size(0)
         if self.comm_op == "all_reduce":
-            # tmp receives the GEMM's tiles; the per-group copies (the collective's stand-in) land in out
-            tmp = torch.empty((x.size(0), n), dtype=x.dtype, device=x.device)
-            out = torch.empty((x.size(0), n), dtype=x.dtype, device=x.device)
-            self.overlap_class.set_staging(out)
-            self.overlap_class.gemm_allreduce_overlap(x, self.weight, tmp, self.counter, self.reorder_array, 1,
-                                                      self.cseg_cpu, self.cseg_gpu, self.algo, False)
-            return out
-        tmp = torch.empty((x.size(0), n), dtype=x.dtype, device=x.device)
-        out = torch.empty((x.size(0) // self.world_size, n), dtype=x.dtype, device=x.device)
-        self.overlap_class.gemm_reducescatter_overlap(x, self.weight, tmp, out, self.counter, self.reorder_array,
-                                                      self.row_array, 1, self.cseg_cpu, self.cseg_gpu, self.algo,
-                                                      False)
-        return out
+            return self.overlap_class.allreduce_linear(x, self.weight, self.counter, self.reorder_array, self.cseg_cpu,
+                                                       self.cseg_gpu, self.algo)
+        return self.overlap_class.reducescatter_linear(x, self.weight, self.counter, self.reorder_array, self.row_array,
+                                                       self.cseg_cpu, self.cseg_gpu, self.algo)
