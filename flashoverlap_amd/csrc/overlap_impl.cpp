@@ -187,34 +187,22 @@ std::shared_ptr<SplitWorkspace> SplitWorkspace::of_stream(int device, void* stre
     return w;
 }
 
-// The GEMM, with a workspace if its shape can use one.  `signals`: some of its tiles are signalled
-// (the workspace's counters are then used, and have to start at zero).
-void OverlapImpl::launch_gemm(fo_gemm_call& call, const at::Tensor& like, bool signals) {
+// The GEMM, with a workspace if its shape can use one.
+// A captured call runs unsplit: its graph may be replayed beside later calls on this stream, after this
+// object is gone and any number of times, so neither the stream's workspace nor memory that is given back
+// when the call returns may be written by it, and nothing here lives as long as the graph.
+void OverlapImpl::launch_gemm(fo_gemm_call& call, const at::Tensor& like) {
     size_t need = 0;
     FO_CALL(fo_gemm_workspace(&call, &need));
     int step = 0;
     while (step < 3 && need > ((size_t)4 << 20 << 2 * step)) ++step;
-    if (need == 0 || step == 3) {
+    int capturing = 0;
+    if (need && step < 3) FO_CALL(fo_stream_is_capturing(gemm_stream_, &capturing));
+    if (need == 0 || step == 3 || capturing) {
         FO_CALL(fo_gemm_launch(&call, gemm_stream_));
         return;
     }
     const int64_t bytes = (int64_t)4 << 20 << 2 * step;
-    int capturing = 0;
-    FO_CALL(fo_stream_is_capturing(gemm_stream_, &capturing));
-    if (capturing) {
-        // A graph gets memory of its own (it may be replayed beside later calls on this stream): torch's
-        // allocator takes it from the graph's pool.  Captures that torch does not see run unsplit.
-        if ((void*)c10::hip::getCurrentHIPStream().stream() == gemm_stream_) {
-            at::Tensor own = at::empty({(int64_t)need}, like.options().dtype(at::kByte));
-            if (signals) own.narrow(0, 0, FO_WORKSPACE_ZEROED).zero_();
-            call.workspace = own.data_ptr();
-            call.workspace_bytes = need;
-            FO_CALL(fo_gemm_launch(&call, gemm_stream_));
-            return;
-        }
-        FO_CALL(fo_gemm_launch(&call, gemm_stream_));
-        return;
-    }
     const int device = like.device().index();
     if (!workspace_ || workspace_device_ != device || workspace_stream_ != gemm_stream_) {
         workspace_ = SplitWorkspace::of_stream(device, gemm_stream_);
@@ -250,7 +238,7 @@ void OverlapImpl::Gemm(at::Tensor A, at::Tensor B, at::Tensor C, int64_t Algo) {
     const fo_host::GemmShape s = fo_host::check_gemm(A, B, C, "mutlass_gemm");
     c10::DeviceGuard guard(A.device());
     fo_gemm_call call = describe(FO_GEMM_PLAIN, s, Algo, 1, A, B, C, at::Tensor(), false);
-    launch_gemm(call, C, false);
+    launch_gemm(call, C);
 }
 
 // Called before the GEMM is enqueued.  While the caller's stream is being captured into a
@@ -406,7 +394,7 @@ void OverlapImpl::overlapped_call(fo_gemm_call& call, const fo_host::SignalShape
         call.slice_stride = slice_stride;
     }
     fork_comm_stream(waited, g.G);
-    launch_gemm(call, C, waited > 0);
+    launch_gemm(call, C);
     consume_groups(C, dst, (int64_t)g.BM * g.BN, cseg_cpu, cseg_gpu, MM, waited, per_round, call.nslices, slice_stride);
     raise_on_timeout(MM, who);
 }
@@ -477,7 +465,7 @@ void OverlapImpl::GemmAllReduce(at::Tensor A, at::Tensor B, at::Tensor C, int64_
     void* dst = staging_like(C).data_ptr();
     const bool after = reads_from(call, dst, C.numel());
     if (!after) call.deliver = dst;
-    launch_gemm(call, C, false);
+    launch_gemm(call, C);
     if (after) bulk_consume(C.data_ptr(), dst, C.numel() * C.element_size());
 }
 

@@ -22,7 +22,7 @@
 // GEMM stream, shared by the objects that launch on it and given back with the last of them: calls on
 // one stream follow each other, and the mutex keeps a call's two launches together when several
 // threads enqueue.  Grows in three steps to at most 64 MiB; a smaller buffer that launches may still
-// be using is kept beside the larger one.
+// be using is kept beside the larger one.  Captured calls do not use it (launch_gemm).
 struct SplitWorkspace {
     std::mutex mutex;
     at::Tensor buffer[3];   // 4, 16 and 64 MiB, made when first needed
@@ -128,7 +128,7 @@ class OverlapImpl : public torch::CustomClassHolder {
     void consume_groups(const at::Tensor& C, void* dst, int64_t tile_elems, const at::Tensor& cseg_cpu,
                         const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int per_round, int nslices, int64_t slice_stride);
     void bulk_consume(const void* src, void* dst, size_t bytes);
-    void launch_gemm(fo_gemm_call& call, const at::Tensor& like, bool signals);
+    void launch_gemm(fo_gemm_call& call, const at::Tensor& like);
     int* expired_word(const at::Tensor& like);
     void refuse_checked_capture(const char* who);
     void prepare_call(const at::Tensor& MM, const char* who);

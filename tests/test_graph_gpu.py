@@ -91,3 +91,120 @@ def test_overlapped_call_replays_from_a_graph(dev, w, mode):
                 assert torch.equal(y, want_y)
     finally:
         capi.check(capi.lib().fo_set_wait_timeout_ms(5000))
+
+
+@pytest.fixture
+def short_waits():
+    """A wait that cannot be satisfied (graph branches run in the wrong order) must fail the test, not stall it."""
+    capi.check(capi.lib().fo_set_wait_timeout_ms(2000))
+    yield
+    capi.check(capi.lib().fo_set_wait_timeout_ms(5000))
+
+
+def _whole_numbers(dev, dt, gen, *shape):
+    """Small integers: every sum is exact in fp32, so a call that is split over K and one that is not agree bit for bit."""
+    return torch.randint(-2, 3, shape, generator=gen).to(dt).to(dev)
+
+
+@pytest.mark.parametrize("M,N,K,w,ws", [
+    (1024, 1024, 512, 4, 1),       # every group is delivered by the epilogue
+    (128, 4096, 4096, 32, 1),      # split over K when it is not captured, every group delivered
+    (128, 4096, 4096, 8, 4),
+    (8192, 4352, 64, 100, 1),      # groups of a round released together, the last ones delivered
+    (8192, 4352, 64, 100, 4),
+    (4352, 4096, 1544, 200, 1),    # the same, and sixteen tiles split over K when it is not captured
+])
+def test_default_mode_replays_from_a_graph(dev, short_waits, M, N, K, w, ws):
+    """The automatic mode: a warmed call that is captured allocates nothing, and every replay gives what the
+    eager call gives, also with eager calls of the same object in between."""
+    flashoverlap_amd.load()
+    algo, dt = 1, torch.bfloat16
+    BM, BN, _ = capi.algo_tile(algo)
+    TM, TN = M // BM, N // BN
+    cseg = tiling.uniform_cseg(TM * TN, w)
+    cs = torch.tensor(cseg, dtype=torch.int32)
+    cs_gpu = cs.to(dev)
+    RA = tiling.reorder_indices(TM * TN, tiling.raster_hint(M, N, algo), dev).reshape(TM, TN)
+    RE = tiling.generate_row_remap_array(M, N, BM, BN, cseg, ws, dev) if ws > 1 else None
+    gen = torch.Generator().manual_seed(13)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        o = torch.classes.flashoverlap_class.OverlapImpl()
+        o.mccl_init(ws - 1, ws, torch.ops.flashoverlap_op.generate_mccl_id())
+        o.mutlass_init()
+        o.overlap_init()
+        A, B = _whole_numbers(dev, dt, gen, M, K), _whole_numbers(dev, dt, gen, N, K)
+        W = (1 + 0.1 * torch.randn(N, generator=gen)).to(dt).to(dev)
+        C, recv, y = (torch.zeros(rows, N, dtype=dt, device=dev) for rows in (M, M // ws, M // ws))
+        counter = torch.zeros(len(cseg), dtype=torch.int32, device=dev)
+        o.set_staging(recv)
+
+        def call():
+            if ws > 1:
+                o.gemm_reducescatter_overlap(A, B, C, recv, counter, RA, RE, 1, cs, cs_gpu, algo, False)
+            else:
+                o.gemm_allreduce_overlap(A, B, C, counter, RA, 1, cs, cs_gpu, algo, False)
+            torch.ops.flashoverlap_op.reorder_rmsnorm(recv, y, W, BM // ws, BN, 1, RA)
+
+        for _ in range(2):
+            call()
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            made = torch.cuda.memory_stats()["allocation.all.allocated"]
+            call()
+            assert torch.cuda.memory_stats()["allocation.all.allocated"] == made
+        for replay in range(3):
+            print(f"graph replay {replay} {M}x{N}x{K} w={w} ws={ws}", flush=True)
+            A.copy_(_whole_numbers(dev, dt, gen, M, K))
+            call()
+            side.synchronize()
+            want = [t.clone() for t in (C, recv, y)]
+            assert want[2].float().abs().sum() > 0
+            for t in (C, recv, y):
+                t.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert o.wait_timeouts(True) == 0 and not counter.any()
+            assert all(torch.equal(t, w_) for t, w_ in zip((C, recv, y), want))
+
+
+def test_capture_that_torch_does_not_see(dev):
+    """A capture begun through the runtime on torch's current stream: torch's allocator knows nothing of it and
+    hands memory that is given back inside it to the next tensor.  The graph may write to nothing but C."""
+    import ctypes
+    flashoverlap_amd.load()
+    L, dt = capi.lib(), torch.bfloat16
+    M, N, K = 128, 4096, 4096       # split over K when it is not captured
+    gen = torch.Generator().manual_seed(17)
+    side = torch.cuda.Stream()
+    stream = ctypes.c_void_p(side.cuda_stream)
+    graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+    with torch.cuda.stream(side):
+        o = torch.classes.flashoverlap_class.OverlapImpl()
+        o.mutlass_init()
+        A, B = _whole_numbers(dev, dt, gen, M, K), _whole_numbers(dev, dt, gen, N, K)
+        C = torch.zeros(M, N, dtype=dt, device=dev)
+        o.mutlass_gemm(A, B, C, 1)
+        side.synchronize()
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        assert L.hipStreamBeginCapture(stream, 2) == 0       # relaxed
+        o.mutlass_gemm(A, B, C, 1)
+        assert L.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+        assert L.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+        others = [torch.full((n << 18,), 7.0, device=dev) for n in (4, 16, 17, 64) for _ in range(2)]
+        for replay in range(3):
+            print(f"raw graph replay {replay}", flush=True)
+            A.copy_(_whole_numbers(dev, dt, gen, M, K))
+            want = (A.float() @ B.float().t()).to(dt)
+            C.zero_()
+            assert L.hipGraphLaunch(run, stream) == 0
+            side.synchronize()
+            assert torch.equal(C, want)
+            assert all((t == 7.0).all() for t in others)
+            o.mutlass_gemm(A, B, C, 1)                       # eager, split
+            assert torch.equal(C, want)
+        side.synchronize()
+        assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
