@@ -225,12 +225,22 @@ void OverlapImpl::launch_gemm(fo_gemm_call& call, const at::Tensor& like) {
     FO_CALL(fo_gemm_launch(&call, gemm_stream_));
 }
 
-// Whether a receive buffer shares memory with an operand: then it cannot be written while the GEMM reads.
-static bool reads_from(const fo_gemm_call& c, const void* dst, int64_t dst_elems) {
-    const auto hits = [&](const void* p, int64_t elems) {
-        return (const char*)dst < (const char*)p + 2 * elems && (const char*)p < (const char*)dst + 2 * dst_elems;
-    };
-    return hits(c.A, (int64_t)c.M * c.K) || hits(c.B, (int64_t)c.N * c.K);
+static bool shares_memory(const void* p, int64_t elems, const void* dst, int64_t dst_elems) {
+    return (const char*)dst < (const char*)p + 2 * elems && (const char*)p < (const char*)dst + 2 * dst_elems;
+}
+static bool inside_output(const fo_gemm_call& c, const void* dst, int64_t dst_elems) {
+    return shares_memory(c.D, (int64_t)c.M * c.N, dst, dst_elems);
+}
+
+// Whether the GEMM's epilogue may write the receive buffer: not if it shares memory with an operand, which
+// other workgroups still read, nor with C, whose rows other workgroups write (a rank's receive buffer can
+// be the first rows of C: a copy that starts when its group is complete writes rows of groups that are
+// complete too).  C itself as the buffer of an all-reduce is no such case: both stores of an element are
+// made by one lane, to one address, with one value.
+static bool can_deliver(const fo_gemm_call& c, const void* dst, int64_t dst_elems) {
+    if (shares_memory(c.A, (int64_t)c.M * c.K, dst, dst_elems) || shares_memory(c.B, (int64_t)c.N * c.K, dst, dst_elems))
+        return false;
+    return !inside_output(c, dst, dst_elems) || (dst == c.D && c.mode != FO_GEMM_SCATTER);
 }
 
 void OverlapImpl::Gemm(at::Tensor A, at::Tensor B, at::Tensor C, int64_t Algo) {
@@ -304,9 +314,12 @@ int OverlapImpl::groups_to_wait_for(const fo_gemm_call& call, const int* cseg, i
 // with its norm, 133 of them of the host, and takes 165; 7424x6016x640 in 5 of 302 148 -> 130, 9856x6400x1408
 // in 14 of 275 253 -> 230.  It also leaves the automatic mode without the persistent kernel, of which
 // two (of two objects, on two streams) can hold the registers that a GEMM they wait for needs.
+//
+// in_order: dst lies in C, and a group's copy writes where an earlier group's is read from: the copies
+// follow each other, the last one too.
 void OverlapImpl::consume_groups(const at::Tensor& C, void* dst, int64_t tile_elems, const at::Tensor& cseg_cpu,
                                  const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int per_round,
-                                 int nslices, int64_t slice_stride) {
+                                 int nslices, int64_t slice_stride, bool in_order) {
     const int G = (int)cseg_cpu.numel();
     const int* cseg = cseg_cpu.data_ptr<int>();
     const int slice_first = slice_stride ? 0 : (int)my_rank_;      // stride 0: only this rank's slice
@@ -340,6 +353,7 @@ void OverlapImpl::consume_groups(const at::Tensor& C, void* dst, int64_t tile_el
         // (10-20 us on this platform) between its copy and the caller's next kernel.
         const bool last = g == G - 1;
         void* stream = last ? gemm_stream_ : comm_stream_;
+        if (last && in_order && g > 0) FO_CALL(fo_stream_join(comm_stream_, gemm_stream_));
         const int64_t comm = tile_elems * cseg[g];
         // the groups up to `end` complete in the round in which this one does
         int end = g + 1;
@@ -383,9 +397,9 @@ void OverlapImpl::overlapped_call(fo_gemm_call& call, const fo_host::SignalShape
     call.MM = MM.data_ptr<int>();
     const int64_t kept = (int64_t)call.M * call.N / (slice_stride ? 1 : call.nslices);
     int per_round = 0;
-    const int waited = reads_from(call, dst, kept) ? g.G
-                                                   : groups_to_wait_for(call, cseg_cpu.data_ptr<int>(), call.nslices,
-                                                                        &call.deliver_from, &per_round);
+    const int waited = can_deliver(call, dst, kept) ? groups_to_wait_for(call, cseg_cpu.data_ptr<int>(), call.nslices,
+                                                                         &call.deliver_from, &per_round)
+                                                    : g.G;
     if (waited < g.G) {
         call.deliver = dst;
         call.group_start = group_start_.data_ptr<int>();
@@ -395,7 +409,8 @@ void OverlapImpl::overlapped_call(fo_gemm_call& call, const fo_host::SignalShape
     }
     fork_comm_stream(waited, g.G);
     launch_gemm(call, C);
-    consume_groups(C, dst, (int64_t)g.BM * g.BN, cseg_cpu, cseg_gpu, MM, waited, per_round, call.nslices, slice_stride);
+    consume_groups(C, dst, (int64_t)g.BM * g.BN, cseg_cpu, cseg_gpu, MM, waited, per_round, call.nslices, slice_stride,
+                   inside_output(call, dst, kept));
     raise_on_timeout(MM, who);
 }
 
@@ -463,7 +478,7 @@ void OverlapImpl::GemmAllReduce(at::Tensor A, at::Tensor B, at::Tensor C, int64_
     c10::DeviceGuard guard(A.device());
     fo_gemm_call call = describe(FO_GEMM_PLAIN, s, Algo, 1, A, B, C, at::Tensor(), false);
     void* dst = staging_like(C).data_ptr();
-    const bool after = reads_from(call, dst, C.numel());
+    const bool after = !can_deliver(call, dst, C.numel());
     if (!after) call.deliver = dst;
     launch_gemm(call, C);
     if (after) bulk_consume(C.data_ptr(), dst, C.numel() * C.element_size());

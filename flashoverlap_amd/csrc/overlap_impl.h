@@ -126,7 +126,8 @@ class OverlapImpl : public torch::CustomClassHolder {
     int groups_to_wait_for(const fo_gemm_call& call, const int* cseg, int nslices, int* first_slot, int* per_round);
     void fork_comm_stream(int waited, int G);
     void consume_groups(const at::Tensor& C, void* dst, int64_t tile_elems, const at::Tensor& cseg_cpu,
-                        const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int per_round, int nslices, int64_t slice_stride);
+                        const at::Tensor& cseg_gpu, at::Tensor& MM, int waited, int per_round, int nslices, int64_t slice_stride,
+                        bool in_order);
     void bulk_consume(const void* src, void* dst, size_t bytes);
     void launch_gemm(fo_gemm_call& call, const at::Tensor& like);
     int* expired_word(const at::Tensor& like);

@@ -136,3 +136,59 @@ def test_groups_of_a_round_released_together(api, dev, ws, stacked, group):
         assert o.wait_timeouts(True) == 0 and not mm.any()
         got.append((c, d))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("M,N,K,cseg", [
+    (1024, 1024, 512, [16, 16, 0, 20, 12]),      # one round: all of it would be delivered
+    (8192, 2304, 64, [300, 300, 424, 64, 64]),   # groups of a round, and a last round
+])
+@pytest.mark.parametrize("ws,rank", [(2, 1), (4, 0), (4, 3)])
+def test_receive_buffer_in_the_first_rows_of_c(api, dev, M, N, K, cseg, ws, rank):
+    """D = C[:M / ws]: a group's rows are written over rows of groups that are complete, one group after the other."""
+    algo, dt = 1, torch.bfloat16
+    print(f"D in C {M}x{N}x{K} rank {rank} of {ws}", flush=True)
+    BM, BN, _ = capi.algo_tile(algo)
+    TM, TN = M // BM, N // BN
+    cs = torch.tensor(cseg, dtype=torch.int32)
+    RA = tiling.reorder_indices(TM * TN, tiling.raster_hint(M, N, algo), dev).reshape(TM, TN)
+    RE = tiling.generate_row_remap_array(M, N, BM, BN, cseg, ws, dev)
+    A, B = _inputs(dev, dt, M, N, K)
+    o = _object(api, 0, rank, ws)
+    mm = torch.zeros(len(cseg), dtype=torch.int32, device=dev)
+    want_c, want_d = torch.empty(M, N, dtype=dt, device=dev), torch.empty(M // ws, N, dtype=dt, device=dev)
+    o.gemm_reducescatter_overlap(A, B, want_c, want_d, mm, RA, RE, 1, cs, cs.to(dev), algo, False)
+    for mode in (0, 1):
+        o.set_consumer_mode(mode)
+        for _ in range(3):
+            c = torch.full((M, N), 7.0, dtype=dt, device=dev)
+            o.gemm_reducescatter_overlap(A, B, c, c[:M // ws], mm, RA, RE, 1, cs, cs.to(dev), algo, False)
+            torch.cuda.synchronize()
+            assert o.wait_timeouts(True) == 0 and not mm.any()
+            assert torch.equal(c[:M // ws], want_d) and torch.equal(c[M // ws:], want_c[M // ws:])
+
+
+@pytest.mark.parametrize("M,N,K,group", [(1024, 1024, 512, 8), (8192, 2304, 64, 200), (128, 4096, 4096, 8)])
+def test_all_reduce_in_place(api, dev, M, N, K, group):
+    """The staging buffer is C itself, with and without overlap: C is what it is with a buffer of its own."""
+    algo, dt = 1, torch.float16
+    BM, BN, _ = capi.algo_tile(algo)
+    TM, TN = M // BM, N // BN
+    cseg = tiling.uniform_cseg(TM * TN, group)
+    cs = torch.tensor(cseg, dtype=torch.int32)
+    RA = tiling.reorder_indices(TM * TN, tiling.raster_hint(M, N, algo), dev).reshape(TM, TN)
+    A, B = _inputs(dev, dt, M, N, K)
+    o = _object(api, 0)
+    mm = torch.zeros(len(cseg), dtype=torch.int32, device=dev)
+    got = []
+    for in_place in (False, True):
+        c = torch.full((2, M, N), 7.0, dtype=dt, device=dev)
+        other = torch.empty(M, N, dtype=dt, device=dev)
+        o.set_staging(c[0] if in_place else other)
+        o.gemm_allreduce_overlap(A, B, c[0], mm, RA, 1, cs, cs.to(dev), algo, False)
+        torch.cuda.synchronize()
+        o.set_staging(c[1] if in_place else other)
+        o.gemm_allreduce(A, B, c[1], algo)
+        torch.cuda.synchronize()
+        assert o.wait_timeouts(True) == 0 and not mm.any()
+        got.append(c)
+    assert torch.equal(got[0], got[1])
