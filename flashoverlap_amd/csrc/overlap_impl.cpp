@@ -210,19 +210,33 @@ void OverlapImpl::launch_gemm(fo_gemm_call& call, const at::Tensor& like) {
         workspace_stream_ = gemm_stream_;
     }
     std::lock_guard<std::mutex> lock(workspace_->mutex);
-    at::Tensor& buffer = workspace_->buffer[step];
-    if (!buffer.defined()) {
-        buffer = at::empty({bytes}, like.options().dtype(at::kByte));
-        buffer.narrow(0, 0, FO_WORKSPACE_ZEROED).zero_();
-        const auto current = c10::hip::getCurrentHIPStream();
-        if ((void*)current.stream() != gemm_stream_) {   // once per buffer: filled on one stream, used on another
-            current.synchronize();
-            buffer.record_stream(c10::hip::getStreamFromExternal((hipStream_t)gemm_stream_, (c10::DeviceIndex)device));
-        }
+    if (!workspace_->buffer[step].defined()) make_workspace(like, step, bytes);
+    if (workspace_->buffer[step].defined()) {
+        call.workspace = workspace_->buffer[step].data_ptr();
+        call.workspace_bytes = (size_t)bytes;
     }
-    call.workspace = buffer.data_ptr();
-    call.workspace_bytes = (size_t)bytes;
     FO_CALL(fo_gemm_launch(&call, gemm_stream_));
+}
+
+// The workspace only makes a call faster.  Where the device has no memory for it the call runs without, and
+// so do the later ones of that size on this stream: an allocation that fails first gives all cached memory back
+// and waits for the device, which must not happen on every call, and a shape keeps its order of additions.
+void OverlapImpl::make_workspace(const at::Tensor& like, int step, int64_t bytes) {
+    if (workspace_->refused[step]) return;
+    at::Tensor made;
+    try {
+        made = at::empty({bytes}, like.options().dtype(at::kByte));
+    } catch (const c10::OutOfMemoryError&) {
+        workspace_->refused[step] = true;
+        return;
+    }
+    made.narrow(0, 0, FO_WORKSPACE_ZEROED).zero_();
+    const auto current = c10::hip::getCurrentHIPStream();
+    if ((void*)current.stream() != gemm_stream_) {   // once per buffer: filled on one stream, used on another
+        current.synchronize();
+        made.record_stream(c10::hip::getStreamFromExternal((hipStream_t)gemm_stream_, (c10::DeviceIndex)workspace_device_));
+    }
+    workspace_->buffer[step] = std::move(made);
 }
 
 static bool shares_memory(const void* p, int64_t elems, const void* dst, int64_t dst_elems) {

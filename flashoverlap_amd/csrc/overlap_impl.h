@@ -26,6 +26,7 @@
 struct SplitWorkspace {
     std::mutex mutex;
     at::Tensor buffer[3];   // 4, 16 and 64 MiB, made when first needed
+    bool refused[3] = {};   // there was no memory for it
     static std::shared_ptr<SplitWorkspace> of_stream(int device, void* stream);
 };
 
@@ -130,6 +131,7 @@ class OverlapImpl : public torch::CustomClassHolder {
                         bool in_order);
     void bulk_consume(const void* src, void* dst, size_t bytes);
     void launch_gemm(fo_gemm_call& call, const at::Tensor& like);
+    void make_workspace(const at::Tensor& like, int step, int64_t bytes);
     int* expired_word(const at::Tensor& like);
     void refuse_checked_capture(const char* who);
     void prepare_call(const at::Tensor& MM, const char* who);

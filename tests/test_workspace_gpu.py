@@ -1,0 +1,51 @@
+"""The workspace of GEMMs that are split over K: an object makes it where it can, and a call for which it cannot
+be made is computed without.  Integer-valued inputs: split or not, the result is the same bit for bit."""
+import pytest
+import torch
+
+import flashoverlap_amd
+
+pytestmark = pytest.mark.gpu
+
+M, N, K = 128, 4096, 7168      # 32 tiles in 8 parts of 64 KiB: the workspace is the largest one, 64 MiB
+
+
+@pytest.fixture
+def call(dev):
+    """A plain GEMM on an object and a stream of its own, and what it has to give."""
+    flashoverlap_amd.load()
+    gen = torch.Generator().manual_seed(19)
+    A, B = (torch.randint(-2, 3, (r, K), generator=gen).to(torch.bfloat16).to(dev) for r in (M, N))
+    want = (A.float() @ B.float().t()).to(torch.bfloat16)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        o = torch.classes.flashoverlap_class.OverlapImpl()
+        o.mutlass_init()
+        C = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+
+    def run():
+        C.zero_()
+        torch.cuda.synchronize()
+        o.mutlass_gemm(A, B, C, 1)
+        torch.cuda.synchronize()
+        return torch.equal(C, want)
+
+    run.stream = stream
+    return run
+
+
+def test_no_memory_for_the_workspace(call):
+    def reserved():
+        return torch.cuda.memory_reserved() / torch.cuda.get_device_properties(0).total_memory
+
+    ooms = torch.cuda.memory_stats()["num_ooms"]
+    with torch.cuda.stream(call.stream):
+        torch.cuda.empty_cache()
+        torch.cuda.set_per_process_memory_fraction(reserved())
+        try:
+            assert call() and call()
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert torch.cuda.memory_stats()["num_ooms"] == ooms + 1    # asked for once
+        assert call()
