@@ -6,6 +6,7 @@
 #include "overlap_impl.h"
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 
 #include <map>
@@ -223,6 +224,8 @@ void OverlapImpl::launch_gemm(fo_gemm_call& call, const at::Tensor& like) {
 // and waits for the device, which must not happen on every call, and a shape keeps its order of additions.
 void OverlapImpl::make_workspace(const at::Tensor& like, int step, int64_t bytes) {
     if (workspace_->refused[step]) return;
+    // made and cleared on the GEMM's stream, whichever is current
+    c10::hip::HIPStreamGuard on(c10::hip::getStreamFromExternal((hipStream_t)gemm_stream_, (c10::DeviceIndex)workspace_device_));
     at::Tensor made;
     try {
         made = at::empty({bytes}, like.options().dtype(at::kByte));
@@ -231,11 +234,6 @@ void OverlapImpl::make_workspace(const at::Tensor& like, int step, int64_t bytes
         return;
     }
     made.narrow(0, 0, FO_WORKSPACE_ZEROED).zero_();
-    const auto current = c10::hip::getCurrentHIPStream();
-    if ((void*)current.stream() != gemm_stream_) {   // once per buffer: filled on one stream, used on another
-        current.synchronize();
-        made.record_stream(c10::hip::getStreamFromExternal((hipStream_t)gemm_stream_, (c10::DeviceIndex)workspace_device_));
-    }
     workspace_->buffer[step] = std::move(made);
 }
 

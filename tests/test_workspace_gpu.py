@@ -27,11 +27,11 @@ def call(dev):
     def run():
         C.zero_()
         torch.cuda.synchronize()
-        o.mutlass_gemm(A, B, C, 1)
+        run.launch()
         torch.cuda.synchronize()
-        return torch.equal(C, want)
+        return run.right()
 
-    run.stream = stream
+    run.stream, run.launch, run.right = stream, lambda: o.mutlass_gemm(A, B, C, 1), lambda: torch.equal(C, want)
     return run
 
 
@@ -49,3 +49,13 @@ def test_no_memory_for_the_workspace(call):
             torch.cuda.set_per_process_memory_fraction(1.0)
         assert torch.cuda.memory_stats()["num_ooms"] == ooms + 1    # asked for once
         assert call()
+
+
+def test_first_call_from_another_stream(call):
+    """torch's current stream is not the GEMM's when the workspace is made."""
+    before = torch.cuda.memory_stats(0)["allocation.all.allocated"]
+    assert torch.cuda.current_stream() != call.stream
+    call.launch()
+    assert torch.cuda.memory_stats(0)["allocation.all.allocated"] > before
+    torch.cuda.synchronize()
+    assert call.right() and call()
