@@ -224,6 +224,11 @@ void OverlapImpl::launch_gemm(fo_gemm_call& call, const at::Tensor& like) {
 // and waits for the device, which must not happen on every call, and a shape keeps its order of additions.
 void OverlapImpl::make_workspace(const at::Tensor& like, int step, int64_t bytes) {
     if (workspace_->refused[step]) return;
+    // Taking memory can mean a hipMalloc, which would end a capture of the current stream (the GEMM's own is not
+    // being captured, launch_gemm): the next call makes the buffer.
+    int capturing = 0;
+    FO_CALL(fo_stream_is_capturing((void*)c10::hip::getCurrentHIPStream().stream(), &capturing));
+    if (capturing) return;
     // made and cleared on the GEMM's stream, whichever is current
     c10::hip::HIPStreamGuard on(c10::hip::getStreamFromExternal((hipStream_t)gemm_stream_, (c10::DeviceIndex)workspace_device_));
     at::Tensor made;

@@ -59,3 +59,22 @@ def test_first_call_from_another_stream(call):
     assert torch.cuda.memory_stats(0)["allocation.all.allocated"] > before
     torch.cuda.synchronize()
     assert call.right() and call()
+
+
+def test_first_call_while_another_stream_is_captured(call):
+    """The GEMM's stream is not the one that is captured: the call runs at once, and takes no memory."""
+    graph = torch.cuda.CUDAGraph()
+    other = torch.cuda.Stream()
+    x = torch.zeros(1024, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=other, capture_error_mode="thread_local"):
+        x.add_(1)
+        made = torch.cuda.memory_stats()["allocation.all.allocated"]
+        call.launch()
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == made
+    torch.cuda.synchronize()
+    assert call.right()
+    for _ in range(2):
+        graph.replay()
+        assert call()
+    assert (x == 2).all()
