@@ -6,6 +6,7 @@
 #include <atomic>
 #include <string_view>
 #include <type_traits>
+#include <utility>
 
 #include "fo_gemm_body.h"
 #include "fo_internal.h"
@@ -176,7 +177,7 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
     // An event pair armed by fo_time_next_launch belongs to this call whether or not it gets as far
     // as a launch: taken here, ahead of the validation, so that a rejected call cannot leave it
     // behind for some later, unrelated launch.
-    const LaunchTimer timer = t_launch_timer;
+    LaunchTimer timer = t_launch_timer;
     t_launch_timer = LaunchTimer{};
     if (timer.start) {   // a dispatch that carries events cannot be recorded into a graph
         hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -242,7 +243,7 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
     if ((uintptr_t)c.deliver & 15) return fail(FO_ERR_ARG, "fo_gemm: operands must be 16-byte aligned");
     if (is_skinny(c)) return launch_skinny(dtype, M, N, K, A, B, D, c.deliver, timer, stream);
     Plan plan;
-    if (int e = plan_for(c, c.workspace && !timer.start, &plan)) return e;
+    if (int e = plan_for(c, c.workspace, &plan)) return e;
     if (c.workspace_bytes < plan.bytes)
         if (int e = plan_for(c, false, &plan)) return e;
     p.GM = (M + plan.macro.m - 1) / plan.macro.m; p.GN = (N + plan.macro.n - 1) / plan.macro.n;
@@ -254,6 +255,8 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
         p.partial = (float*)((char*)c.workspace + FO_WORKSPACE_ZEROED);
     }
     const int macro = plan.macro.m;
+    hipEvent_t reduced = nullptr;   // of a split call the pair spans both launches
+    if (plan.tiles) std::swap(reduced, timer.stop);
     const DeviceFacts* facts;
     if (int e = device_facts(&facts)) return e;
     // A workgroup that has its CU to itself takes the ring of four panels ahead: nothing else hides the latency of
@@ -266,7 +269,7 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
         rc = macro == 256 ? launch_mt<_Float16, 256>(mode, edge, p, timer, stream) : launch_mt<_Float16, 128>(mode, edge, p, timer, stream);
     else
         rc = macro == 256 ? launch_mt<__bf16, 256>(mode, edge, p, timer, stream) : launch_mt<__bf16, 128>(mode, edge, p, timer, stream);
-    if (rc == FO_OK && plan.tiles) rc = launch_split_reduce(mode, dtype, macro, p, stream);
+    if (rc == FO_OK && plan.tiles) rc = launch_split_reduce(mode, dtype, macro, p, reduced, stream);
     return rc;
 }
 

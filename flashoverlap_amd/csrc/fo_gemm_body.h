@@ -588,7 +588,7 @@ static int launch_gemm_kernel(const GemmParams& p, const LaunchTimer& timer, hip
         configured.fetch_or(bit, std::memory_order_release);
     }
     const int grid = p.split_from + p.split_tiles * p.splits;
-    if (timer.start) hipExtLaunchKernelGGL(KERN, dim3(grid), dim3(256), SMEM, stream, timer.start, timer.stop, 0, p);
+    if (timer.start || timer.stop) hipExtLaunchKernelGGL(KERN, dim3(grid), dim3(256), SMEM, stream, timer.start, timer.stop, 0, p);
     else hipLaunchKernelGGL(KERN, dim3(grid), dim3(256), SMEM, stream, p);
     FO_HIP(hipGetLastError());
     return FO_OK;

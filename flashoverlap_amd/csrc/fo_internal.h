@@ -24,6 +24,7 @@ int algo_tile(int algo, int* BM, int* BN, int* BK);
 // fo_time_next_launch: a pair of events that the next GEMM or RMSNorm launch of this thread
 // attaches to its own dispatch, so that the time between them is the kernel's, without the
 // launch gaps an event pair recorded around the launch includes.  Taken by the launch that uses it.
+// A call of two launches attaches `start` to the first and `stop` to the second.
 struct LaunchTimer {
     hipEvent_t start = nullptr, stop = nullptr;
 };
@@ -46,8 +47,9 @@ constexpr int kSkinnyRows = 32;
 int launch_skinny(int dtype, int M, int N, int K, const void* A, const void* B, void* D, void* D2, const LaunchTimer& timer,
                   hipStream_t stream);
 
-// fo_splitk.hip: sums the parts of the split tiles and stores the tiles as the GEMM's epilogue would
-int launch_split_reduce(int mode, int dtype, int macro, const GemmParams& p, hipStream_t stream);
+// fo_splitk.hip: sums the parts of the split tiles and stores the tiles as the GEMM's epilogue would (stop: null, or
+// an event of its end)
+int launch_split_reduce(int mode, int dtype, int macro, const GemmParams& p, hipEvent_t stop, hipStream_t stream);
 
 // fo_static.hip
 int gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN, const int* cseg, int G, const void* A,

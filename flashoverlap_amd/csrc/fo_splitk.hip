@@ -9,6 +9,7 @@
 // tile alone (eight of 64 KiB at some 50 bytes per ns: 9 us), here every 16 rows of a wavefront's
 // quadrant are a workgroup.  Bound by the memory-side cache the parts come from.
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 
 #include "fo_gemm_common.h"
 #include "fo_internal.h"
@@ -111,19 +112,25 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const GemmParams p) {
     }
 }
 
-template <typename T, int MT>
-static int launch_t(int mode, const GemmParams& p, hipStream_t stream) {
+template <typename T, int MT, int MODE>
+static int launch_one(const GemmParams& p, hipEvent_t stop, hipStream_t stream) {
     const dim3 grid(p.split_tiles * 4 * (MT / 32)), block(256);
-    if (mode == kPlain) hipLaunchKernelGGL((split_reduce_kernel<T, MT, kPlain>), grid, block, 0, stream, p);
-    else if (mode == kSignal) hipLaunchKernelGGL((split_reduce_kernel<T, MT, kSignal>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((split_reduce_kernel<T, MT, kScatter>), grid, block, 0, stream, p);
+    if (stop) hipExtLaunchKernelGGL((split_reduce_kernel<T, MT, MODE>), grid, block, 0, stream, nullptr, stop, 0, p);
+    else hipLaunchKernelGGL((split_reduce_kernel<T, MT, MODE>), grid, block, 0, stream, p);
     FO_HIP(hipGetLastError());
     return FO_OK;
 }
 
-int launch_split_reduce(int mode, int dtype, int macro, const GemmParams& p, hipStream_t stream) {
-    if (dtype == FO_F16) return macro == 256 ? launch_t<_Float16, 256>(mode, p, stream) : launch_t<_Float16, 128>(mode, p, stream);
-    return macro == 256 ? launch_t<__bf16, 256>(mode, p, stream) : launch_t<__bf16, 128>(mode, p, stream);
+template <typename T, int MT>
+static int launch_t(int mode, const GemmParams& p, hipEvent_t stop, hipStream_t stream) {
+    if (mode == kPlain) return launch_one<T, MT, kPlain>(p, stop, stream);
+    return mode == kSignal ? launch_one<T, MT, kSignal>(p, stop, stream) : launch_one<T, MT, kScatter>(p, stop, stream);
+}
+
+int launch_split_reduce(int mode, int dtype, int macro, const GemmParams& p, hipEvent_t stop, hipStream_t stream) {
+    if (dtype == FO_F16)
+        return macro == 256 ? launch_t<_Float16, 256>(mode, p, stop, stream) : launch_t<_Float16, 128>(mode, p, stop, stream);
+    return macro == 256 ? launch_t<__bf16, 256>(mode, p, stop, stream) : launch_t<__bf16, 128>(mode, p, stop, stream);
 }
 
 }  // namespace fo

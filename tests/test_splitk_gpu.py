@@ -183,3 +183,38 @@ def test_small_tile_delivers_into_larger_layout_tiles(dev, M, N, K, algo, ws):
     out = torch.empty(T * BM, BN, dtype=dt, device=dev)
     out[RE.long() if ws > 1 else slice(None)] = rows.view(-1, BN)
     assert torch.equal(D, out) and torch.equal(D2, out) and mm.item() == 0
+
+
+def test_timed_call_runs_what_the_untimed_one_does(dev):
+    """The event pair of fo_time_next_launch spans both launches of a split call, and leaves the call as it is."""
+    L, dt, (M, N, K) = capi.lib(), torch.bfloat16, (128, 4096, 7168)
+    g = torch.Generator().manual_seed(5)
+    A, B = (torch.randn(r, K, generator=g).to(dt).to(dev) for r in (M, N))
+    evs = [C.c_void_p() for _ in range(4)]
+    for e in evs:
+        capi.check(L.fo_event_create(C.byref(e)))
+    inner0, inner1, outer0, outer1 = evs
+    got = []
+    for timed, split in ((False, False), (False, True), (True, True)):
+        D = torch.zeros(M, N, dtype=dt, device=dev)
+        c, ws, need = _call(0, dt, 1, A, B, D)
+        assert need > 4096
+        if not split:
+            c.workspace, c.workspace_bytes = None, 0
+        torch.cuda.synchronize()
+        capi.check(L.fo_event_record(outer0, None))
+        if timed:
+            capi.check(L.fo_time_next_launch(inner0, inner1))
+        capi.check(L.fo_gemm_launch(C.byref(c), None))
+        capi.check(L.fo_event_record(outer1, None))
+        torch.cuda.synchronize()
+        got.append(D)
+    assert not torch.equal(got[0], got[1])      # the order of additions shows which of the two ran
+    assert torch.equal(got[1], got[2])
+    inner, outer = C.c_float(), C.c_float()
+    capi.check(L.fo_event_elapsed_ms(inner0, inner1, C.byref(inner)))
+    capi.check(L.fo_event_elapsed_ms(outer0, outer1, C.byref(outer)))
+    for e in evs:
+        capi.check(L.fo_event_destroy(e))
+    assert 0 < inner.value <= outer.value
+    assert 2 * (M + N) * K / (inner.value * 1e-3) < 10e12    # the operands' bytes alone: the first launch is in it
