@@ -1,4 +1,4 @@
-"""Build-time checks on the code the compiler makes of the GEMM kernel (no GPU needed).
+"""Build-time checks on the code the compiler makes of the GEMM kernels (no GPU needed).
 
 The kernel issues its MFMAs from inline assembly, which the compiler treats as
 opaque: it neither knows their latency nor inserts the wait states the hardware
@@ -20,23 +20,39 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 MIN_WAIT_STATES = 16   # the longest MFMA of this family needs fewer before its result may be read
 
 
-@pytest.fixture(scope="module")
-def gemm_asm(tmp_path_factory):
+# The files that instantiate the kernel body, and how often
+INSTANCES = {
+    "fo_gemm.hip": 40,        # 2 types x 2 macro tiles x (plain 2 + plain any-shape 2 + signal 3 + scatter 3)
+    "fo_gemm_tall.hip": 8,    # 2 types x (plain + plain any-shape + signal + scatter)
+    "fo_gemm_deep.hip": 16,   # 2 types x 2 macro tiles x the same
+}
+
+
+@pytest.fixture(scope="module", params=list(INSTANCES))
+def gemm_asm(request, tmp_path_factory):
     hipcc = os.path.join(build.ROCM, "bin", "hipcc")
     if not os.path.exists(hipcc):
         pytest.skip("no hipcc")
-    out = tmp_path_factory.mktemp("asm") / "fo_gemm.s"
+    out = tmp_path_factory.mktemp("asm") / "gemm.s"
     flags = [f for f in build.HIPCC_FLAGS if f != "-fPIC"]
-    cmd = [hipcc, *flags, "--cuda-device-only", "-S", os.path.join(build.CSRC, "fo_gemm.hip"), "-o", str(out)]
+    cmd = [hipcc, *flags, "--cuda-device-only", "-S", os.path.join(build.CSRC, request.param), "-o", str(out)]
     subprocess.run(cmd, check=True, capture_output=True, timeout=600)
-    return out.read_text()
+    bodies, meta = _kernels(out.read_text())
+    assert len(bodies) == len(meta) == INSTANCES[request.param]
+    return bodies, meta
+
+
+def test_every_file_with_the_kernel_body_is_checked():
+    with_body = [f for f in build.HIP_SOURCES
+                 if '#include "fo_gemm_body.h"' in open(os.path.join(build.CSRC, f)).read()]
+    assert sorted(with_body) == sorted(INSTANCES)
 
 
 def _kernels(text):
-    """name -> (instruction lines, metadata dict) for every gemm_kernel instantiation."""
+    """name -> (instruction lines, metadata dict) for every instantiation of the kernel body."""
     bodies, name = {}, None
     for line in text.splitlines():
-        m = re.match(r"^(_ZN2fo11gemm_kernel\S+):", line)
+        m = re.match(r"^(_ZN2fo\d+gemm_(?:tall_|deep_)?kernel\S+):", line)
         if m:
             name = m.group(1)
             bodies[name] = []
@@ -49,7 +65,7 @@ def _kernels(text):
             if code:
                 bodies[name].append(code)
     meta = {}
-    for m in re.finditer(r"\.name:\s+(_ZN2fo11gemm_kernel\S+)\n(?:.*\n)*?\s+\.vgpr_count:\s+(\d+)\n\s+\.vgpr_spill_count:\s+(\d+)",
+    for m in re.finditer(r"\.name:\s+(_ZN2fo\d+gemm_(?:tall_|deep_)?kernel\S+)\n(?:.*\n)*?\s+\.vgpr_count:\s+(\d+)\n\s+\.vgpr_spill_count:\s+(\d+)",
                          text):
         meta[m.group(1)] = {"vgpr": int(m.group(2)), "spill": int(m.group(3))}
     return bodies, meta
@@ -59,8 +75,7 @@ AGPR = re.compile(r"\ba(\d+|\[\d+:\d+\])")
 
 
 def test_no_accumulator_access_close_behind_an_mfma(gemm_asm):
-    bodies, _ = _kernels(gemm_asm)
-    assert len(bodies) == 40            # 2 types x 2 macro tiles x (plain 2 + plain any-shape 2 + signal 3 + scatter 3)
+    bodies, _ = gemm_asm
     for name, ins in bodies.items():
         assert sum(i.startswith("v_mfma") for i in ins) > 0
         waited = None                   # wait states since the last MFMA of this straight-line stretch
@@ -80,7 +95,7 @@ def test_no_accumulator_access_close_behind_an_mfma(gemm_asm):
 
 def test_no_mfma_close_behind_an_accumulator_write(gemm_asm):
     """The other direction: the zeroed accumulators must have landed before the first MFMA adds to them."""
-    bodies, _ = _kernels(gemm_asm)
+    bodies, _ = gemm_asm
     for name, ins in bodies.items():
         since_write = None
         for i in ins:
@@ -98,8 +113,7 @@ def test_no_mfma_close_behind_an_accumulator_write(gemm_asm):
 
 
 def test_register_budget_and_no_spills(gemm_asm):
-    _, meta = _kernels(gemm_asm)
-    assert len(meta) == 40
+    _, meta = gemm_asm
     for name, m in meta.items():
         assert m["spill"] == 0, f"{name} spills {m['spill']} registers"
         # 512 registers per SIMD lane: what the GEMM leaves free is all the consumer's wavefronts
@@ -121,7 +135,7 @@ def test_no_vector_write_to_the_data_of_a_store_just_issued(gemm_asm):
     instructions apart, but the accumulator reads are assembly statements it cannot see into, and it
     may give them the registers of a store just issued (in an experimental kernel that drained
     accumulators between stores this corrupted single rows now and then)."""
-    bodies, _ = _kernels(gemm_asm)
+    bodies, _ = gemm_asm
     stores = 0
     for name, ins in bodies.items():
         for at, code in enumerate(ins):
