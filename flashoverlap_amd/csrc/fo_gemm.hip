@@ -70,12 +70,16 @@ struct Plan {
 };
 
 // Microseconds of a k-step of 64 of a macro tile, and of a round's start and end (launch, first panels,
-// stores).  Measured on shapes from 1024x1024x1024 to 8192x4096x7168, bf16 and fp16: with more than
+// stores).  Fitted on shapes from 1024x1024x1024 to 8192x4096x7168, bf16 and fp16: with more than
 // two thirds of the CUs at work all the time the chip comes to its power limit, and the k-steps get longer.
-// 2048x4096x7168 bf16: 114 us in 128x128 tiles, 101 in 256x128, 130 in 256x256; 4096x4096x4096: 116, 101, 90;
-// 1024x1024x1024: 9.2 in 64x64, 11.0 in 128x128.
+// Kernel alone, bf16, 2048x4096x7168: 101 us in 128x128 tiles, 92 in 256x128, 129 in 256x256; 4096x4096x4096: 112, 102, 90.
+// The 64x64 and 128x128 figures are older than the ring of four panels (fo_gemm_deep.hip), with which both take
+// less than this says: 1024x1024x1024 5.7 us in 64x64 tiles (here 8.4) and 8.8 in 128x128 (10.9), 1024x1024x4096
+// 15.2 (24.8) and 26.7 (32.9), 512x2048x2056 8.8 (17.5) and 14.7 (23.0).  The order of the two is as measured; against
+// a split over K, 64x64 tiles are charged too much (64x8192x3584: 15.5 us a call split, 13.1 unsplit).
 // straddle: rows that do not start on cache lines (K no multiple of 64) ask the L2 for every line twice
-// (2304x1664x5424: 77 us in 256x128 tiles, 55 in 128x128; 5504x1536 in 256x256: 123 with K 6912, 148 with 6944).
+// (2048x4096, K 7168 and 7176: 101 and 144 us in 128x128 tiles, 92 and 114 in 256x128, 129 and 133 in 256x256; a K that
+// is a multiple of 32 costs half of that: 5504x1536, K 6912, 6944, 6952, in 128x128 tiles 135, 157, 184, in 256x256 118, 118, 129).
 static double panel_us(Macro t, double busy, bool straddle) {   // busy: share of the CUs
     const double hot = busy <= 0.65 ? 0.0 : busy >= 1.0 ? 1.0 : (busy - 0.65) / 0.35;
     if (t.n == 256) return 1.08 + 0.28 * hot + 0.2 * straddle * (1.0 - hot);
@@ -88,8 +92,8 @@ static double round_us(Macro t) { return t.n == 256 ? 7.0 : t.m == 256 ? 5.0 : t
 // full; of a round that is at most half full the tiles can be split over K instead, if the parts
 // (which write MT * MT floats each, and are read again by a second launch) stay worth it.
 // Of the 128x128 tiles a CU holds two, and while one starts or stores the other multiplies: they take
-// k-steps only, however many come to a CU (9856x2048x1216, 4.8 to a CU: 46 us, 56 in 256x256 tiles;
-// 7168x1152x3520: 55, 64; 4608x4096x4096: 147, 119).  That also pairs them up as they come, so the parts of
+// k-steps only, however many come to a CU (9856x2048x1216, 4.8 to a CU: 45 us, 56 in 256x256 tiles;
+// 7168x1152x3520: 48, 64; 4608x4096x4096: 134, 155, or 118 with the last 32 of its 288 tiles split).  That also pairs them up as they come, so the parts of
 // an odd round out can share a CU with a whole tile while another two whole ones share theirs
 // (1407x3088x7360, 275 tiles of which 19 in 13 parts: 94 us, 68 in 256x256 tiles in 3): behind an odd number of
 // whole rounds nothing is split.
@@ -120,8 +124,8 @@ static Plan make_plan(int BM, int BN, int M, int N, int K, bool any_tile, bool m
             best = {t, total, 0, 1, panels, 0};
         }
         if (!may_split || t.m != t.n || rest * 2 > cus || (paired && whole % 2)) continue;
-        // A part written and read again, and what the second launch adds (16x4096x7168 in 2, 4, 8, 16
-        // parts: 31.0, 19.7, 15.0, 15.7 us, 54.7 unsplit; 2688x1920x4944 in 2: 63, 88 unsplit, 72 in 256x128 tiles;
+        // A part written and read again, and what the second launch adds (16x4096x7168, with the ring of two panels, in
+        // 2, 4, 8, 16 parts: 31.0, 19.7, 15.0, 15.7 us, 54.7 unsplit; 2688x1920x4944 in 2: 63, 88 unsplit, 72 in 256x128 tiles;
         // 8191x4097x7168 in 2, 4, 8: 376, 360, 362, 435 unsplit; 71x856x600 with its norm in 4: 13.4, 10.6 in 64x64 tiles).
         const double part_us = t.m == 256 ? 0.07 : 0.022, launch_us = 3.0;
         // the k-steps of a chip that is never idle, against some 24 more in which the parts pass through memory

@@ -42,7 +42,11 @@ struct GemmParams;
 int launch_gemm_deep(int macro, int mode, int dtype, bool edge, const GemmParams& p, const LaunchTimer& timer, hipStream_t stream);
 int launch_gemm_tall(int mode, int dtype, bool edge, const GemmParams& p, const LaunchTimer& timer, hipStream_t stream);
 
-// fo_skinny.hip: the plain GEMM for M <= kSkinnyRows
+// fo_skinny.hip: the plain GEMM for M <= kSkinnyRows.  bf16, us a call with 16 and 32 rows here, and with 33 and 64 in
+// macro tiles (split over K but for the last shape), weights from the memory-side cache: 4096x7168 10.6 11.0 | 15.0 15.5,
+// 8192x3584 10.6 11.5 | 14.8 15.3, 1024x8192 5.9 7.6 | 11.0 11.5, 3512x1408 4.9 4.8 | 6.6 6.5; weights from HBM: 13.0 16.1 |
+// 16.8 17.4, 12.9 16.2 | 16.6 17.0, 11.0 14.3 | 11.9 12.6, 5.7 5.6 | 8.1 9.3.  The kernel grows with the rows (A is copied
+// by every workgroup) and the macro tiles do not: at 32 rows the two meet where the weights come from HBM.
 constexpr int kSkinnyRows = 32;
 int launch_skinny(int dtype, int M, int N, int K, const void* A, const void* B, void* D, void* D2, const LaunchTimer& timer,
                   hipStream_t stream);

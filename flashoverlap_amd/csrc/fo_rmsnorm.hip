@@ -39,7 +39,7 @@ struct Vec8<__bf16> {
 };
 
 constexpr int kRowsPerBlock = 4;  // one wavefront per row; neighbouring rows read neighbouring tile segments
-constexpr int kWideThreads = 256;  // rows too long for one wavefront's registers: one workgroup per row
+constexpr int kWideThreads = 256;  // rows too long for a workgroup's registers: one workgroup and two passes per row
 
 // Ordinary loads, streaming (non-temporal) stores: the result is not read again here, and it
 // must not displace the GEMM operands held in the memory-side cache.  Measured on 8192 x 4096

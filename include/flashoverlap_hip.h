@@ -138,7 +138,10 @@ int fo_gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN,
  *             to overlap with (their groups complete with the GEMM itself) this
  *             replaces the counter, the wait and the copy that reads D again.
  *             deliver_from must be the first slot of a group.  The GEMM's stream
- *             orders a later kernel behind the delivery.
+ *             orders a later kernel behind the delivery.  It may not share memory
+ *             with A or B, nor with D (whose rows other workgroups write), except
+ *             that it may be D itself where every element stays in its place
+ *             (plain and signalling GEMM).
  *   nslices, slice_first, slice_count, slice_stride, group_start
  *             (scatter mode only) as in fo_wait_consume; group_start is a device
  *             array of G ints, the first slot of every group; group_table is
@@ -224,10 +227,12 @@ int fo_raster_hint(int algo, int M, int N, int* hint_host);
  *                  for the kernel that reads it next); 1: non-temporal
  *                  everywhere; 0: ordinary everywhere.
  *   "macro_tile"   the tile one workgroup computes.  0 (default): chosen per
- *                  shape (128x128, 256x128 or 256x256, whichever keeps the GPU
- *                  busier); 128, 256 or 256128 (256x128): forced, where the
- *                  layout tile divides it or the GEMM is the plain one.  The
- *                  issue order fo_raster_hint reports follows the setting. */
+ *                  shape (128x128, 256x128 or 256x256; 64x64 where nothing is
+ *                  signalled; a kernel of its own for a plain GEMM of up to 32
+ *                  rows), by an estimate of the time each takes; 128, 256 or
+ *                  256128 (256x128): forced, where the layout tile divides it or
+ *                  the GEMM is the plain one.  The issue order fo_raster_hint
+ *                  reports follows the setting. */
 int fo_tune(const char* key, int value);
 
 /* ---- counting / wait -------------------------------------------------- */
