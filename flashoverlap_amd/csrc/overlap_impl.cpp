@@ -204,42 +204,48 @@ void OverlapImpl::launch_gemm(fo_gemm_call& call, const at::Tensor& like) {
         return;
     }
     const int64_t bytes = (int64_t)4 << 20 << 2 * step;
-    const int device = like.device().index();
-    if (!workspace_ || workspace_device_ != device || workspace_stream_ != gemm_stream_) {
-        workspace_ = SplitWorkspace::of_stream(device, gemm_stream_);
-        workspace_device_ = device;
-        workspace_stream_ = gemm_stream_;
-    }
-    std::lock_guard<std::mutex> lock(workspace_->mutex);
-    if (!workspace_->buffer[step].defined()) make_workspace(like, step, bytes);
-    if (workspace_->buffer[step].defined()) {
-        call.workspace = workspace_->buffer[step].data_ptr();
+    const std::shared_ptr<SplitWorkspace> w = workspace_on(like.device().index());
+    std::lock_guard<std::mutex> lock(w->mutex);
+    if (!w->buffer[step].defined()) make_workspace(*w, like, step, bytes);
+    if (w->buffer[step].defined()) {
+        call.workspace = w->buffer[step].data_ptr();
         call.workspace_bytes = (size_t)bytes;
     }
     FO_CALL(fo_gemm_launch(&call, gemm_stream_));
 }
 
+// This object's hold on the workspace of its GEMM stream.  Threads may launch on one object at the same time.
+std::shared_ptr<SplitWorkspace> OverlapImpl::workspace_on(int device) {
+    std::lock_guard<std::mutex> lock(workspace_mutex_);
+    if (!workspace_ || workspace_device_ != device || workspace_stream_ != gemm_stream_) {
+        workspace_ = SplitWorkspace::of_stream(device, gemm_stream_);
+        workspace_device_ = device;
+        workspace_stream_ = gemm_stream_;
+    }
+    return workspace_;
+}
+
 // The workspace only makes a call faster.  Where the device has no memory for it the call runs without, and
 // so do the later ones of that size on this stream: an allocation that fails first gives all cached memory back
 // and waits for the device, which must not happen on every call, and a shape keeps its order of additions.
-void OverlapImpl::make_workspace(const at::Tensor& like, int step, int64_t bytes) {
-    if (workspace_->refused[step]) return;
+void OverlapImpl::make_workspace(SplitWorkspace& w, const at::Tensor& like, int step, int64_t bytes) {
+    if (w.refused[step]) return;
     // Taking memory can mean a hipMalloc, which would end a capture of the current stream (the GEMM's own is not
     // being captured, launch_gemm): the next call makes the buffer.
     int capturing = 0;
     FO_CALL(fo_stream_is_capturing((void*)c10::hip::getCurrentHIPStream().stream(), &capturing));
     if (capturing) return;
     // made and cleared on the GEMM's stream, whichever is current
-    c10::hip::HIPStreamGuard on(c10::hip::getStreamFromExternal((hipStream_t)gemm_stream_, (c10::DeviceIndex)workspace_device_));
+    c10::hip::HIPStreamGuard on(c10::hip::getStreamFromExternal((hipStream_t)gemm_stream_, like.device().index()));
     at::Tensor made;
     try {
         made = at::empty({bytes}, like.options().dtype(at::kByte));
     } catch (const c10::OutOfMemoryError&) {
-        workspace_->refused[step] = true;
+        w.refused[step] = true;
         return;
     }
     made.narrow(0, 0, FO_WORKSPACE_ZEROED).zero_();
-    workspace_->buffer[step] = std::move(made);
+    w.buffer[step] = std::move(made);
 }
 
 static bool shares_memory(const void* p, int64_t elems, const void* dst, int64_t dst_elems) {

@@ -110,6 +110,7 @@ class OverlapImpl : public torch::CustomClassHolder {
 
     at::Tensor staging_;
     at::Tensor expired_;          // one int32 on the device: expired waits of this object's calls
+    std::mutex workspace_mutex_;
     std::shared_ptr<SplitWorkspace> workspace_;
     int workspace_device_ = -1;
     void* workspace_stream_ = nullptr;
@@ -131,7 +132,8 @@ class OverlapImpl : public torch::CustomClassHolder {
                         bool in_order);
     void bulk_consume(const void* src, void* dst, size_t bytes);
     void launch_gemm(fo_gemm_call& call, const at::Tensor& like);
-    void make_workspace(const at::Tensor& like, int step, int64_t bytes);
+    std::shared_ptr<SplitWorkspace> workspace_on(int device);
+    void make_workspace(SplitWorkspace& w, const at::Tensor& like, int step, int64_t bytes);
     int* expired_word(const at::Tensor& like);
     void refuse_checked_capture(const char* who);
     void prepare_call(const at::Tensor& MM, const char* who);

@@ -78,3 +78,38 @@ def test_first_call_while_another_stream_is_captured(call):
         graph.replay()
         assert call()
     assert (x == 2).all()
+
+
+def test_threads_on_one_object(dev):
+    """Plain calls of several threads on one object, the first ones at the same time, with workspaces of two sizes."""
+    import threading
+    flashoverlap_amd.load()
+    gen = torch.Generator().manual_seed(23)
+    shapes = [(128, 4096, 7168), (128, 1024, 4096)]
+    work = []
+    for m, n, k in shapes:
+        A, B = (torch.randint(-2, 3, (r, k), generator=gen).to(torch.bfloat16).to(dev) for r in (m, n))
+        work.append((A, B, (A.float() @ B.float().t()).to(torch.bfloat16)))
+    outs = [[torch.zeros(m, n, dtype=torch.bfloat16, device=dev) for m, n, _ in shapes] for _ in range(8)]
+    o = torch.classes.flashoverlap_class.OverlapImpl()
+    o.mutlass_init()
+    torch.cuda.synchronize()
+    start, failed = threading.Barrier(len(outs)), []
+
+    def worker(mine, first):
+        try:
+            start.wait()
+            for i in range(20):
+                s = (first + i) % 2
+                o.mutlass_gemm(work[s][0], work[s][1], mine[s], 1)
+        except Exception as e:
+            failed.append(e)
+
+    threads = [threading.Thread(target=worker, args=(mine, t % 2)) for t, mine in enumerate(outs)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not failed
+    assert all(torch.equal(c, w[2]) for mine in outs for c, w in zip(mine, work))
