@@ -164,9 +164,20 @@ static int plan_for(const fo_gemm_call& c, bool workspace, Plan* plan) {
 // A few rows of A: a kernel of its own, unless a macro tile is asked for.
 static bool is_skinny(const fo_gemm_call& c) { return c.mode == kPlain && c.M <= kSkinnyRows && !knob(knobs().macro_tile); }
 
+// Sizes with which the kernels' offsets, and make_plan's tile counts, stay inside their types.
+static int check_limits(int M, int N, int K) {
+    if ((long long)M * N >= (1LL << 31)) return fail(FO_ERR_LIMIT, "fo_gemm: M*N=%lld needs 64-bit tile offsets", (long long)M * N);
+    // (the rows a macro tile may reach beyond an operand must still have 32-bit byte offsets)
+    if (((long long)M + 256) * K >= (1LL << 31) || ((long long)N + 256) * K >= (1LL << 31))
+        return fail(FO_ERR_LIMIT, "fo_gemm: an operand of %lld elements exceeds the 4 GiB a buffer descriptor addresses",
+                    (long long)(M > N ? M : N) * K);
+    return FO_OK;
+}
+
 int gemm_workspace(const fo_gemm_call& c, size_t* bytes) {
     *bytes = 0;
     if (c.M <= 0 || c.N <= 0 || c.K <= 0) return fail(FO_ERR_SHAPE, "fo_gemm_workspace: empty problem %dx%dx%d", c.M, c.N, c.K);
+    if (int e = check_limits(c.M, c.N, c.K)) return e;
     if (is_skinny(c)) return FO_OK;
     Plan plan;
     if (int e = plan_for(c, true, &plan)) return e;
@@ -202,11 +213,7 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream) {
     if (!any_shape && (M % BM || N % BN))
         return fail(FO_ERR_SHAPE, "fo_gemm_signal: M=%d N=%d not multiples of the %dx%d tile", M, N, BM, BN);
     if (K % 8) return fail(FO_ERR_SHAPE, "fo_gemm: K=%d not a multiple of 8 (operand rows must be 16-byte aligned)", K);
-    if ((long long)M * N >= (1LL << 31)) return fail(FO_ERR_LIMIT, "fo_gemm: M*N=%lld needs 64-bit tile offsets", (long long)M * N);
-    // (the rows a macro tile may reach beyond an operand must still have 32-bit byte offsets)
-    if (((long long)M + 256) * K >= (1LL << 31) || ((long long)N + 256) * K >= (1LL << 31))
-        return fail(FO_ERR_LIMIT, "fo_gemm: an operand of %lld elements exceeds the 4 GiB a buffer descriptor addresses",
-                    (long long)(M > N ? M : N) * K);
+    if (int e = check_limits(M, N, K)) return e;
     if (K % kBK && ((long long)M * K >= (1LL << 30) || (long long)N * K >= (1LL << 30)))
         return fail(FO_ERR_LIMIT, "fo_gemm: K=%d is not a multiple of %d and an operand exceeds the 2 GiB this case addresses", K, kBK);
     if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)D) & 15) return fail(FO_ERR_ARG, "fo_gemm: operands must be 16-byte aligned");

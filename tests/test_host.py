@@ -212,3 +212,12 @@ def test_oracle_is_not_reachable_from_the_product():
             if f.endswith((".py", ".cpp", ".h", ".hip")):
                 src = open(os.path.join(dirpath, f)).read()
                 assert "oracle" not in src, f"{f} mentions the oracle"
+
+
+@pytest.mark.parametrize("M,N,K", [(1 << 24, 1 << 24, 64), (46341, 46341, 8), ((1 << 31) - 1, 1, 8), (1, (1 << 31) - 1, 8)])
+def test_workspace_refuses_what_the_gemm_refuses(fo_lib, M, N, K):
+    """Sizes whose tile counts overflow (16777216 squared: to no tile at all) are refused before a plan is made."""
+    call = capi.GemmCall(mode=0, dtype=capi.FO_BF16, algo=1, M=M, N=N, K=K)
+    need = ctypes.c_size_t(7)
+    assert fo_lib.fo_gemm_workspace(ctypes.byref(call), ctypes.byref(need)) == capi.FO_ERR_LIMIT
+    assert need.value == 0
