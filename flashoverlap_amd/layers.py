@@ -93,13 +93,13 @@ class OverlapRowParallelLayer(nn.Module):
     def _bind(self):
         # looking a method up on a script object costs 0.6 us, of a call that takes 8
         o = self.overlap_class
-        self._bound = (o, o.allreduce_linear if self.comm_op == "all_reduce" else o.reducescatter_linear)
+        self._bound = (o, o.allreduce_linear, o.reducescatter_linear)
 
     def forward(self, x):
         if self._bound[0] is not self.overlap_class:
             self._bind()
+        _, allreduce, reducescatter = self._bound
         if self.comm_op == "all_reduce":
-            return self._bound[1](x, self.weight, self.counter, self.reorder_array, self.cseg_cpu, self.cseg_gpu,
-                                  self.algo)
-        return self._bound[1](x, self.weight, self.counter, self.reorder_array, self.row_array, self.cseg_cpu,
-                              self.cseg_gpu, self.algo)
+            return allreduce(x, self.weight, self.counter, self.reorder_array, self.cseg_cpu, self.cseg_gpu, self.algo)
+        return reducescatter(x, self.weight, self.counter, self.reorder_array, self.row_array, self.cseg_cpu,
+                             self.cseg_gpu, self.algo)
