@@ -66,8 +66,6 @@ static __device__ __forceinline__ float acc_write(float v) {
 // More wait states than the longest MFMA needs before its result can be read.
 static __device__ __forceinline__ void settle_mfma() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
-constexpr int kMaxHereSplits = 6;   // parts of a 64x64 tile, added up in the GEMM
-constexpr int kBK = 64;             // k-elements per LDS buffer
 constexpr int kRowBytes = kBK * 2;  // one panel row in LDS: 128 bytes = 8 chunks of 16
 
 enum { kPlain = 0, kSignal = 1, kScatter = 2 };

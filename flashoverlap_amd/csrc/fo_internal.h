@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "../../include/flashoverlap_hip.h"
+#include "fo_plan.h"
 
 namespace fo {
 
@@ -31,7 +32,6 @@ struct LaunchTimer {
 extern thread_local LaunchTimer t_launch_timer;
 
 // fo_gemm.hip
-constexpr size_t kMaxWorkspace = (size_t)64 << 20;   // bytes of the parts of split tiles, at most
 int launch_gemm(const fo_gemm_call& c, hipStream_t stream, bool keep_d = true, fo_workspace_fn ask = nullptr, void* context = nullptr);
 int gemm_workspace(const fo_gemm_call& c, size_t* bytes);
 int gemm_rounds(int algo, int M, int N, int* per_round, int* last_first);
@@ -48,7 +48,6 @@ int launch_gemm_tall(int mode, int dtype, bool edge, const GemmParams& p, const 
 // 8192x3584 10.6 11.5 | 14.8 15.3, 1024x8192 5.9 7.6 | 11.0 11.5, 3512x1408 4.9 4.8 | 6.6 6.5; weights from HBM: 13.0 16.1 |
 // 16.8 17.4, 12.9 16.2 | 16.6 17.0, 11.0 14.3 | 11.9 12.6, 5.7 5.6 | 8.1 9.3.  The kernel grows with the rows (A is copied
 // by every workgroup) and the macro tiles do not: at 32 rows the two meet where the weights come from HBM.
-constexpr int kSkinnyRows = 32;
 int launch_skinny(int dtype, int M, int N, int K, const void* A, const void* B, void* D, void* D2, int ld, bool across,
                   const LaunchTimer& timer, hipStream_t stream);   // across: D is stored transposed
 

@@ -1,0 +1,128 @@
+// Which macro tile computes a shape, and which tiles are split over K: the estimate and the choice, on the host alone.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+
+#include "../../include/flashoverlap_hip.h"
+
+namespace fo {
+
+constexpr int kBK = 64;             // k-elements per LDS buffer
+constexpr int kMaxHereSplits = 6;   // parts of a 64x64 tile, added up in the GEMM
+constexpr size_t kMaxWorkspace = (size_t)64 << 20;   // bytes of the parts of split tiles, at most
+constexpr int kSkinnyRows = 32;     // rows that the skinny kernel takes (fo_internal.h has its times)
+
+struct Macro {
+    int m, n;
+};
+
+// How a shape is computed: the macro tile, and which macro tiles are split over K.
+struct Plan {
+    Macro macro;
+    int from, tiles, splits, panels;   // the last `tiles` macro tiles, in `splits` parts of `panels` panels; 0: none
+    size_t bytes;                      // workspace of the parts
+    double us;                         // estimated
+    int strip_m, strip_n;              // the last rows or columns of D that a skinny GEMM computes (at most one of the two)
+};
+
+// Estimated microseconds of a GEMM in macro tiles of one kind.  Fitted on 1449 plain shapes of 33 to 8192 rows, 512 to 8192
+// columns and K 512 to 8192, fp16 and bf16, each timed in every tile and in most splits (some 11000 kernels): half of the
+// estimates are within 5 % of the time, and the plan taken by them is on average 0.7 % slower than the fastest one
+// measured (the estimate before, which knew the 64x64 and the lone 128x128 tiles only as they were without the
+// ring of four panels: 7 %; 512x2048x2056 18.4 us, now 12.2; 1024x1024x4096 20.3, 15.5; 4945x4576x1408 69.7, 59.8).
+// With more than half of the CUs at work all the time the k-steps of the larger tiles get longer; at the chip's power limit, in
+// several full rounds, by more than is said here, but no other tile comes near 256x256 there.
+struct Shape {
+    int panels, cus;
+    double straddle;     // rows that do not start on cache lines ask the L2 for a line twice: all of them, or half where K is a multiple of 32
+    double operands_us;  // A and B at 8.4 TB/s
+    double out_mb;       // D, in 10^6 bytes
+};
+// 64x64 in `parts` parts each.  One to a CU, or two, each of which then hides the other's latency.  The parts are added up
+// by the workgroup that finishes last, the more of them the longer (fo_gemm_body.h).
+inline double us_64(const Shape& s, int total, int parts, int per) {
+    const double load = (double)total * parts / s.cus;
+    const double step = load <= 1.0 ? 0.172 + ((parts == 1 ? 0.035 : 0.0) + 0.06 * load) * s.straddle + 0.023 * load : 0.375 + 0.165 * s.straddle;
+    return 2.9 + std::max(per * step, s.operands_us) + (parts > 1 ? 2.0 + 0.35 * parts : 0.0);
+}
+// 128x128, `rest` of them in `parts` parts behind `whole` times as many whole tiles as CUs.  While they fit one to a CU they
+// have the ring of four panels; of more than that a CU holds two, and while one starts or stores the other multiplies: they take
+// k-steps only.  That also pairs them up as they come: parts behind an odd number of whole tiles to a CU share
+// theirs with a whole one, behind an even number with each other.  The parts are written and read again, by a second launch.
+inline double us_128(const Shape& s, int whole, int rest, int parts, int per) {
+    const double load = (double)rest * parts / s.cus, add = parts > 1 ? 0.8 + 0.022 * rest * parts : 0.0;
+    if (whole == 0) return 5.5 + std::max(per * (0.375 + 0.125 * s.straddle), s.operands_us) + add;
+    const double last = parts > 1 && whole % 2 ? 1.0 : 0.5 * (1.0 + load);
+    return 2.0 + (0.471 + 0.159 * s.straddle) * (s.panels * whole + per * last) + add + 0.23 * s.out_mb;
+}
+// The larger tiles have a CU to themselves, and a round of them takes as long if it is not full.  (256x128 with its three panels
+// ahead: fitted on 240 shapes of 60 to 1100 such tiles, operands from HBM; the plans are 0.7 % slower than the fastest measured.)
+inline double hot(double busy) { return std::min(1.0, std::max(0.0, 2.0 * busy - 1.0)); }
+inline double us_256(const Shape& s, int whole, int rest, int parts, int per) {
+    auto round_us = [&](double busy, int panels) { return 7.8 + panels * (1.089 + 0.101 * hot(busy) + 0.09 * s.straddle * (1.0 - hot(busy))); };
+    const double load = (double)rest * parts / s.cus;
+    if (parts > 1) return whole * round_us(1.0, s.panels) + round_us(load, per) + 0.063 * rest * parts + 0.164 * s.out_mb;
+    return (whole + 1) * round_us((whole + load) / (whole + 1), s.panels) + 0.164 * s.out_mb;
+}
+inline double us_256x128(const Shape& s, int whole, int rest) {
+    const double busy = (whole + (double)rest / s.cus) / (whole + 1);
+    return (whole + 1) * (4.8 + s.panels * (0.675 + std::max(0.136 * hot(busy), 0.1 * s.straddle))) + 0.1 * s.out_mb;
+}
+
+// The plan whose estimated time is the smallest.  Of a round that is at most half full the 128x128 and 256x256 tiles can be
+// split over K; 64x64 tiles are all split or none, while they come to two workgroups a CU at most.
+inline Plan make_plan(int BM, int BN, int M, int N, int K, bool any_tile, bool may_split, bool all_tiles, Macro forced, int cus) {
+    const Shape s{(K + kBK - 1) / kBK, cus, K % kBK == 0 ? 0.0 : K % 32 == 0 ? 0.5 : 1.0, ((double)M + N) * K * 2 / 8.4e6, (double)M * N * 2e-6};
+    Plan best{};
+    double best_us = 1e30;
+    for (const Macro t : {Macro{256, 256}, Macro{256, 128}, Macro{128, 128}, Macro{64, 64}}) {
+        if (forced.m ? t.m != forced.m || t.n != forced.n : !any_tile && (t.m % BM || t.n % BN)) continue;
+        if ((t.m != t.n || t.m == 64) && !all_tiles) continue;
+        const int total = ((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n);
+        if (t.m == 64 && total > 2 * cus) continue;
+        const int whole = t.m == 64 ? 0 : (total - 1) / cus, rest = total - whole * cus;
+        const int most = !may_split || t.m != t.n ? 1 : t.m == 64 ? kMaxHereSplits : t.m == 128 ? 10 : 16;
+        for (int n = 1; n <= most; ++n) {
+            const int per = (s.panels + n - 1) / n, parts = (s.panels + per - 1) / per;
+            if (n > 1 && (per < (t.m == 64 ? 3 : 4) || rest * n > (t.m == 64 ? 2 * cus : cus))) break;
+            if (parts != n) continue;   // (the same as with fewer)
+            const size_t bytes = n == 1 ? 0 : FO_WORKSPACE_ZEROED + (size_t)rest * n * t.m * t.n * sizeof(float);
+            if (bytes > FO_WORKSPACE_ZEROED + kMaxWorkspace) break;
+            const double us = t.m == 64 ? us_64(s, total, n, per) : t.m == 128 ? us_128(s, whole, rest, n, per)
+                              : t.n == 256 ? us_256(s, whole, rest, n, per) : us_256x128(s, whole, rest);
+            if (us >= best_us) continue;
+            best_us = us;
+            best = n == 1 ? Plan{t, total, 0, 1, s.panels, 0, us} : Plan{t, total - rest, rest, n, per, bytes, us};
+        }
+    }
+    return best;
+}
+
+// A plain GEMM of which a few rows or columns lie behind the last whole multiple of 128: as macro tiles they are a row or column
+// of tiles that multiplies zeros, often a round of its own.  The skinny kernel (with the operands exchanged, for columns) reads the
+// other operand once more, at HBM's rate if it is large, and starts like any launch.  It runs in front of the tiles, which then
+// find that operand in the memory-side cache.  Taken where that is estimated to be shorter by 5 %, or by 8 us (the rounds that both have
+// in common err alike), and where the rows of the operands start on cache lines: the estimates of others err by up to a third, which
+// only columns, whose tiles also store ragged rows, make up for.  On 80 shapes for which it is estimated to be so, time / time in
+// tiles: strips of columns 0.92 (1.01 at worst), with K an odd multiple of 32 0.88 (1.02), of rows 0.96 (1.02) and 0.99 (1.24, not taken).
+// Plain GEMM, its bulk copy and the norm, us, in tiles / so: 8191x4097x7168 bf16 353 / 339, 8192x4104x1024 106 / 93,
+// 2080x4112x4096 fp16 85 / 78.
+inline double us_strip(int other_rows, int K) { return 4.5 + (double)other_rows * K * 2 / 5.2e6; }
+inline void consider_strip(Plan* plan, int BM, int BN, int M, int N, int K, bool may_split, bool all_tiles, int cus) {
+    const int rest_m = M % 128, rest_n = N % 128;
+    auto consider = [&](int sm, int sn) {
+        const double strip = us_strip(sm ? N : M, K);
+        if (M - sm <= 0 || N - sn <= 0 || strip >= plan->us) return;
+        Plan other = make_plan(BM, BN, M - sm, N - sn, K, true, may_split, all_tiles, Macro{0, 0}, cus);
+        if (!other.macro.m || other.us + strip >= plan->us - std::min(0.05 * plan->us, 8.0)) return;
+        *plan = other;
+        plan->us = other.us + strip;
+        plan->strip_m = sm;
+        plan->strip_n = sn;
+    };
+    if (rest_m && rest_m <= kSkinnyRows && K % 64 == 0) consider(rest_m, 0);
+    if (rest_n && rest_n <= kSkinnyRows && K % 32 == 0) consider(0, rest_n);
+}
+
+}  // namespace fo
