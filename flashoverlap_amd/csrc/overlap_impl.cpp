@@ -449,6 +449,7 @@ void OverlapImpl::overlapped_call(fo_gemm_call& call, const fo_host::SignalShape
     const int waited = can_deliver(call, dst, kept) ? groups_to_wait_for(call, cseg_cpu.data_ptr<int>(), call.nslices,
                                                                          &call.deliver_from, &per_round)
                                                     : g.G;
+    released_ = waited;
     if (waited || call.mode == FO_GEMM_SCATTER) {   // (an all-reduce that signals nothing looks no group up)
         call.group_table = group_table_for(cseg_cpu, cseg_gpu, g.T);
         call.group_start = group_start_.data_ptr<int>();

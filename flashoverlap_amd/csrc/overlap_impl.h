@@ -11,6 +11,7 @@
 #include <ATen/ATen.h>
 #include <torch/custom_class.h>
 
+#include <atomic>
 #include <cstdint>
 #include <memory>
 #include <mutex>
@@ -83,6 +84,9 @@ class OverlapImpl : public torch::CustomClassHolder {
     // wait and one copy launch), 1 = one (wait, consume) launch pair per group like the
     // reference's host loop, 2 = one persistent wait+consume kernel.
     void SetConsumerMode(int64_t mode);
+    // Groups of the last overlapped call that were released through their counters; the others (in the automatic mode,
+    // all of them up to that K) were delivered by the GEMM, and how they were cut makes no difference to its time.
+    int64_t ReleasedGroups() const { return released_; }
     // Workgroups of the persistent consumer (default and maximum: one per CU).
     void SetConsumerBlocks(int64_t blocks);
     // The waits on the group counters are bounded (the reference's spin forever,
@@ -107,6 +111,7 @@ class OverlapImpl : public torch::CustomClassHolder {
     int64_t consumer_mode_ = 0;
     int64_t consumer_blocks_ = 0;   // 0: not chosen yet (one per CU at first use)
     bool check_timeouts_ = false;
+    std::atomic<int64_t> released_{0};
 
     at::Tensor staging_;
     at::Tensor expired_;          // one int32 on the device: expired waits of this object's calls

@@ -55,6 +55,7 @@ TORCH_LIBRARY(flashoverlap_class, m) {
         // additions
         .def("staging", &OverlapImpl::Staging)
         .def("set_consumer_mode", &OverlapImpl::SetConsumerMode)
+        .def("released_groups", &OverlapImpl::ReleasedGroups)
         .def("set_staging", &OverlapImpl::SetStaging)
         .def("allreduce_linear", &OverlapImpl::AllReduceLinear)
         .def("reducescatter_linear", &OverlapImpl::ReduceScatterLinear)

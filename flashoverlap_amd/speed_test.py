@@ -119,9 +119,11 @@ def perf_baseline(M, N, K, comm_op, world_size=1, dtype=torch.float16, device="c
 
 
 def perf_running(M, N, K, BM, BN, Algo, cSeg, hint, comm_op, world_size=1, dtype=torch.float16, device="cuda",
-                 keep=None, **kw):
+                 keep=None, release=False, **kw):
     """test/test.py:120-207.  `keep`, if a dict, receives the operands and outputs of the last
-    iteration (for checking them)."""
+    iteration (for checking them).  With `release`, a call whose groups the automatic mode would all have
+    delivered by the GEMM is timed in the mode that releases each through its counter: only there does
+    the time depend on cSeg."""
     cSeg_CPU = torch.tensor(cSeg, dtype=torch.int32)
     cSeg_GPU = cSeg_CPU.to(device)
     TM, TN = tiling.div_up(M, BM), tiling.div_up(N, BN)
@@ -144,6 +146,10 @@ def perf_running(M, N, K, BM, BN, Algo, cSeg, hint, comm_op, world_size=1, dtype
         fn = lambda: o.gemm_allreduce_overlap(A, B, C, counters, RA, 1, cSeg_CPU, cSeg_GPU, Algo, False)
     else:
         fn = lambda: o.gemm_reducescatter_overlap(A, B, C, D, counters, RA, RE, 1, cSeg_CPU, cSeg_GPU, Algo, False)
+    if release and len(cSeg) > 1:
+        fn()
+        if o.released_groups() == 0:
+            o.set_consumer_mode(1)
     dur = _timed(fn, **kw)
     if keep is not None:
         # host time to enqueue one call (nothing is waited for): what the torch-API path costs the CPU

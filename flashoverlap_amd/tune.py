@@ -25,7 +25,9 @@ the transfer, so the model does not rescale the GEMM time as the reference does
 for its two reserved processors.  Beyond the reference: the predictive search
 also times its few best candidates and keeps the one that measured best, and
 both searches time the single-group call so that the file never holds a
-partition that lost against not overlapping at all.
+partition that lost against not overlapping at all.  They time partitions whose
+groups are released as they complete: where OverlapImpl's automatic mode has the
+GEMM deliver all groups, in consumer mode 1, for which the `cSeg` found is meant.
 """
 from __future__ import annotations
 
@@ -198,7 +200,8 @@ def _pick_candidate(M, N, K, BM_list, BN_list, dur_list, Algo_list, wave_units, 
 
 
 def _time(M, N, K, BM, BN, Algo, cseg, hint, comm_op, world_size, dtype, **kw) -> float:
-    return speed_test.perf_running(M, N, K, BM, BN, Algo, cseg, hint, comm_op, world_size, dtype, "cuda", **kw)
+    return speed_test.perf_running(M, N, K, BM, BN, Algo, cseg, hint, comm_op, world_size, dtype, "cuda",
+                                   release=True, **kw)
 
 
 def exhaustive_search(M: int, N: int, K: int, comm_op: str = "all_reduce", world_size: int = 1, dtype=torch.float16,

@@ -91,3 +91,26 @@ def test_bandwidth_curve_then_predictive_search(dev, tmp_path):
     assert "Bandwidth curve captured." in said and any("predicted" in s and "measured" in s for s in said)
     assert got["ms"] > 0
     _check_overlapped_call(cfg, "reduce_scatter", ws)
+
+
+@pytest.mark.parametrize("comm_op,ws", [("all_reduce", 1), ("reduce_scatter", 4)])
+def test_searches_time_groups_that_are_released(dev, monkeypatch, comm_op, ws):
+    """A partition is timed with its groups released through their counters, also where the automatic mode, in which
+    an object starts, has the GEMM deliver them all."""
+    flashoverlap_amd.load()
+    made, timed = [], []
+    make, measure = speed_test._overlap_object, speed_test._timed
+    monkeypatch.setattr(speed_test, "_overlap_object", lambda *a: made.append(make(*a)) or made[-1])
+
+    def note(fn, **kw):
+        t = measure(fn, **kw)
+        timed.append(made[-1].released_groups())
+        return t
+
+    monkeypatch.setattr(speed_test, "_timed", note)
+    hint = tiling.raster_hint(M, N, 1)
+    for cseg in ([1024, 1024], [512, 512, 1024]):
+        tune._time(M, N, K, 128, 128, 1, cseg, hint, comm_op, ws, torch.float16, **FAST)
+        assert timed[-1] == len(cseg)
+        speed_test.perf_running(M, N, K, 128, 128, 1, cseg, hint, comm_op, ws, torch.float16, "cuda", **FAST)
+        assert timed[-1] == 0          # delivered, as a user's call is
