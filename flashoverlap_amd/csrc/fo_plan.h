@@ -26,11 +26,14 @@ struct Plan {
     int strip_m, strip_n;              // the last rows or columns of D that a skinny GEMM computes (at most one of the two)
 };
 
-// Estimated microseconds of a GEMM in macro tiles of one kind.  Fitted on 1449 plain shapes of 33 to 8192 rows, 512 to 8192
-// columns and K 512 to 8192, fp16 and bf16, each timed in every tile and in most splits (some 11000 kernels): half of the
-// estimates are within 5 % of the time, and the plan taken by them is on average 0.7 % slower than the fastest one
-// measured (the estimate before, which knew the 64x64 and the lone 128x128 tiles only as they were without the
-// ring of four panels: 7 %; 512x2048x2056 18.4 us, now 12.2; 1024x1024x4096 20.3, 15.5; 4945x4576x1408 69.7, 59.8).
+// Estimated microseconds of a GEMM in macro tiles of one kind.  Fitted on 1138 shapes of 33 to 16384 rows, 512 to 8192
+// columns and K 512 to 8192, fp16 and bf16, each timed in the tiles and splits that come near (some 6000 kernels), with operands
+// from HBM and with operands that the memory-side cache holds, so that the plans taken are short in both and few are much longer
+// than the fastest one measured.  On 334 other shapes the plan taken is on average 1.3 % (HBM) and 0.9 % (cached) slower than
+// the fastest, 23 and 17 % at worst; with the constants before, which were fitted to the times, 1.6 and 0.8 %, 37 and 17 % at
+// worst.  Those priced parts of 256x256 tiles too low, and lone 128x128 tiles with operands from HBM.  us, HBM and cached, before | now:
+// 2041x4096x7168 fp16 113.0 111.2 | 104.2 101.5, 77x7680x7936 bf16 33.9 25.7 | 29.8 25.0, 4608x1152x4544 fp16 68.2 53.6 | 61.6 50.0,
+// 6683x1336x1600 bf16 51.6 38.9 | 38.6 37.0, 640x3840x7872 fp16 74.4 51.0 | 52.1 52.4.
 // With more than half of the CUs at work all the time the k-steps of the larger tiles get longer; at the chip's power limit, in
 // several full rounds, by more than is said here, but no other tile comes near 256x256 there.
 struct Shape {
@@ -51,23 +54,22 @@ inline double us_64(const Shape& s, int total, int parts, int per) {
 // k-steps only.  That also pairs them up as they come: parts behind an odd number of whole tiles to a CU share
 // theirs with a whole one, behind an even number with each other.  The parts are written and read again, by a second launch.
 inline double us_128(const Shape& s, int whole, int rest, int parts, int per) {
-    const double load = (double)rest * parts / s.cus, add = parts > 1 ? 0.8 + 0.022 * rest * parts : 0.0;
-    if (whole == 0) return 5.5 + std::max(per * (0.375 + 0.125 * s.straddle), s.operands_us) + add;
+    const double load = (double)rest * parts / s.cus, add = parts > 1 ? 0.86 + 0.023 * rest * parts : 0.0;
+    if (whole == 0) return 4.06 + std::max(per * (0.458 + 0.155 * s.straddle), s.operands_us) + add;
     const double last = parts > 1 && whole % 2 ? 1.0 : 0.5 * (1.0 + load);
-    return 2.0 + (0.471 + 0.159 * s.straddle) * (s.panels * whole + per * last) + add + 0.23 * s.out_mb;
+    return 2.12 + (0.497 + 0.168 * s.straddle) * (s.panels * whole + per * last) + add + 0.144 * s.out_mb;
 }
-// The larger tiles have a CU to themselves, and a round of them takes as long if it is not full.  (256x128 with its three panels
-// ahead: fitted on 240 shapes of 60 to 1100 such tiles, operands from HBM; the plans are 0.7 % slower than the fastest measured.)
+// The larger tiles have a CU to themselves, and a round of them takes as long if it is not full.
 inline double hot(double busy) { return std::min(1.0, std::max(0.0, 2.0 * busy - 1.0)); }
 inline double us_256(const Shape& s, int whole, int rest, int parts, int per) {
-    auto round_us = [&](double busy, int panels) { return 7.8 + panels * (1.089 + 0.101 * hot(busy) + 0.09 * s.straddle * (1.0 - hot(busy))); };
+    auto round_us = [&](double busy, int panels) { return 8.63 + panels * (1.107 + 0.145 * hot(busy) + 0.087 * s.straddle * (1.0 - hot(busy))); };
     const double load = (double)rest * parts / s.cus;
-    if (parts > 1) return whole * round_us(1.0, s.panels) + round_us(load, per) + 0.063 * rest * parts + 0.164 * s.out_mb;
-    return (whole + 1) * round_us((whole + load) / (whole + 1), s.panels) + 0.164 * s.out_mb;
+    if (parts > 1) return whole * round_us(1.0, s.panels) + round_us(load, per) + 0.072 * rest * parts;
+    return (whole + 1) * round_us((whole + load) / (whole + 1), s.panels);
 }
 inline double us_256x128(const Shape& s, int whole, int rest) {
     const double busy = (whole + (double)rest / s.cus) / (whole + 1);
-    return (whole + 1) * (4.8 + s.panels * (0.675 + std::max(0.136 * hot(busy), 0.1 * s.straddle))) + 0.1 * s.out_mb;
+    return (whole + 1) * (4.98 + s.panels * (0.662 + std::max(0.043 * hot(busy), 0.219 * s.straddle))) + 0.125 * s.out_mb;
 }
 
 // The plan whose estimated time is the smallest.  Of a round that is at most half full the 128x128 and 256x256 tiles can be
