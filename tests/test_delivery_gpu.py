@@ -1,7 +1,7 @@
-"""The GEMM's epilogue as the last groups' consumer: a call in the automatic mode, which delivers the
-groups that complete with the GEMM, against the same call with every group waited for and copied
-(consumer mode 1).  The same tiles take another way to the same place, so every buffer has to be
-bit-identical, and the counters have to end at zero either way."""
+"""The GEMM's epilogue as the groups' consumer: a call in the automatic mode, which delivers every group up to
+K = 8192 and above it those that complete with the GEMM, against the same call with every group waited for and
+copied (consumer mode 1).  The same tiles take another way to the same place, so every buffer has to be
+bit-identical, and the counters have to end at zero either way.  released_groups() says which way they took."""
 import ctypes as C
 
 import pytest
@@ -30,8 +30,20 @@ def _object(api, mode, rank=0, size=1):
 
 
 def _inputs(dev, dt, M, N, K):
-    g = torch.Generator().manual_seed(M + 3 * N + 7 * K)
-    return tuple((torch.randn(r, K, generator=g) / K ** 0.25).to(dt).to(dev) for r in (M, N))
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 7 * K)
+    return tuple((torch.randn(r, K, generator=g, device=dev) / K ** 0.25).to(dt) for r in (M, N))
+
+
+def _released(mode, M, N, K, algo, cseg):
+    """The groups of a call that go through their counters: in the automatic mode none up to K = 8192, and above
+    it those with a tile in front of the last round of workgroups, but for the last one."""
+    if mode:
+        return len(cseg)
+    if K <= 8192:
+        return 0
+    per, late = C.c_int(), C.c_int()
+    capi.check(capi.lib().fo_gemm_rounds(algo, M, N, C.byref(per), C.byref(late)))
+    return sum(sum(cseg[:g]) < late.value for g in range(len(cseg) - 1))
 
 
 @pytest.mark.parametrize("M,N,K,algo,cseg", [
@@ -40,6 +52,7 @@ def _inputs(dev, dt, M, N, K):
     (512, 768, 128, 2, [5, 7]),                  # 128x256 layout tiles: half macro tiles and whole ones
     (768, 384, 72, 4, [1] * 9),                  # 256x128
     (8192, 2304, 64, 1, [600, 424, 64, 64]),     # 288 macro tiles of 256: a first round and 32 tiles of a second
+    (8192, 2304, 8200, 1, [600, 424, 64, 64]),   # the same with the groups of the first round released
 ])
 @pytest.mark.parametrize("ws,stacked", [(1, False), (4, False), (8, True)])
 def test_delivered_groups_equal_copied_groups(api, dev, M, N, K, algo, cseg, ws, stacked):
@@ -66,6 +79,7 @@ def test_delivered_groups_equal_copied_groups(api, dev, M, N, K, algo, cseg, ws,
                 o.gemm_allreduce_overlap(A, B, c, mm, RA, 1, cs, cs.to(dev), algo, False)
         torch.cuda.synchronize()
         assert o.wait_timeouts(True) == 0 and not mm.any()
+        assert o.released_groups() == _released(mode, M, N, K, algo, cseg)
         got.append((c, d))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
@@ -109,9 +123,9 @@ def test_rounds_of_a_shape(dev):
 @pytest.mark.parametrize("ws,stacked", [(1, False), (4, False), (4, True)])
 @pytest.mark.parametrize("group", [13, 100, 700])
 def test_groups_of_a_round_released_together(api, dev, ws, stacked, group):
-    """Two whole rounds and a bit: the groups of a round take one wait and one copy launch; with 13 tiles
-    to a group there are more groups to a round than lanes to a wavefront."""
-    M, N, K, algo, dt = 8192, 4352, 64, 1, torch.float16
+    """Two whole rounds and a bit, and a K above that with which every group is delivered: the groups of a round take
+    one wait and one copy launch; with 13 tiles to a group there are more groups to a round than lanes to a wavefront."""
+    M, N, K, algo, dt = 8192, 4352, 8200, 1, torch.float16
     BM, BN, _ = capi.algo_tile(algo)
     TM, TN = M // BM, N // BN
     cseg = tiling.uniform_cseg(TM * TN, group)
@@ -134,6 +148,7 @@ def test_groups_of_a_round_released_together(api, dev, ws, stacked, group):
                 o.gemm_allreduce_overlap(A, B, c, mm, RA, 1, cs, cs.to(dev), algo, False)
         torch.cuda.synchronize()
         assert o.wait_timeouts(True) == 0 and not mm.any()
+        assert o.released_groups() == _released(mode, M, N, K, algo, cseg)
         got.append((c, d))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
@@ -167,7 +182,8 @@ def test_receive_buffer_in_the_first_rows_of_c(api, dev, M, N, K, cseg, ws, rank
             assert torch.equal(c[:M // ws], want_d) and torch.equal(c[M // ws:], want_c[M // ws:])
 
 
-@pytest.mark.parametrize("M,N,K,group", [(1024, 1024, 512, 8), (8192, 2304, 64, 200), (128, 4096, 4096, 8)])
+@pytest.mark.parametrize("M,N,K,group", [(1024, 1024, 512, 8), (8192, 2304, 64, 200), (128, 4096, 4096, 8),
+                                         (8192, 2304, 8200, 200)])   # the last: groups of the first round released
 def test_all_reduce_in_place(api, dev, M, N, K, group):
     """The staging buffer is C itself, with and without overlap: C is what it is with a buffer of its own."""
     algo, dt = 1, torch.float16
@@ -190,6 +206,7 @@ def test_all_reduce_in_place(api, dev, M, N, K, group):
         o.gemm_allreduce(A, B, c[1], algo)
         torch.cuda.synchronize()
         assert o.wait_timeouts(True) == 0 and not mm.any()
+        assert o.released_groups() == _released(0, M, N, K, algo, cseg)
         got.append(c)
     assert torch.equal(got[0], got[1])
 
@@ -197,7 +214,7 @@ def test_all_reduce_in_place(api, dev, M, N, K, group):
 @pytest.mark.parametrize("M,N,K,group", [
     (8192, 4352, 8192, 100),     # the longest K with which every group is delivered
     (8192, 4352, 8200, 100),     # and one above it: the groups of the first rounds are waited for, round by round
-    (16384, 8192, 72, 1000),     # 256 MiB of output: stored past the caches
+    (16384, 8192, 72, 1000),     # delivered, 256 MiB of output: stored past the caches
 ])
 @pytest.mark.parametrize("ws", [1, 4])
 def test_which_groups_are_delivered(api, dev, M, N, K, group, ws):
@@ -224,6 +241,7 @@ def test_which_groups_are_delivered(api, dev, M, N, K, group, ws):
             o.gemm_allreduce_overlap(A, B, c, mm, RA, 1, cs, cs.to(dev), algo, False)
         torch.cuda.synchronize()
         assert o.wait_timeouts(True) == 0 and not mm.any()
+        assert o.released_groups() == _released(mode, M, N, K, algo, cseg)
         got.append((c, d))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 

@@ -103,16 +103,18 @@ def short_waits():
 
 def _whole_numbers(dev, dt, gen, *shape):
     """Small integers: every sum is exact in fp32, so a call that is split over K and one that is not agree bit for bit."""
-    return torch.randint(-2, 3, shape, generator=gen).to(dt).to(dev)
+    return torch.randint(-2, 3, shape, generator=gen, dtype=torch.int8).to(dev).to(dt)
 
 
 @pytest.mark.parametrize("M,N,K,w,ws", [
     (1024, 1024, 512, 4, 1),       # every group is delivered by the epilogue
     (128, 4096, 4096, 32, 1),      # split over K when it is not captured, every group delivered
     (128, 4096, 4096, 8, 4),
-    (8192, 4352, 64, 100, 1),      # groups of a round released together, the last ones delivered
-    (8192, 4352, 64, 100, 4),
-    (4352, 4096, 1544, 200, 1),    # the same, and sixteen tiles split over K when it is not captured
+    (8192, 4352, 64, 100, 1),      # delivered, in three rounds
+    (8192, 4352, 8200, 100, 1),    # groups of a round released together on the second stream, the last ones delivered
+    (8192, 4352, 8200, 100, 4),
+    (4352, 4096, 1544, 200, 1),    # delivered, and sixteen tiles split over K when it is not captured
+    (4352, 4096, 8200, 200, 1),    # released, and split
 ])
 def test_default_mode_replays_from_a_graph(dev, short_waits, M, N, K, w, ws):
     """The automatic mode: a warmed call that is captured allocates nothing, and every replay gives what the
@@ -154,6 +156,7 @@ def test_default_mode_replays_from_a_graph(dev, short_waits, M, N, K, w, ws):
             made = torch.cuda.memory_stats()["allocation.all.allocated"]
             call()
             assert torch.cuda.memory_stats()["allocation.all.allocated"] == made
+        assert (o.released_groups() > 0) == (K > 8192)     # the captured call's
         for replay in range(3):
             print(f"graph replay {replay} {M}x{N}x{K} w={w} ws={ws}", flush=True)
             A.copy_(_whole_numbers(dev, dt, gen, M, K))

@@ -122,6 +122,45 @@ def test_monitor_sampling_and_vote_agree_with_the_raster(ready):
     assert agree > 0.9
 
 
+@pytest.mark.parametrize("ws,rank", [(1, 0), (4, 2)])
+@pytest.mark.parametrize("K,checked,released", [(8200, False, 4), (8200, True, 6), (200, True, 6), (200, False, 0)])
+def test_linear_calls_whose_groups_are_released(ready, ws, rank, K, checked, released):
+    """A linear call keeps no C, and makes one where groups are copied out of it: of a K above that with which every group
+    is delivered, those of the first of two rounds, and in checked mode all.  Small whole numbers: the result is the plain product."""
+    dev, dt, M, N, algo = ready, torch.bfloat16, 8192, 2304, 1
+    BM, BN, _ = capi.algo_tile(algo)
+    TM, TN = M // BM, N // BN
+    cseg = [300, 300, 300, 124, 64, 64]       # 1024 layout tiles to the first round
+    cs = torch.tensor(cseg, dtype=torch.int32)
+    RA = tiling.reorder_indices(TM * TN, tiling.raster_hint(M, N, algo), dev).reshape(TM, TN)
+    gen = torch.Generator(device=dev).manual_seed(K)
+    A, B = (torch.randint(-2, 3, (r, K), generator=gen, device=dev).to(dt) for r in (M, N))
+    rows = (A.float() @ B.float().t()).to(dt).view(TM, BM, TN, BN).permute(0, 2, 1, 3).reshape(TM * TN, BM, BN)
+    slots = torch.empty_like(rows)
+    slots[RA.view(-1).long()] = rows
+    o = torch.classes.flashoverlap_class.OverlapImpl()
+    o.mccl_init(rank, ws, torch.ops.flashoverlap_op.generate_mccl_id())
+    o.mutlass_init()
+    o.overlap_init()
+    o.set_check_timeouts(checked)
+    mm = torch.zeros(len(cseg), dtype=torch.int32, device=dev)
+    if ws == 1:
+        want = slots.view(M, N)
+        call = lambda: o.allreduce_linear(A, B, mm, RA, cs, cs.to(dev), algo)
+    else:
+        RE = tiling.generate_row_remap_array(M, N, BM, BN, cseg, ws, dev)
+        placed = torch.empty(TM * TN * BM, BN, dtype=dt, device=dev)
+        placed[RE.long()] = slots.view(-1, BN)
+        starts = [sum(cseg[:g]) * BM for g in range(len(cseg))]
+        want = torch.cat([placed[r + rank * n * BM // ws:r + (rank + 1) * n * BM // ws] for r, n in zip(starts, cseg)]).view(M // ws, N)
+        call = lambda: o.reducescatter_linear(A, B, mm, RA, RE, cs, cs.to(dev), algo)
+    for _ in range(3):
+        got = call()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and o.released_groups() == released and not mm.any()
+    assert _no_timeouts(o)
+
+
 @pytest.mark.parametrize("comm_op,ws,rank,dt", [("all_reduce", 1, 0, torch.float16), ("reduce_scatter", 8, 3, torch.bfloat16)])
 def test_correctness_examples(ready, tmp_path, comm_op, ws, rank, dt):
     """The two example scripts of the reference as one command: its result lines, and True."""
