@@ -1,5 +1,5 @@
-"""The GEMM with four panels ahead (64x64 tiles, and 128x128 ones that have a CU to themselves): K from less
-than one panel to more than the ring holds, whole and partial last panels, tiles whole and cut, against exact
+"""The GEMM with four panels ahead (64x64 tiles, and 128x128 ones that have a CU to themselves) and with three (256x128):
+K from less than one panel to more than a full turn of the rings (of three and four slots: twelve panels), whole and partial last panels, tiles whole and cut, against exact
 sums.  The operands are small whole numbers, so every fp32 sum is exact and the result is its rounding."""
 import pytest
 import torch
@@ -20,12 +20,12 @@ def _object():
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("macro", [0, 128])   # 0: 64x64 at these sizes
-@pytest.mark.parametrize("k", [8, 64, 72, 128, 192, 200, 256, 264, 320, 384, 576, 632])
+@pytest.mark.parametrize("macro", [0, 128, 256128])   # 0: 64x64 at these sizes
+@pytest.mark.parametrize("k", [8, 64, 72, 128, 192, 200, 256, 264, 320, 384, 576, 632, 768, 776, 1088, 1672])
 def test_every_length_of_k(k, macro, dtype):
     o = _object()
     g = torch.Generator().manual_seed(k)
-    for m, n in [(128, 256), (64, 128), (101, 203)]:
+    for m, n in [(128, 256), (64, 128), (101, 203), (300, 136)]:
         a = torch.randint(-3, 4, (m, k), generator=g)
         b = torch.randint(-3, 4, (n, k), generator=g)
         want = (a.double() @ b.double().t()).to(dtype)

@@ -58,6 +58,24 @@ def test_split_plain(dev, dt, M, N, K):
     assert not ws[:1024].any() and (ws[need // 4:] == 1e30).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(128, 128, 8192), (33, 129, 4104), (100, 1160, 7168), (128, 4096, 4096), (256, 2048, 4160)])
+def test_split_plain_by_a_second_launch(dev, M, N, K):
+    """The shapes that go to 64x64 tiles, which add their parts up themselves, in 128x128 ones: the reduction stores
+    whole and ragged tiles, and delivers them."""
+    L = capi.lib()
+    try:
+        capi.check(L.fo_tune(b"macro_tile", 128))
+        c = capi.GemmCall(mode=0, dtype=capi.FO_BF16, algo=1, M=M, N=N, K=K, rLDN=1, nslices=1)
+        need = C.c_size_t()
+        capi.check(L.fo_gemm_workspace(C.byref(c), C.byref(need)))
+        tiles = -(-M // 128) * -(-N // 128)
+        assert need.value > 4096 and (need.value - 4096) % (tiles * 128 * 128 * 4) == 0
+        for dt in (torch.float16, torch.bfloat16):
+            test_split_plain(dev, dt, M, N, K)
+    finally:
+        capi.check(L.fo_tune(b"macro_tile", 0))
+
+
 @pytest.mark.parametrize("M,N,K,algo", [(128, 1024, 4096, 1), (384, 640, 2056, 1), (512, 256, 4096, 2), (256, 640, 4096, 4),
                                         (4352, 4096, 1544, 1)])
 @pytest.mark.parametrize("ws", [1, 4])
@@ -108,9 +126,11 @@ def test_split_signal_and_scatter(dev, M, N, K, algo, ws):
                 assert torch.equal(mine, rows[r0 + k * nr // ws:r0 + (k + 1) * nr // ws])
 
 
-@pytest.mark.parametrize("M,N,K", [(256, 128, 64), (384, 256, 72), (8, 136, 128), (600, 385, 200), (1536, 2048, 192)])
+@pytest.mark.parametrize("M,N,K", [(256, 128, 64), (384, 256, 72), (8, 136, 128), (600, 385, 200), (1536, 2048, 192),
+                                   (384, 256, 264), (600, 385, 840), (256, 384, 1664)])
 def test_tall_tile_gives_the_bits_of_the_square_one(dev, M, N, K):
-    """The 256x128 macro tile on one, two and three panels, half and ragged tiles: the order of additions is the same."""
+    """The 256x128 macro tile on fewer panels than its ring holds, as many, one more and several turns of it, half
+    and ragged tiles: the order of additions is the same."""
     L = capi.lib()
     g = torch.Generator().manual_seed(M + N + K)
     A, B = (torch.randn(r, K, generator=g).to(torch.bfloat16).to(dev) for r in (M, N))

@@ -1,23 +1,34 @@
 """The workspace of GEMMs that are split over K: an object makes it where it can, and a call for which it cannot
 be made is computed without.  Integer-valued inputs: split or not, the result is the same bit for bit."""
+import ctypes
+
 import pytest
 import torch
 
 import flashoverlap_amd
+from flashoverlap_amd import capi
 
 pytestmark = pytest.mark.gpu
 
-M, N, K = 128, 4096, 7168      # 32 tiles in 8 parts of 64 KiB: the workspace is the largest one, 64 MiB
+M, N, K = 4225, 4104, 1984     # 17 x 17 macro tiles of 256x256, the 33 behind a whole round in parts: the largest workspace
+
+
+def _step(m, n, k):
+    """Which of the workspaces of 4, 16 and 64 MiB a plain call takes."""
+    c = capi.GemmCall(mode=0, dtype=capi.FO_BF16, algo=1, M=m, N=n, K=k, rLDN=1, nslices=1)
+    need = ctypes.c_size_t()
+    capi.check(capi.lib().fo_gemm_workspace(ctypes.byref(c), ctypes.byref(need)))
+    return need.value and sum(need.value > 4096 + (s << 20) for s in (4, 16)) + 1
 
 
 @pytest.fixture
 def call(dev):
     """A plain GEMM on an object and a stream of its own, and what it has to give."""
     flashoverlap_amd.load()
+    assert _step(M, N, K) == 3
     gen = torch.Generator().manual_seed(19)
     A, B = (torch.randint(-2, 3, (r, K), generator=gen).to(torch.bfloat16).to(dev) for r in (M, N))
-    want = (A.float() @ B.float().t()).to(torch.bfloat16)
-    torch.cuda.synchronize()
+    want = (A.float() @ B.float().t()).to(torch.bfloat16).cpu()     # compared there: one of the tests leaves the device no memory
     stream = torch.cuda.Stream()
     with torch.cuda.stream(stream):
         o = torch.classes.flashoverlap_class.OverlapImpl()
@@ -31,7 +42,7 @@ def call(dev):
         torch.cuda.synchronize()
         return run.right()
 
-    run.stream, run.launch, run.right = stream, lambda: o.mutlass_gemm(A, B, C, 1), lambda: torch.equal(C, want)
+    run.stream, run.launch, run.right = stream, lambda: o.mutlass_gemm(A, B, C, 1), lambda: torch.equal(C.cpu(), want)
     return run
 
 
@@ -85,7 +96,8 @@ def test_threads_on_one_object(dev):
     import threading
     flashoverlap_amd.load()
     gen = torch.Generator().manual_seed(23)
-    shapes = [(128, 4096, 7168), (128, 1024, 4096)]
+    shapes = [(256, 4096, 7168), (128, 1024, 4096)]
+    assert [_step(*s) for s in shapes] == [2, 1]
     work = []
     for m, n, k in shapes:
         A, B = (torch.randint(-2, 3, (r, k), generator=gen).to(torch.bfloat16).to(dev) for r in (m, n))
