@@ -103,8 +103,10 @@ int gemm_workspace(const fo_gemm_call& c, size_t* bytes) {
 }
 
 // A delivered buffer of this many bytes is stored past the memory-side cache, of whose 256 MiB the norm that
-// reads it next would find little (16384x8192x1024 with its norm: 371 us, 359 so; x512 298, 284); a smaller one is left
-// there (12288x8192x1024, 192 MiB: 257, 273; plain 8191x8184x512, 128 MiB, 161, 190; 8192x4096x512, 64 MiB, 66, 72).
+// reads it next would find little; a smaller one is left there.  Plain call with its norm, us, left there / past it:
+// 8192x4096x1024, 64 MiB, 98 / 103; 12288x8192x1024, 192 MiB, 240 / 253; 16384x7168x1024, 224 MiB, 295 / 289; 16384x8192x1024 and
+// x512, 256 MiB, 347 / 323 and 260 / 246; 16384x9216x1024, 288 MiB, 403 / 366; 16384x12288x1024, 384 MiB, 528 / 492;
+// 16384x16384x1024 and x512, 512 MiB, 726 / 709 and 576 / 553.
 static constexpr long long kStreamDeliverFrom = 256ll << 20;
 
 int launch_gemm(const fo_gemm_call& c, hipStream_t stream, bool keep_d, fo_workspace_fn ask, void* context) {

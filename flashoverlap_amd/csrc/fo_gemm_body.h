@@ -62,7 +62,9 @@
 // copy: 63.1 -> 58.8).  Of the two copies of a call that delivers every tile, D itself is what nobody reads next: stored
 // past the caches it leaves them to the other one (write-through / so, with the norm: 16384x8192x1024 386 / 371 us, 3840x7808x880
 // 86 / 78, 7424x6016x640 116 / 111, plain 8191x8184x512 with its bulk copy 187 / 161; in one round, level).  A caller that keeps only
-// the other one passes no D.
+// the other one passes no D.  One that does read C next, in its copy's place, pays up to 5 % where C would have stayed in a cache (plain
+// call with a norm of C, write-through / so: 7424x6016x640 92.5 / 97.0, 3840x7808x880 75.0 / 78.6, 8192x4096x1024 87.4 / 88.9,
+// 4096x4096x4096 109.5 / 110.5) and gains with a larger one (8191x8184x512 136 / 134, 16384x8192x1024 354 / 323).
 //
 // Semantics follow the reference epilogues src/overlap/gemm_with_signal.h:145-201
 // and src/overlap/gemm_with_scatter.h:146-196; the kernel itself shares nothing
@@ -465,7 +467,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
             // The parts of a 64x64 tile are added up by whichever workgroup finishes last: the others leave their sums
             // with write-through stores, wait for the acknowledgement and count themselves; the last one reads them with
             // loads that are served beyond this XCD's caches, adds in the order of k, its own from registers, and goes on
-            // to the epilogue.  Nobody waits for another workgroup.  In 2 to 4 parts this is 16 to 48 KiB to read;
+            // to the epilogue.  Nobody waits for another workgroup.  In 2 to 6 parts this is 16 to 80 KiB to read;
             // a 128x128 tile's 64 KiB a part, at the 43 bytes per ns that one CU gets, took longer than the reduction's launch
             // (128x4096x7168 with its norm: 25.6 us in 4 parts here, 21.7 in 8 with the launch, 20.2 in two of 64x64).
             constexpr int NB = NBM * NBN;

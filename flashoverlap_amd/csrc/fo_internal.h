@@ -25,7 +25,7 @@ int algo_tile(int algo, int* BM, int* BN, int* BK);
 // fo_time_next_launch: a pair of events that the next GEMM or RMSNorm launch of this thread
 // attaches to its own dispatch, so that the time between them is the kernel's, without the
 // launch gaps an event pair recorded around the launch includes.  Taken by the launch that uses it.
-// A call of two launches attaches `start` to the first and `stop` to the second.
+// A call of several launches attaches `start` to the first and `stop` to the last.
 struct LaunchTimer {
     hipEvent_t start = nullptr, stop = nullptr;
 };

@@ -19,7 +19,7 @@
 // 4-8 % faster with non-temporal ones.
 static constexpr size_t kStreamCopiesFrom = 64u << 20;
 
-// Longest K with which the GEMM's epilogue delivers all groups (groups_to_wait_for).
+// Longest K with which the GEMM's epilogue delivers all groups: a choice, see groups_to_wait_for.
 static constexpr int kDeliverAllK = 8192;
 
 OverlapImpl::OverlapImpl() = default;
@@ -337,7 +337,9 @@ void OverlapImpl::fork_comm_stream(int waited, int G) {
 // norm, early groups copied / all delivered, bf16 unless said, us: 7424x6016x640 141 / 110, 3840x7808x880 105 / 78,
 // 8192x4096x512 93 / 66, 12288x8192x1024 290 / 255, 16384x8192x1024 385 / 359, reducescatter 15104x1280x2936 fp16 in a
 // world of two 160 / 140.  The longer a round the better the copies hide: 8192x8192x8192 791 / 787, 8192x8192x16384
-// 1549 / 1542, level.  There groups are released as they complete, which is what lets a consumer start early.
+// 1549 / 1542, level.  So the limit is no crossing, at which one of the two becomes the slower: it is a choice, within
+// the lengths at which neither costs anything.  Above it groups are released as they complete, which is what lets a
+// consumer start early; below, a caller who wants that takes an explicit mode.
 // Checked mode and monitor mode keep every group on its counter (the first reports a count that
 // does not come out, the second takes its tickets from the signals), and so do the explicit modes.
 int OverlapImpl::groups_to_wait_for(const fo_gemm_call& call, const int* cseg, int nslices, int* first_slot,
