@@ -112,7 +112,7 @@ def main() -> int:
     ap.add_argument("--consumer", default="auto", choices=["auto", "per_group", "persistent"])
     ap.add_argument("--last-group", default="settle_then_join", choices=["main", "comm", "settle", "settle_then_join"],
                     help="how the last group is released (per-group consumer): settle_then_join (default, what "
-                         "OverlapImpl does): on the GEMM's own stream by one launch that settles the counter and copies, "
+                         "OverlapImpl does in its consumer mode 1): on the GEMM's own stream by one launch that settles the counter and copies, "
                          "the earlier groups joined behind it; settle: the same with the join in front; main: wait "
                          "kernel + copy on the GEMM's stream behind the join; comm: on the second stream like every "
                          "other group, as the reference does")
@@ -121,7 +121,7 @@ def main() -> int:
                          "which runs one kernel at a time)")
     ap.add_argument("--fork", action="store_true",
                     help="order the second stream behind the main stream before the GEMM, which OverlapImpl does when "
-                         "the call is being captured into a graph (costs 5-9 us of a step when done eagerly)")
+                         "a call that releases groups is being captured into a graph (costs 5-9 us of a step when done eagerly)")
     ap.add_argument("--tune", action="append", default=[], metavar="KNOB=VALUE",
                     help="library knob for this run (fo_tune: store_mode, release_mode, copy_streaming_stores)")
     a = ap.parse_args()
@@ -196,8 +196,10 @@ def main() -> int:
             self.table = torch.empty(T, dtype=torch.int32, device=dev)
             capi.check(L.fo_build_group_table(self.cseg_d.data_ptr(), self.G, T, self.table.data_ptr(), None))
             self.RE = tiling.generate_row_remap_array(M, N, BM, BN, self.cseg, ws, dev) if ws > 1 else None
-            # Same rule as OverlapImpl: up to 32 groups the reference's structure (one wait kernel and one
-            # consumer launch per group, src/overlap_impl.cu:257-265), beyond that one persistent kernel.
+            # What is timed here is the signalled path: every group released through its counter, up to 32 groups
+            # in the reference's structure (one wait kernel and one consumer launch per group,
+            # src/overlap_impl.cu:257-265; OverlapImpl's consumer mode 1), beyond that by one persistent
+            # kernel (mode 2).  OverlapImpl's automatic mode would deliver all groups of these workloads.
             self.per_group = a.consumer == "per_group" or (a.consumer == "auto" and self.G <= 32)
 
     def gemm_signal(g):
@@ -222,7 +224,7 @@ def main() -> int:
                                          None, a.consumer_blocks, None, comm))
             capi.check(L.fo_stream_join(comm, main_stream))
             return
-        # like OverlapImpl: the groups before the last are copied beside the GEMM; if that is a lot of data,
+        # like OverlapImpl::consume_groups: the groups before the last are copied beside the GEMM; if that is a lot of data,
         # with non-temporal stores (1), else with ordinary ones (2); the last group always with ordinary ones
         beside = 2 * BM * BN * sum(g.cseg[:-1])
         beside_policy = 1 if beside >= (64 << 20) else 2

@@ -389,9 +389,9 @@ int fo_stream_join(void* signaller, void* waiter);
  * fo_reorder_rmsnorm* launch made by the calling thread attaches the two events (from
  * fo_event_create) to its own dispatch; fo_event_elapsed_ms between them is then the
  * kernel's duration, as a profiler reports it, without the launch gaps that an event
- * pair recorded around the call includes.  A GEMM that is split over K (fo_gemm_launch with a
- * workspace) is two dispatches: the pair spans them, from the start of the first to the end of
- * the second.  Passing two nulls cancels. */
+ * pair recorded around the call includes.  A GEMM can be up to three dispatches (the last rows or
+ * columns, the tiles, and with a workspace the sum of tiles that are split over K): the pair spans
+ * them, from the start of the first to the end of the last.  Passing two nulls cancels. */
 int fo_time_next_launch(void* start_event, void* stop_event);
 /* *capturing = 1 while `stream` is recording into a graph (stream capture), else 0.
  * No counterpart in the reference, whose overlapped call cannot be captured. */
