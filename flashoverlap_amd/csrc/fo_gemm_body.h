@@ -82,9 +82,6 @@
 
 namespace fo {
 
-constexpr int kTurnFrom = 48;   // panels of K from which on the XCDs begin at different ones
-static_assert(kTurnFrom / kXcds > 4, "the first panels, as many as any ring is deep, are copied without a turn");
-
 // LDS of the panel slots: `depth` of A and one more of B.
 constexpr int ring_bytes(int mtm, int mtn, int depth) { return (depth * mtm + (depth + 1) * mtn) * kRowBytes; }
 
@@ -133,21 +130,12 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
         at_tile = whole_tile_pos(p, tile);
     }
     const TileCoord mt = macro_tile_at<MTM, MTN>(p, at_tile);
-    // One round of 256x128 tiles: the XCDs begin at eight places of K, panel kt of a workgroup is panel kt + turn, and behind the last
-    // one comes the first.  Workgroups in step otherwise ask for the same few columns of every row at a time, and rows whose length is a
-    // multiple of 256 bytes or more spread these over few memory channels.  Inside an XCD, whose workgroups share panels in their
-    // L2, all begin at the same place, and neighbours three eighths apart (one eighth: 4096x1024x5120 52.7 us, 49.8 so).
-    // Plain GEMM and its copy, bf16, operands from HBM, us, all at panel 0 / so: 2688x1920x4928 72.3 / 61.1, 2048x4096x6144
-    // 107.3 / 93.5, 768x8192x4096 59.8 / 53.1, 4096x1024x5120 54.3 / 49.5, 2048x4096x5120 81.0 / 75.7, x3584 55.0 / 51.0, x7168 107.7 / 103.9,
-    // x7680 116.5 / 112.2; with operands from the memory-side cache mostly level (2048x4096x6144 79.9 / 80.5, 2688x1920x4928 53.5 / 54.5),
-    // with few rows up to 3 % more (1024x8192x3584 48.8 / 48.9, fp16 50.7 / 52.4; with its receive copy and norm 49.7 / 50.0).  With operands
-    // that it holds in part: 2041x4096x7168 fp16 with its norm 111.7 / 108.5.  From 48 panels on: 2048x4096x3072 and below gain
-    // nothing.  Nor do parts of split tiles, which begin at different places as it is (128x4096x7168 with its norm 19.5 / 19.9); several rounds
-    // of 256x256 tiles lose (8192x4096x7168 with its norm 348 / 357, 8192x8192x3584 346 / 355).  (A last, partial panel would have
-    // to be told from the others wherever it comes.)
+    // One round of 256x128 tiles (turn_panels in fo_plan.h): the XCDs begin at eight places of K, panel kt of a workgroup is panel
+    // kt + turn, and behind the last one comes the first.  Inside an XCD all begin at the same place, for they share panels in its L2,
+    // and neighbours three eighths apart (one eighth: 1.026 times as long on 70 shapes, bf16, operands from HBM).  Parts of split tiles
+    // begin at different places as it is, and several rounds of 256x256 tiles lose (8192x4096x7168 with its norm 348 / 357 us).
     int turn = 0;
-    if constexpr (MTM != MTN)
-        if (K % kBK == 0 && NP >= kTurnFrom && p.split_from <= kWave) turn = (int)(blockIdx.x * 3u % kXcds) * (NP / kXcds);
+    if constexpr (MTM != MTN) turn = (int)(blockIdx.x * 3u % kXcds) * p.turn;
     int k_first = kt0 + turn;   // panel kt of this workgroup is panel kt + k_first of K (the main loop turns back to the first)
     // M and N are multiples of the layout tile, not necessarily of the macro
     // tile: the last row or column of macro tiles may be half inside.  Such a

@@ -86,6 +86,7 @@ struct GemmParams {
     // leave it in `partial`; the reduction adds the parts up and stores the tiles (of 64x64 tiles, the
     // workgroup that finishes a tile's last part does).
     int split_from, split_tiles, splits, split_panels;
+    int turn;     // 256x128 tiles: panels of K between the places where the XCDs begin, 0: all at the first
     float* partial;
     int* arrived;                               // strips of each layout tile that the reduction has stored; parts of each 64x64 tile that are in `partial`
     // delivery (null: none): tiles at slots >= deliver_from are stored there too, and not signalled

@@ -15,6 +15,7 @@
 namespace fo {
 
 constexpr int kTallDepth = 3;
+static_assert(kTurnFrom / kXcds >= kTallDepth, "the first panels, as many as the ring is deep, are copied without a turn");
 
 template <typename T, int MODE, bool EDGE>
 __global__ void __launch_bounds__(256) gemm_tall_kernel(const GemmParams p) {
