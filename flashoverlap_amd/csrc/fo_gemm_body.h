@@ -450,11 +450,27 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
         ring_a[DEPTH - 1] = a0;
         ring_b[DEPTH] = b0;
     };
-    for (; kt < NP - DEPTH; ++kt) {
-        last_panel_next(kt + DEPTH + 1 == NP);   // this k-step copies panel kt + DEPTH
-        if constexpr (MTM != MTN) k_first -= kt + DEPTH == NP - turn ? NP : 0;   // (not while the first DEPTH panels are copied: NP - turn >= NP / 8)
-        kstep(kt, ring_a[0], ring_a[1], ring_b[1], ring_b[DEPTH], template_int<DEPTH>{});
-        rotate();
+    if constexpr (MTM == MTN) {
+        for (; kt < NP - DEPTH; ++kt) {
+            last_panel_next(kt + DEPTH + 1 == NP);   // this k-step copies panel kt + DEPTH
+            kstep(kt, ring_a[0], ring_a[1], ring_b[1], ring_b[DEPTH], template_int<DEPTH>{});
+            rotate();
+        }
+    } else {
+        // Before one k-step the copies change: they turn back to the first panel, or are those of the last one.  (Never both: where
+        // they turn no panel is partial, and the last one's offsets are those of all.)
+        int stop = turn ? NP - turn - DEPTH : NP - DEPTH - 1;
+        while (kt < NP - DEPTH) {
+            if (kt == stop) {
+                last_panel_next(true);
+                k_first -= turn ? NP : 0;
+                stop = NP - DEPTH;
+            }
+            do {
+                kstep(kt, ring_a[0], ring_a[1], ring_b[1], ring_b[DEPTH], template_int<DEPTH>{});
+                rotate();
+            } while (++kt < stop);
+        }
     }
     static_for<DEPTH>([&](auto t_c) {
         constexpr int after = DEPTH - 1 - decltype(t_c)::value;

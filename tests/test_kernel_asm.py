@@ -190,3 +190,23 @@ def test_consumer_copy_variants_differ_in_their_stores(tmp_path):
     assert len(found) == 2
     for name, vgpr, spill in found:
         assert int(vgpr) <= 72 and int(spill) == 0, (name, vgpr, spill)
+
+
+def test_the_main_loop_of_256x128_tiles_selects_nothing(gemm_asm):
+    """The change of the copies' addresses before one k-step lies outside the loop over the k-steps: a comparison and selects in
+    every k-step made each call of these tiles up to 1 % longer."""
+    bodies, _ = gemm_asm
+    for name, ins in bodies.items():
+        if "gemm_tall_kernel" not in name:
+            continue
+        labels = {i[:-1]: at for at, i in enumerate(ins) if i.endswith(":")}
+        loops = []
+        for at, i in enumerate(ins):
+            m = re.match(r"s_c?branch\S* (\S+)", i)
+            if m and labels.get(m.group(1), at) < at:
+                body = ins[labels[m.group(1)]:at]
+                if any(x.startswith("v_mfma") for x in body):
+                    loops.append(body)
+        body = min(loops, key=len)   # (the others are around it, or of blocks that lie behind their successors)
+        assert sum(x.startswith("v_mfma") for x in body) == 64, f"{name}: not a k-step"
+        assert not [x for x in body if x.startswith(("v_cndmask", "s_cselect"))], name
