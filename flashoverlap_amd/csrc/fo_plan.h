@@ -12,7 +12,8 @@ namespace fo {
 constexpr int kBK = 64;             // k-elements per LDS buffer
 constexpr int kMaxHereSplits = 6;   // parts of a 64x64 tile, added up in the GEMM
 constexpr int kTurnFrom = 48;       // panels of K from which on the XCDs begin at different ones (turn_panels)
-constexpr int kLowRow = 200;        // rows of the matrix in a last row of 256x128 tiles that is low
+constexpr int kLowRow = 200;        // rows of the matrix, at most, in a last row of 256x128 tiles that is low
+constexpr int kThinColumn = 32;     // columns of it in a last column of tiles whose workgroups run ahead
 constexpr size_t kMaxWorkspace = (size_t)64 << 20;   // bytes of the parts of split tiles, at most
 constexpr int kSkinnyRows = 32;     // rows that the skinny kernel takes (fo_internal.h has its times)
 
@@ -110,22 +111,24 @@ inline Plan make_plan(int BM, int BN, int M, int N, int K, bool any_tile, bool m
 // Workgroups in step ask for the same few columns of every row at a time; apart, an XCD finds what another one has read already in the
 // memory-side cache.  So it pays where the XCDs share the rows of A: where every band of four rows of tiles, the last one too, has at
 // least a column of its tiles on a second XCD.  Rows that one XCD has to itself come from HBM all the same, now while the others do not wait for
-// the same columns, and that is slower, unless they are the few of a low last row.  Where the last column of tiles is less than half full its
-// workgroups copy less and run ahead by themselves.  (That much is measured; that it is the memory channels and caches is a conjecture.)
-// Operands from HBM, bf16 and fp16, all at panel 0 / apart: 622 shapes of this rule 1.086 (geometric mean; the slowest 0.97), the 355
-// others 0.992 (0.93 at worst).  us, K = 4160 bf16: 2048x3328 57.7 / 52.4, 2176x2304 56.9 / 51.0, 3072x2176 58.1 / 53.7; 2304x2304 57.6 / 60.6, 3328x2048
-// 58.3 / 61.8, 7168x896 59.7 / 63.5; K = 6272: 1024x5888 83.8 / 78.5, 1024x5824 80.1 / 79.0, 1024x5792 77.3 / 79.5; 2248x3072 1.08 times
-// as fast, 2280x3072 0.97.  From the memory-side cache level (110 shapes 0.9995, 0.991 at worst).  From 48 panels on: the gain begins earlier
-// (2048x4096x2432 39.8 / 38.8, x3136 48.8 / 47.5; 640x8832x2048 30.2 / 29.0), but was measured on six shapes there, not on this range.
+// the same columns, and that is slower, unless the last row of tiles is low.  Where the last column of tiles has few columns of the matrix its
+// workgroups copy less and run ahead by themselves.  (That much is measured; that it is the channels and caches is a conjecture.)
+// Operands from HBM, bf16 and fp16, all at panel 0 / apart: 790 shapes of this rule 1.077 (geometric mean; the slowest 0.96), the 466
+// others 0.990 (0.93 at worst).  us, K = 4160 bf16: 2048x3328 57.7 / 52.4, 2176x2304 56.9 / 51.0, 3072x2176 58.1 / 53.7; 2304x2304 57.6 / 60.6, 3328x2048
+// 58.3 / 61.8, 7168x896 59.7 / 63.5; K = 6272: 2248x3072 87.2 / 81.5, 2280x3072 86.4 / 89.0; 1024x5888 83.8 / 78.5, 1024x5840 82.3 / 80.1,
+// 1024x5792 77.3 / 79.5.  From the memory-side cache level (110 shapes 0.9995, 0.991 at worst).  From 48 panels on: the gain begins earlier
+// (2048x4096x2432 39.8 / 38.8, 640x8832x2048 30.2 / 29.0), but was measured on six shapes there, not on this range.
 inline int turn_panels(Macro macro, int M, int N, int K, int cus) {
     if (macro.m == macro.n || K % kBK || K / kBK < kTurnFrom) return 0;
     constexpr int kBand = kGroupM / 2;
     const int GM = (M + macro.m - 1) / macro.m, GN = (N + macro.n - 1) / macro.n, tiles = GM * GN;
     const int last_band = (GM - 1) % kBand + 1, last_row = M - (GM - 1) * macro.m, last_column = N - (GN - 1) * macro.n;
-    if (tiles > cus || last_column < macro.n / 2) return 0;
-    auto on_two_xcds = [&](int rows) { return rows * (GN - 1) * kXcds >= tiles; };
-    if (GM > kBand && !on_two_xcds(kBand)) return 0;
-    return on_two_xcds(last_band) || (last_band == 1 && last_row <= kLowRow) ? K / kBK / kXcds : 0;
+    if (tiles > cus || last_column <= kThinColumn) return 0;
+    // a band of that many rows exceeds an XCD's share of the tiles, by at least so many
+    auto exceeds = [&](int rows, int by) { return (rows * GN - by) * kXcds >= tiles; };
+    if (GM > kBand && !exceeds(kBand, kBand)) return 0;
+    const bool low = last_row <= kLowRow && (last_band == 1 || exceeds(last_band, 1));
+    return low || exceeds(last_band, last_band) ? K / kBK / kXcds : 0;
 }
 
 // A plain GEMM of which a few rows or columns lie behind the last whole multiple of 128: as macro tiles they are a row or column

@@ -19,7 +19,10 @@ MEASURED = {
     (7680, 1024, 4160): (63.2, 66.6), (9216, 896, 4160): (64.0, 68.3), (10240, 640, 4160): (61.0, 64.5),
     # 200 rows and 232 in the last row of tiles
     (2248, 3072, 6272): (87.2, 81.5), (2280, 3072, 6272): (86.4, 89.0),
-    # few columns in the last column of tiles, and more than half of it
+    # a last band of three rows, 70 and 128 rows in the last of them
+    (5702, 1280, 4288): (64.8, 62.8), (5760, 1152, 4160): (60.1, 56.6), (5760, 896, 4160): (58.9, 60.3),
+    # 8, 16 and 32 columns in the last column of tiles, 40 and more
+    (3755, 1320, 8128): (106.8, 96.4), (2663, 2220, 7616): (101.6, 95.9),
     (1024, 5768, 6272): (77.8, 80.0), (1024, 5792, 6272): (77.3, 79.5), (1024, 5840, 6272): (82.3, 80.1), (768, 8096, 6272): (78.5, 80.5),
     (768, 8160, 6272): (84.7, 81.2), (2432, 2960, 6272): (79.2, 83.0), (3584, 2064, 6272): (80.9, 83.1), (3584, 2144, 6272): (89.2, 82.7),
 }
