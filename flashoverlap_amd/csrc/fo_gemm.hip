@@ -201,7 +201,8 @@ int launch_gemm(const fo_gemm_call& c, hipStream_t stream, bool keep_d, fo_works
     p.GM = (p.M + plan.macro.m - 1) / plan.macro.m; p.GN = (p.N + plan.macro.n - 1) / plan.macro.n;
     p.gn_magic = raster_magic(p.GN);
     p.split_from = plan.from; p.split_tiles = plan.tiles; p.splits = plan.splits; p.split_panels = plan.panels;
-    p.turn = turn_panels(plan.macro, p.M, p.N, K, facts->cus);
+    // A call without a workspace adds in the order of k, in whatever tile.
+    p.turn = ask || (c.workspace && enough) ? turn_panels(plan.macro, p.M, p.N, K, facts->cus) : 0;
     if (plan.tiles) {
         if ((uintptr_t)workspace & 15) return fail(FO_ERR_ARG, "fo_gemm: the workspace must be 16-byte aligned");
         p.arrived = (int*)workspace;

@@ -153,9 +153,16 @@ int fo_gemm_signal_static(int dtype, int algo, int M, int N, int K, int rLDN,
  *             shape can use (0: none).  Less is as good as none: the tiles are
  *             then not split.  Its first FO_WORKSPACE_ZEROED bytes must be zero
  *             before the first call; every call leaves them zero.  Calls that can
- *             run at the same time need workspaces of their own.  Results differ
- *             from those without a workspace by the order of fp32 additions;
- *             for one shape they are always the same. */
+ *             run at the same time need workspaces of their own.  Without
+ *             one (or with less) every sum is taken in the order of k, except in
+ *             the kernel for a plain GEMM of up to 32 rows and for as few rows or
+ *             columns behind the last whole tiles.  A call that passes one, also
+ *             for a shape that can use 0 bytes of it, leaves the order of the
+ *             fp32 additions to the library: parts of k are added up, and the
+ *             workgroups of a round may begin at different places of K.  Results
+ *             then differ by that order from those without, and those of equal
+ *             rows of A (or B) in different tiles from each other; for one shape
+ *             and setting of fo_tune they are always the same. */
 #define FO_WORKSPACE_ZEROED 4096
 enum fo_gemm_mode { FO_GEMM_PLAIN = 0, FO_GEMM_SIGNAL = 1, FO_GEMM_SCATTER = 2 };
 struct fo_gemm_call {
@@ -188,7 +195,8 @@ int fo_gemm_deliver(const struct fo_gemm_call* call, void* stream);
 /* fo_gemm_launch (keep_d 0: fo_gemm_deliver) for callers that keep workspaces of their own
  * and need not know the shape's: if it can use one, `workspace` is asked for at
  * least `bytes` bytes and sets *out, to null for none (the tiles are then not
- * split).  It is called before anything is launched; a status other than FO_OK
+ * split).  The order of the fp32 additions is the library's, as in a call that
+ * passes a workspace.  It is called before anything is launched; a status other than FO_OK
  * is returned as this call's, which then launches nothing.  It must not throw.  The
  * call's own workspace is not looked at. */
 typedef int (*fo_workspace_fn)(void* context, size_t bytes, void** out);
@@ -221,7 +229,11 @@ int fo_build_group_tables(const int* cseg_dev, int G, int T, int* group_table, i
 int fo_raster_hint(int algo, int M, int N, int* hint_host);
 
 /* Process-wide tuning knobs of the GEMM epilogue, for measurement; no
- * counterpart in the reference.  Results are identical for every setting.
+ * counterpart in the reference.  Results are the same for every setting, but
+ * for the order of fp32 additions where fo_gemm_call::workspace leaves it open
+ * and in a plain GEMM of few rows or with few behind its last whole tiles:
+ * there "macro_tile" chooses it, and "release_mode" and "store_mode" 0, for
+ * which not every tile is built.
  * The knobs are atomics: a thread may set one while others launch, and a
  * launch reads each knob once.
  *   "release_mode" 1 (default): the tile stores are agent-scope write-through

@@ -127,10 +127,11 @@ def test_split_signal_and_scatter(dev, M, N, K, algo, ws):
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 128, 64), (384, 256, 72), (8, 136, 128), (600, 385, 200), (1536, 2048, 192),
-                                   (384, 256, 264), (600, 385, 840), (256, 384, 1664)])
+                                   (384, 256, 264), (600, 385, 840), (256, 384, 1664), (256, 384, 3008), (512, 385, 3072),
+                                   (1152, 2176, 3520), (2048, 2048, 4096)])
 def test_tall_tile_gives_the_bits_of_the_square_one(dev, M, N, K):
     """The 256x128 macro tile on fewer panels than its ring holds, as many, one more and several turns of it, half
-    and ragged tiles: the order of additions is the same."""
+    and ragged tiles, and on as many as begin apart in K where a workspace is passed: without one the order of additions is the same."""
     L = capi.lib()
     g = torch.Generator().manual_seed(M + N + K)
     A, B = (torch.randn(r, K, generator=g).to(torch.bfloat16).to(dev) for r in (M, N))

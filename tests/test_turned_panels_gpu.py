@@ -117,10 +117,12 @@ def test_scattered_tiles(m, n, k, algo, dtype, dev, tall):
     counters = torch.zeros(len(cseg), dtype=torch.int32, device=dev)
     re = tiling.generate_row_remap_array(m, n, bm, bn, cseg, world, dev)
     d, recv = (torch.full((t * bm, bn), 7.0, dtype=dtype, device=dev) for _ in range(2))
+    unused = torch.zeros(4096, dtype=torch.uint8, device=dev)   # these tiles are not split; without one K is not begun apart
     call = capi.GemmCall(mode=2, dtype=capi.dtype_code(dtype), algo=algo, M=m, N=n, K=k, rLDN=1, A=a.data_ptr(), B=b.data_ptr(),
                          D=d.data_ptr(), cseg_dev=cs.data_ptr(), G=len(cseg), group_table=table.data_ptr(), MM=counters.data_ptr(),
                          RA=ra.data_ptr(), RE=re.data_ptr(), deliver=recv.data_ptr(), deliver_from=start[half], nslices=world,
-                         slice_count=world, slice_stride=m * n // world, group_start=st.data_ptr())
+                         slice_count=world, slice_stride=m * n // world, group_start=st.data_ptr(),
+                         workspace=unused.data_ptr(), workspace_bytes=unused.nbytes)
     capi.check(capi.lib().fo_gemm_launch(C.byref(call), None))
     torch.cuda.synchronize()
     assert counters.cpu().tolist() == cseg[:half] + [0] * (len(cseg) - half)
