@@ -458,7 +458,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p) {
         }
     } else {
         // Before one k-step the copies change: they turn back to the first panel, or are those of the last one.  (Never both: where
-        // they turn no panel is partial, and the last one's offsets are those of all.)
+        // they turn no panel is partial, and the last one's offsets are those of all.)  Asked for in every k-step, by compares and
+        // selects, it took 1 % longer with cached operands, 5 % where M or N is ragged (110 shapes).
         int stop = turn ? NP - turn - DEPTH : NP - DEPTH - 1;
         while (kt < NP - DEPTH) {
             if (kt == stop) {

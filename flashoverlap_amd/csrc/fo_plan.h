@@ -40,6 +40,8 @@ struct Plan {
 // 6683x1336x1600 bf16 51.6 38.9 | 38.6 37.0, 640x3840x7872 fp16 74.4 51.0 | 52.1 52.4.
 // With more than half of the CUs at work all the time the k-steps of the larger tiles get longer; at the chip's power limit, in
 // several full rounds, by more than is said here, but no other tile comes near 256x256 there.
+// (256x128 tiles are priced as they were before K was begun apart in them and their loop lost its selects: they are now up to a tenth
+// shorter.  Of 70 shapes given to other tiles by less than 12 %, 30 would be 3 to 14 % faster in them; over all 70 the choice is level.)
 struct Shape {
     int panels, cus;
     double straddle;     // rows that do not start on cache lines ask the L2 for a line twice: all of them, or half where K is a multiple of 32
